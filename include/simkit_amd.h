@@ -489,6 +489,20 @@ int sk_sim_set_coarse(sk_sim* sim, const double* X, int per_agg);
  * order[nv]). A mesh renumbered in this order has the identity row order,
  * so the SpMV's per-row stores are contiguous. */
 int sk_sell_order(const int32_t* T, int64_t nv, int64_t nt, int32_t* order);
+/* Host-only, no counterpart in the reference: a numbering for the resident
+ * PCG, which gives each of n_parts workgroups one contiguous range of rows.
+ * The vertices are cut into n_parts compact parts by recursive coordinate
+ * bisection of X (host, nv x 3); part g is order[part_ptr[g] ..
+ * part_ptr[g + 1]), by descending number of neighbours within it. part_ptr
+ * holds up to 257 entries. n_parts = 0 (a mesh too large for one row per
+ * thread): order is sk_sell_order's. precision: sk_precision. */
+int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
+                  int* n_parts, int32_t* part_ptr);
+/* The rows of the simulator's mesh as n contiguous ranges (ptr_host[n + 1],
+ * as sk_part_order returns them), one per workgroup of the resident PCG; n =
+ * 0 restores the default cut into equal ranges. No counterpart in the
+ * reference. */
+int sk_sim_set_parts(sk_sim* sim, int n, const int32_t* ptr_host);
 /* Host-only, no counterpart in the reference: the vertices of X (host,
  * nv x 3) grouped by the aggregates sk_sim_set_coarse would form with
  * per_agg, ascending within each aggregate (order[nv]), the number of

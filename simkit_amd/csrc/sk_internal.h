@@ -3,6 +3,8 @@
 
 #include "sk_common.h"
 
+#include <memory>
+#include <mutex>
 #include <type_traits>
 #include <vector>
 
@@ -108,6 +110,8 @@ struct Reducer {
   }
 };
 
+struct ResidentPlan;  // sk_resident.h
+
 }  // namespace sk
 
 struct sk_mesh {
@@ -152,6 +156,10 @@ struct sk_mesh {
   sk::DevBuf<double> fst;     // [nt][12] staged element forces
   sk::DevBuf<uint8_t> eflag;  // [nt] element pass: 1 where the closed-form eigensystem was not used
   sk::Reducer red;
+  std::vector<int32_t> h_bptr, h_bcol;  // bptr and bcol on the host
+  // cuts of the rows for the resident PCG (the last few, shared by the mesh's simulators)
+  std::mutex plan_mu;
+  std::vector<std::shared_ptr<sk::ResidentPlan>> plans;
   double* pinned = nullptr;   // 16 host-pinned doubles for scalar readback
 };
 

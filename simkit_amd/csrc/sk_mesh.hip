@@ -15,9 +15,12 @@
 #include "sk_elem.h"
 #include "sk_internal.h"
 #include "sk_materials.h"
+#include "sk_resident.h"
 
 #include <algorithm>
 #include <numeric>
+#include <system_error>
+#include <thread>
 
 namespace sk {
 
@@ -609,6 +612,12 @@ int read_scalars(sk_mesh* m, const double* dev, int n, hipStream_t st) {
 // ---------------------------------------------------------------------------
 // Host pattern build (once per mesh)
 // ---------------------------------------------------------------------------
+// Host threads for a mesh of nt tets: one per 20,000, at most 8.
+static int host_threads(int64_t nt) {
+  const int64_t hw = std::max(1u, std::thread::hardware_concurrency());
+  return (int)std::min<int64_t>({8, hw, nt / 20000 + 1});
+}
+
 static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
   SK_REQUIRE(nt < (int64_t(1) << 27), "sk_mesh_create: at most 2^27 tets");
   SK_REQUIRE(nv < (int64_t(1) << 29), "sk_mesh_create: too many vertices");
@@ -624,46 +633,79 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
     for (int64_t e = 0; e < nt; ++e)
       for (int i = 0; i < 4; ++i) vlist[fill[T[4 * e + i]]++] = (int32_t)((e << 2) | i);
   }
-  // sorted neighbour blocks per vertex (including the vertex itself)
-  std::vector<int32_t> bptr(nv + 1, 0), bcol;
-  bcol.reserve(16 * nv);
-  std::vector<int32_t> nb;
-  for (int64_t v = 0; v < nv; ++v) {
-    nb.clear();
-    nb.push_back((int32_t)v);
-    for (int32_t k = vptr[v]; k < vptr[v + 1]; ++k) {
-      const int64_t e = vlist[k] >> 2;
-      for (int j = 0; j < 4; ++j) nb.push_back(T[4 * e + j]);
-    }
-    std::sort(nb.begin(), nb.end());
-    nb.erase(std::unique(nb.begin(), nb.end()), nb.end());
-    bcol.insert(bcol.end(), nb.begin(), nb.end());
-    bptr[v + 1] = (int32_t)bcol.size();
-  }
-  const int64_t nblk = (int64_t)bcol.size();
-  SK_REQUIRE(9 * nblk < (int64_t(1) << 31), "sk_mesh_create: nnz exceeds int32 indexing");
-  std::vector<int32_t> brow(nblk);
-  for (int64_t v = 0; v < nv; ++v)
-    for (int32_t b = bptr[v]; b < bptr[v + 1]; ++b) brow[b] = (int32_t)v;
-  // element -> block map and per-block contribution lists
-  std::vector<int32_t> emap(16 * nt), cptr(nblk + 1, 0), clist(16 * nt);
-  for (int64_t e = 0; e < nt; ++e)
-    for (int i = 0; i < 4; ++i) {
-      const int32_t v = T[4 * e + i];
-      const int32_t* lo = bcol.data() + bptr[v];
-      const int32_t* hi = bcol.data() + bptr[v + 1];
-      for (int j = 0; j < 4; ++j) {
-        const int32_t b = (int32_t)(std::lower_bound(lo, hi, T[4 * e + j]) - bcol.data());
-        emap[(4 * i + j) * nt + e] = b;
-        cptr[b + 1]++;
+  // Row by row, ranges of rows on several threads: each row's sorted neighbour
+  // blocks (itself included), then the element -> block map and the blocks'
+  // contribution lists, from the row's incidences and a table of its blocks.
+  std::vector<int32_t> bptr(nv + 1, 0);
+  const int nth = host_threads(nt);
+  std::vector<std::vector<int32_t>> cols(nth);
+  auto ranges = [&](auto&& fn) {
+    std::vector<std::thread> pool;
+    for (int k = 1; k < nth; ++k) {
+      try {
+        pool.emplace_back([&fn, k, nv, nth] { fn(k, nv * k / nth, nv * (k + 1) / nth); });
+      } catch (const std::system_error&) {  // no thread to be had: here, then
+        fn(k, nv * k / nth, nv * (k + 1) / nth);
       }
     }
+    fn(0, (int64_t)0, nv / nth);
+    for (auto& t : pool) t.join();
+  };
+  ranges([&](int k, int64_t v0, int64_t v1) {
+    std::vector<int32_t> seen(nv, -1), nb;
+    std::vector<int32_t>& out = cols[k];
+    out.reserve(16 * (v1 - v0));
+    for (int64_t v = v0; v < v1; ++v) {
+      nb.assign(1, (int32_t)v);
+      seen[v] = (int32_t)v;
+      for (int32_t q = vptr[v]; q < vptr[v + 1]; ++q) {
+        const int32_t* c = T + 4 * (int64_t)(vlist[q] >> 2);
+        for (int j = 0; j < 4; ++j)
+          if (seen[c[j]] != v) {
+            seen[c[j]] = (int32_t)v;
+            nb.push_back(c[j]);
+          }
+      }
+      std::sort(nb.begin(), nb.end());
+      out.insert(out.end(), nb.begin(), nb.end());
+      bptr[v + 1] = (int32_t)nb.size();
+    }
+  });
+  int64_t nblk = 0;
+  for (auto& c : cols) nblk += (int64_t)c.size();
+  SK_REQUIRE(9 * nblk < (int64_t(1) << 31), "sk_mesh_create: nnz exceeds int32 indexing");
+  std::partial_sum(bptr.begin(), bptr.end(), bptr.begin());
+  std::vector<int32_t> bcol(nblk), brow(nblk), emap(16 * nt), cptr(nblk + 1, 0), clist(16 * nt);
+  ranges([&](int k, int64_t v0, int64_t v1) {
+    std::copy(cols[k].begin(), cols[k].end(), bcol.begin() + bptr[v0]);
+    std::vector<int32_t> at(nv);  // block of the current row at each of its columns
+    for (int64_t v = v0; v < v1; ++v) {
+      for (int32_t b = bptr[v]; b < bptr[v + 1]; ++b) {
+        brow[b] = (int32_t)v;
+        at[bcol[b]] = b;
+      }
+      for (int32_t q = vptr[v]; q < vptr[v + 1]; ++q) {
+        const int64_t e = vlist[q] >> 2;
+        const int i = vlist[q] & 3;
+        for (int j = 0; j < 4; ++j) {
+          const int32_t b = at[T[4 * e + j]];
+          emap[(4 * i + j) * nt + e] = b;
+          cptr[b + 1]++;
+        }
+      }
+    }
+  });
   std::partial_sum(cptr.begin(), cptr.end(), cptr.begin());
-  {
-    std::vector<int32_t> fill(cptr.begin(), cptr.end() - 1);
-    for (int64_t e = 0; e < nt; ++e)
-      for (int ij = 0; ij < 16; ++ij) clist[fill[emap[ij * nt + e]]++] = (int32_t)((e << 4) | ij);
-  }
+  ranges([&](int, int64_t v0, int64_t v1) {
+    std::vector<int32_t> fill(cptr.begin() + bptr[v0], cptr.begin() + bptr[v1]);
+    for (int64_t v = v0; v < v1; ++v)
+      for (int32_t q = vptr[v]; q < vptr[v + 1]; ++q) {
+        const int64_t e = vlist[q] >> 2;
+        const int i = vlist[q] & 3;
+        for (int j = 0; j < 4; ++j)
+          clist[fill[emap[(4 * i + j) * nt + e] - bptr[v0]]++] = (int32_t)((e << 4) | (4 * i + j));
+      }
+  });
   // SELL-C-sigma layout: rows sorted by block count (descending, stable, so
   // rows of equal degree keep their spatial order), chunks of kSellC rows.
   std::vector<int32_t> order(nv);
@@ -764,7 +806,41 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
   SK_TRY(m->eflag.alloc((size_t)nt));
   SK_TRY(m->red.init());
   SK_HIP_CHECK(hipHostMalloc((void**)&m->pinned, 16 * sizeof(double), hipHostMallocDefault));
+  m->h_bptr = std::move(bptr);
+  m->h_bcol = std::move(bcol);
   return SK_OK;
+}
+
+void degree_order(const std::vector<int32_t>& deg, int32_t* order) {
+  std::iota(order, order + deg.size(), 0);
+  std::stable_sort(order, order + deg.size(), [&](int32_t a, int32_t b) { return deg[a] > deg[b]; });
+}
+
+void vertex_degrees(const int32_t* T, int64_t nv, int64_t nt, std::vector<int32_t>& deg) {
+  std::vector<int32_t> vptr(nv + 1, 0), vlist(4 * nt);
+  for (int64_t k = 0; k < 4 * nt; ++k) vptr[T[k] + 1]++;
+  std::partial_sum(vptr.begin(), vptr.end(), vptr.begin());
+  {
+    std::vector<int32_t> fill(vptr.begin(), vptr.end() - 1);
+    for (int64_t e = 0; e < nt; ++e)
+      for (int i = 0; i < 4; ++i) vlist[fill[T[4 * e + i]]++] = (int32_t)e;
+  }
+  // each vertex's neighbours once: seen[w] is the last vertex that counted w
+  std::vector<int32_t> seen(nv, -1);
+  deg.resize(nv);
+  for (int64_t v = 0; v < nv; ++v) {
+    int32_t d = 1;
+    seen[v] = (int32_t)v;
+    for (int32_t k = vptr[v]; k < vptr[v + 1]; ++k) {
+      const int32_t* c = T + 4 * (int64_t)vlist[k];
+      for (int j = 0; j < 4; ++j)
+        if (seen[c[j]] != v) {
+          seen[c[j]] = (int32_t)v;
+          ++d;
+        }
+    }
+    deg[v] = d;
+  }
 }
 
 }  // namespace sk
@@ -803,25 +879,9 @@ int sk_sell_order(const int32_t* T, int64_t nv, int64_t nt, int32_t* order) {
   SK_REQUIRE(T && order, "sk_sell_order: null argument");
   SK_REQUIRE(nv > 0 && nt > 0, "sk_sell_order: empty mesh");
   for (int64_t k = 0; k < 4 * nt; ++k) SK_REQUIRE(T[k] >= 0 && T[k] < nv, "sk_sell_order: tet index out of range");
-  std::vector<int32_t> vptr(nv + 1, 0), vlist(4 * nt);
-  for (int64_t k = 0; k < 4 * nt; ++k) vptr[T[k] + 1]++;
-  std::partial_sum(vptr.begin(), vptr.end(), vptr.begin());
-  {
-    std::vector<int32_t> fill(vptr.begin(), vptr.end() - 1);
-    for (int64_t e = 0; e < nt; ++e)
-      for (int i = 0; i < 4; ++i) vlist[fill[T[4 * e + i]]++] = (int32_t)e;
-  }
-  std::vector<int32_t> deg(nv), nb;
-  for (int64_t v = 0; v < nv; ++v) {
-    nb.clear();
-    nb.push_back((int32_t)v);
-    for (int32_t k = vptr[v]; k < vptr[v + 1]; ++k)
-      for (int j = 0; j < 4; ++j) nb.push_back(T[4 * (int64_t)vlist[k] + j]);
-    std::sort(nb.begin(), nb.end());
-    deg[v] = (int32_t)(std::unique(nb.begin(), nb.end()) - nb.begin());
-  }
-  std::iota(order, order + nv, 0);
-  std::stable_sort(order, order + nv, [&](int32_t a, int32_t b) { return deg[a] > deg[b]; });
+  std::vector<int32_t> deg;
+  vertex_degrees(T, nv, nt, deg);
+  degree_order(deg, order);
   return SK_OK;
 }
 

@@ -1,0 +1,102 @@
+// Resident PCG: the whole block-Jacobi PCG run of one system in a single
+// launch whose workgroups (at most one per CU) keep their rows' matrix blocks
+// on chip - registers first, then LDS, the rest streamed from L2 - and meet
+// once per iteration through self-tagged words in global memory instead of
+// at launch boundaries. Described at resident_pcg_kernel.
+#pragma once
+
+#include "sk_internal.h"
+
+#include <memory>
+
+namespace sk {
+
+constexpr int kResMaxParts = 256;     // workgroups at most (the CUs of an MI355X)
+constexpr int kResLds = 160 * 1024;   // LDS a workgroup may use
+constexpr int kResStaticLds = 2048;   // bound on the kernel's static LDS
+// Threads per workgroup and blocks per thread held in registers, by precision.
+constexpr int kResNT64 = 512, kResKR64 = 8;
+constexpr int kResNT32 = 512, kResKR32 = 14;
+constexpr int kResMaxTier = 4;        // blocks per thread in LDS, and streamed from L2, at most (each)
+
+// Cut of a mesh's rows into contiguous ranges, one per workgroup, with the
+// index data the kernel reads (built once per mesh and cut on the host).
+struct ResidentPlan {
+  std::vector<int32_t> parts;      // [G + 1] the cut (the cache key, with fp32)
+  bool fp32 = false;
+  int G = 0, K = 0, KL = 0, KS = 0;  // blocks per thread: K = registers (up to KR) + LDS (KL) + streamed (KS)
+  int max_rows = 0, max_local = 0, max_halo = 0, n_exp = 0;
+  size_t lds = 0;                  // dynamic LDS bytes
+  DevBuf<int32_t> row0;            // [G + 1]
+  DevBuf<uint16_t> lcol;           // [nblk] (local column << 1) | last block of its row
+  DevBuf<uint16_t> trow;           // [G NT] local row of each thread's first block (rows: none)
+  // The halo of a part: the vertices of other parts that its rows couple to (hvert, ascending; halo_ptr[G + 1]),
+  // and their places among all exported vertices (ResidentArgs::halo, exp0, exslot).
+  DevBuf<int32_t> halo_ptr, hvert, halo, exp0;
+  DevBuf<uint16_t> exslot;
+};
+
+// What the kernel reports to the host (pinned).
+struct ResidentResult {
+  int iter, done, refines, aborted;
+  uint32_t epoch;
+};
+
+// A simulator's side of the resident solver: its plan and exchange buffers.
+struct ResidentState {
+  std::vector<int32_t> parts;            // the caller's cut; empty: the default one
+  std::shared_ptr<ResidentPlan> plan;    // null: not built or not eligible
+  bool tried = false;                    // plan has been looked for
+  bool off = false;                      // a run gave up waiting: launches only from now on
+  DevBuf<uint64_t> slots, zx, xx;
+  DevBuf<char> stream;
+  DevBuf<int> abort_flag;
+  ResidentResult* host = nullptr;        // pinned
+  uint32_t epoch = 0;
+  ~ResidentState();
+};
+
+// Workgroups for a mesh of nv vertices and nblk blocks; 0: not eligible.
+int resident_parts(int64_t nv, int64_t nblk, bool fp32);
+
+// A block of `need` CUs of the current device for one resident run, held
+// until the run has ended: runs of one process that overlap on one GPU never
+// ask for more workgroups together than can be resident at once.
+class ResidentPermit {
+ public:
+  ResidentPermit() = default;
+  ~ResidentPermit() { release(); }
+  ResidentPermit(const ResidentPermit&) = delete;
+  ResidentPermit& operator=(const ResidentPermit&) = delete;
+  // False when the device (or the stream's CU mask) has fewer than `need` CUs.
+  bool acquire(int need, hipStream_t st);
+  void release();
+
+ private:
+  int dev_ = -1, held_ = 0;
+  hipStream_t st_ = nullptr;
+};
+
+struct ResidentSolve {
+  const void* vals;   // SELL values (T)
+  const void* binv;   // block-Jacobi inverses (T)
+  const uint8_t* fixed;
+  const double* g;    // right-hand side is -g on the free DOFs
+  double* dx;
+  double rtol, inner_rtol;
+  int max_iter, max_refine;
+  bool fp32;          // FP32 matrix with FP64 residual replacement
+};
+
+// Looks for (or builds) the plan of a simulator on mesh m and allocates the
+// exchange buffers; R.plan stays null when the mesh is not eligible.
+int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32);
+// Enqueues the run (without waiting); the result is in R.host once the stream
+// has been synchronized.
+int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st);
+// Number of neighbour vertices (itself included) of every vertex.
+void vertex_degrees(const int32_t* T, int64_t nv, int64_t nt, std::vector<int32_t>& deg);
+// The vertices by descending degree, ties in index order (sk_sell_order).
+void degree_order(const std::vector<int32_t>& deg, int32_t* order);
+
+}  // namespace sk

@@ -1,0 +1,1097 @@
+// Resident PCG (see sk_resident.h) and the vertex numbering it likes.
+#include "sk_resident.h"
+
+#include <algorithm>
+#include <cmath>
+#include <condition_variable>
+#include <mutex>
+#include <numeric>
+
+namespace sk {
+namespace {
+
+// ---------------------------------------------------------------------------
+// Exchange through self-tagged words: every 64-bit word carries 32 bits of
+// payload and the 32-bit number (epoch) of the exchange it belongs to, written
+// by one relaxed agent-scope store (which goes through to the memory all XCDs
+// share). A reader polls the words it needs until all carry the epoch, so data
+// and signal arrive in one trip: no flag, fence or cache invalidation.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ void put_word(uint64_t* p, uint32_t epoch, uint32_t v) {
+  __hip_atomic_store(p, ((uint64_t)epoch << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get_word(const uint64_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool tagged(uint64_t w, uint32_t epoch) { return (uint32_t)(w >> 32) == epoch; }
+
+// x, of unknown value to the compiler: what is computed from it inside the
+// iteration (addresses, unpacked fields) is not hoisted out of it into
+// registers that the matrix blocks need.
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
+// Words of a vertex's three components: used, and the stride between vertices
+// (a power of two, so that a vertex's words share one or half a 64-byte chunk).
+template <typename V>
+constexpr int kVertWords = 3 * (int)sizeof(V) / 4;
+template <typename V>
+constexpr int kVertStride = sizeof(V) == 8 ? 8 : 4;
+
+// Reduction slots: eight words (four FP64 sums) of one workgroup in a 64-byte
+// chunk, written by eight neighbouring threads and read by all threads
+// together in memory order. How the words lie decides what a meeting costs:
+// 256 workgroups exchanging ten words each took 4.0 us with one array per
+// word (every word of a workgroup on a line of its own) and 2.1 us this way.
+// The slots are written to kResCopies places, 128 KB apart, each read by a
+// quarter of the workgroups.
+constexpr int kSlotWords = 8;
+constexpr int kResCopies = 4;
+constexpr int kResCopyWords = 16384;
+static_assert(2 * kSlotWords * kResMaxParts <= kResCopyWords, "a copy holds both parities");
+
+template <typename T>
+struct ResidentArgs {
+  int G, K, KL, KS;
+  const int32_t* row0;
+  const int32_t* bptr;
+  const uint16_t* lcol;
+  const uint16_t* trow;
+  const int32_t* sell_pos;
+  const T* vals;
+  const T* binv;
+  const uint8_t* fixed;
+  const double* g;
+  double* x;
+  const int32_t* halo_ptr;
+  const int32_t* hvert;       // halo vertices
+  const int32_t* halo;        // place of each halo vertex among all exported vertices
+  const int32_t* exp0;        // [G + 1] exported vertices of the workgroups before this one
+  const uint16_t* exslot;     // partial slot of each exported vertex's row (see product)
+  uint64_t* slots;  // [kResCopies] x [2][G][kSlotWords]: parity, workgroup, word
+  uint64_t* zx;     // [exported vertices][kVertStride<T>]: A p (or a replaced residual)
+  uint64_t* xx;     // [exported vertices][8]: FP64 correction (kMixed)
+  T* stream;        // [G][KS][9][NT] streamed blocks
+  int* abort_flag;
+  ResidentResult* host;
+  uint32_t epoch;   // last epoch used so far
+  int max_rows, max_local, max_halo;
+  double rtol2, inner_rtol2;
+  int max_iter, max_refine;
+};
+
+// Ends a poll that has lasted kPollTicks (about two seconds of the 100 MHz
+// clock) or that another workgroup has ended: every wait is bounded, and the
+// host then solves by launches.
+constexpr long long kPollTicks = 200000000ll;
+struct Poll {
+  int n = 0;
+  long long t0 = 0;
+  __device__ __forceinline__ bool give_up(const int* abort_flag) {
+    if ((++n & 255) != 0) return false;
+    const long long now = wall_clock64();
+    if (t0 == 0) t0 = now;
+    return now - t0 > kPollTicks || __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+  }
+};
+
+// Barrier that orders LDS only: the workgroup's waves share nothing else inside
+// the loop, and __syncthreads would also wait for the words just stored.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// Sum over the wave in lane 63 (fixed tree of DPP row shifts and broadcasts).
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, kRows, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kCtrl, kRows, 0xf, true);
+  return v + __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: prefix sums of the rows of 16 lanes
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+
+// x + x of the lane 16 (32) away, in both.
+__device__ __forceinline__ double add_row_pair(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  return __longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1]));
+}
+__device__ __forceinline__ double add_half_pair(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)u, (uint32_t)u, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(u >> 32), (uint32_t)(u >> 32), false, false);
+  return __longlong_as_double((long long)(((uint64_t)hi[0] << 32) | lo[0])) +
+         __longlong_as_double((long long)(((uint64_t)hi[1] << 32) | lo[1]));
+}
+
+// One workgroup's view of the exchange.
+template <int NT>
+struct Meet {
+  static constexpr int nw = NT / kWave;
+  double* red;   // [4 nw] wave sums
+  double* tot;   // [4 nw] per-wave sums over the workgroups
+  int* bad;
+  uint64_t* slots;
+  int G;
+  int parity;
+  const int* abort_flag;
+  const int32_t* halo;  // [H] in LDS
+  int H;
+
+  // Wave sums of this thread's NV values into red (a barrier must follow before publish).
+  template <int NV>
+  __device__ __forceinline__ void wave_sums(const double (&v)[NV]) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const double s = wave_sum_last(v[k]);
+      if (threadIdx.x % kWave == kWave - 1) red[k * nw + threadIdx.x / kWave] = s;
+    }
+  }
+  __device__ __forceinline__ double local(int k) const {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < nw; ++w) s += red[k * nw + w];
+    return s;
+  }
+  // The workgroup's NV <= 4 sums, one word per thread.
+  template <int NV>
+  __device__ __forceinline__ void publish(uint32_t epoch) {
+    parity ^= 1;
+    const int w = threadIdx.x % kSlotWords, c = threadIdx.x / kSlotWords;
+    if (G > 1 && c < kResCopies && w < 2 * NV) {
+      const uint64_t u = (uint64_t)__double_as_longlong(local(w >> 1));
+      put_word(slots + (size_t)c * kResCopyWords + (parity * G + (int)blockIdx.x) * kSlotWords + w, epoch,
+               (w & 1) ? (uint32_t)(u >> 32) : (uint32_t)u);
+    }
+  }
+  // Waits for every workgroup's NV sums and (V not void) the words of the
+  // workgroup's halo vertices in `words`, which go to dest (3 V per vertex, in
+  // LDS). Each thread reads words NT apart; what has arrived is not read again.
+  // The sums' wave sums go to tot.
+  template <int NV, typename V>
+  __device__ __forceinline__ void collect(uint32_t epoch, const uint64_t* words, uint32_t* dest) {
+    constexpr int NS = NV > 0 ? kSlotWords * kResMaxParts / NT : 0;  // slot words per thread
+    constexpr int VS = kVertStride<V>, VW = kVertWords<V>;
+    constexpr int NH = sizeof(V) == 8 ? 8 : 5;                       // halo words per thread in flight
+    const int t = opaque(threadIdx.x), sw = t % kSlotWords, hw = t % VS;
+    const uint64_t* s = slots + (size_t)(blockIdx.x % kResCopies) * kResCopyWords + parity * G * kSlotWords + t;
+    const bool halos = words != nullptr;
+    uint32_t need = 0, sum[NS > 0 ? NS : 1];
+#pragma unroll
+    for (int k = 0; k < NS; ++k) {
+      sum[k] = 0;
+      if (G > 1 && sw < 2 * NV && (t + k * NT) / kSlotWords < G) need |= 1u << k;
+    }
+#pragma unroll
+    for (int k = 0; k < NH; ++k) {
+      if (halos && hw < VW && (t + k * NT) / VS < H) need |= 1u << (NS + k);
+    }
+    Poll poll;
+    while (need) {
+      uint64_t a[NS > 0 ? NS : 1], b[NH];
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+        if (need >> k & 1) a[k] = get_word(s + k * NT);
+#pragma unroll
+      for (int k = 0; k < NH; ++k)
+        if (need >> (NS + k) & 1) b[k] = get_word(words + (uint32_t)(halo[(t + k * NT) / VS] * VS + hw));
+#pragma unroll
+      for (int k = 0; k < NS; ++k)
+        if ((need >> k & 1) && tagged(a[k], epoch)) {
+          sum[k] = (uint32_t)a[k];
+          need &= ~(1u << k);
+        }
+#pragma unroll
+      for (int k = 0; k < NH; ++k)
+        if ((need >> (NS + k) & 1) && tagged(b[k], epoch)) {
+          dest[(t + k * NT) / VS * VW + hw] = (uint32_t)b[k];
+          need &= ~(1u << (NS + k));
+        }
+      if (need && poll.give_up(abort_flag)) {
+        *bad = 1;
+        break;
+      }
+    }
+    if (halos) {  // halos larger than NH words per thread
+      for (int j = t + NH * NT; j < H * VS; j += NT) {
+        if (hw >= VW) break;
+        const uint64_t* p = words + (size_t)halo[j / VS] * VS + hw;
+        uint64_t w = get_word(p);
+        while (!tagged(w, epoch)) {
+          if (poll.give_up(abort_flag)) {
+            *bad = 1;
+            break;
+          }
+          w = get_word(p);
+        }
+        dest[j / VS * VW + hw] = (uint32_t)w;
+      }
+    }
+    if constexpr (NV > 0) {
+      if (G == 1) {
+        if ((int)threadIdx.x < nw * NV)
+          tot[threadIdx.x] = threadIdx.x % nw == 0 ? local(threadIdx.x / nw) : 0.0;
+      } else {
+        double d = 0.0;  // both threads of a pair add the pair's double of every slot they read
+#pragma unroll
+        for (int k = 0; k < NS; ++k) {
+          const uint32_t other = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sum[k], 0xB1, 0xf, 0xf, true);
+          const uint32_t lo = (t & 1) ? other : sum[k], hi = (t & 1) ? sum[k] : other;
+          d += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+        }
+        d = dpp_add<0x128, 0xf>(d);  // row_ror 8: the other slot of the row of 16 lanes
+        d = add_half_pair(add_row_pair(d));
+        const int lane = threadIdx.x % kWave;
+        if (lane < 2 * NV && lane % 2 == 0) tot[lane / 2 * nw + threadIdx.x / kWave] = d;
+      }
+    }
+  }
+  // Totals over all workgroups (after the barrier that follows collect).
+  template <int NV>
+  __device__ __forceinline__ void totals(double (&v)[NV]) const {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < nw; ++w) s += tot[k * nw + w];
+      v[k] = s;
+    }
+  }
+};
+
+// Block-Jacobi PCG on H dx = -g (free DOFs), x0 = 0, of one whole run:
+// kMixed = false in T = double to ||r|| <= rtol ||b||; kMixed in T = float with
+// FP64 residual replacement each time the FP32 residual has dropped by
+// inner_rtol, to ||b - A dx|| <= rtol ||b|| in FP64 (the scheme of
+// run_mixed_solve).
+//
+// A workgroup owns a contiguous range of rows; workgroups of one XCD own
+// neighbouring ranges. The rows' matrix blocks, in row order, are dealt K
+// consecutive ones to a thread, which holds the first KR in registers, the
+// next KL in LDS and the last KS in a private global array that L2 serves. The
+// product leaves one partial per (row, thread) pair in LDS at slot row + thread
+// (consecutive for a row, since both only grow along the block list), which
+// the row's thread then sums in order. r and p of the rows and of their halo
+// (the vertices of other workgroups they couple to) live in LDS.
+//
+// One meeting per iteration: after the product every workgroup publishes its
+// exported rows' A p and its shares of
+//   p.Ap, Ap.B^-1 Ap, r.z, r.r   (z = B^-1 r),
+// so that everybody knows alpha = r.z / p.Ap, beta by the next r.z =
+// alpha^2 Ap.B^-1 Ap - r.z (with z.Ap = p.Ap), and the stopping test on r.r,
+// and then updates r, z and p of its own rows and of its halo alike (the same
+// operations on the same values, so that the copies of p never differ). r.z in
+// alpha and r.r are direct sums of the current residual: the expansion enters
+// beta only. Iteration counts at 48^3 equal the two-launch form's (2,731 and
+// 2,837 over a step in FP64 and mixed precision).
+// All workgroups sum the same words in the same order and take the same
+// decisions; results are bit-reproducible for a fixed cut.
+//
+// Why: the two-launch form reads 107 MB (FP64) of values per iteration and
+// pays two launch boundaries; 256 CUs hold 128 MB in registers and 40 MB in
+// LDS, so nothing but the halo has to move. Measured per iteration over a
+// whole step, launches then this kernel: 48^3 FP64 30.8 -> 11.3 us, mixed 20.9
+// -> 8.4; 32^3 mixed 12.6 -> 6.4; 10^3 FP64 11.9 -> 6.0 us. What bounds it is
+// the meeting (about 3.5 us at 256 workgroups, 1.5 us at 8) and the latency of
+// the phases between barriers.
+template <typename T, int NT, int KR, bool kMixed>
+__global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs<T> a) {
+  extern __shared__ double dyn[];
+  __shared__ double s_red[4 * (NT / kWave)];
+  __shared__ double s_tot[4 * (NT / kWave)];
+  __shared__ int s_bad;
+  using PV = std::conditional_t<kMixed, double, T>;  // partials
+  const int t = threadIdx.x;
+  // workgroup b runs on XCD b % 8: neighbouring parts there, so that most halo words stay in its L2
+  const int me = a.G % 8 == 0 ? (blockIdx.x % 8) * (a.G / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int v0 = a.row0[me], R = a.row0[me + 1] - v0;
+  const int b0 = a.bptr[v0], nb = a.bptr[v0 + R] - b0;
+  const int h0 = a.halo_ptr[me], H = a.halo_ptr[me + 1] - h0;
+  const int x0 = a.exp0[me], E = a.exp0[me + 1] - x0;
+  const int K = a.K;
+  PV* part = reinterpret_cast<PV*>(dyn);                              // [max_rows + NT + 1][3]
+  double* P64 = reinterpret_cast<double*>(part + 3 * (a.max_rows + NT + 1));  // [max_local][3] (kMixed)
+  T* P = reinterpret_cast<T*>(P64 + (kMixed ? 3 * a.max_local : 0));  // [max_local][3]
+  T* RL = P + 3 * a.max_local;                                        // [max_local][3] r
+  T* HA = RL + 3 * a.max_local;                                       // [max_halo][3] what the halo's owners sent
+  T* XL = HA + 3 * a.max_halo;                                        // [max_rows][3] x (kMixed; else in a.x)
+  T* L = XL + (kMixed ? 3 * a.max_rows : 0);                          // [KL][9][NT]
+  int32_t* HX = reinterpret_cast<int32_t*>(L + (size_t)9 * NT * a.KL);  // [max_halo] places of the halo vertices
+  uint16_t* EX = reinterpret_cast<uint16_t*>(HX + a.max_halo);        // [NT] partial slots of the exported rows
+  T* S = a.stream + (size_t)me * a.KS * 9 * NT;
+  if (t == 0) s_bad = 0;
+
+  // the thread's blocks and their words (local column << 1 | last of its row)
+  T A[KR][9];
+  uint32_t meta[(KR + 2 * kResMaxTier + 1) / 2];
+#pragma unroll
+  for (int k = 0; k < (KR + 2 * kResMaxTier + 1) / 2; ++k) meta[k] = 0;
+  const int tb0 = t * K;
+  auto load_block = [&](int k, T (&B)[9]) -> uint32_t {
+#pragma unroll
+    for (int m = 0; m < 9; ++m) B[m] = T(0);
+    if (k >= K || tb0 + k >= nb) return 0;
+    const int b = b0 + tb0 + k;
+    const int64_t q = a.sell_pos[b];
+#pragma unroll
+    for (int m = 0; m < 9; ++m) B[m] = a.vals[slot_index<kSellC, 1>(q, m)];
+    return a.lcol[b];
+  };
+  auto word = [&](int k) { return (meta[k / 2] >> (16 * (k & 1))) & 0xffffu; };
+#pragma unroll
+  for (int k = 0; k < KR; ++k) meta[k / 2] |= load_block(k, A[k]) << (16 * (k & 1));
+#pragma unroll
+  for (int k = 0; k < kResMaxTier; ++k)
+    if (k < a.KL) {
+      T B[9];
+      meta[(KR + k) / 2] |= load_block(KR + k, B) << (16 * ((KR + k) & 1));
+#pragma unroll
+      for (int m = 0; m < 9; ++m) L[(k * 9 + m) * NT + t] = B[m];
+    }
+#pragma unroll
+  for (int k = 0; k < kResMaxTier; ++k)
+    if (k < a.KS) {
+      T B[9];
+      constexpr int k0 = KR + kResMaxTier;
+      meta[(k0 + k) / 2] |= load_block(KR + a.KL + k, B) << (16 * ((k0 + k) & 1));
+#pragma unroll
+      for (int m = 0; m < 9; ++m) S[(k * 9 + m) * NT + t] = B[m];
+    }
+  const int slot0 = (int)a.trow[me * NT + t] + t;
+
+  // y = A src for the workgroup's rows, as partials. The source entries of the
+  // next U blocks are read before the current U are multiplied: the partials'
+  // stores would otherwise keep every block's LDS reads behind the last block's.
+  auto product = [&](const auto* __restrict__ src) {
+    using V = std::remove_cv_t<std::remove_reference_t<decltype(src[0])>>;
+    constexpr int U = sizeof(V) == 8 ? 2 : 4;
+#pragma unroll
+    for (int k = 0; k < (KR + 2 * kResMaxTier + 1) / 2; ++k) meta[k] = (uint32_t)opaque((int)meta[k]);
+    const int tt = opaque(t);
+    V y0 = 0, y1 = 0, y2 = 0;
+    PV* o = part + 3 * slot0;
+    auto read = [&](uint32_t lm, V (&p)[3]) {
+      const V* q = src + 3 * (lm >> 1);
+      p[0] = q[0];
+      p[1] = q[1];
+      p[2] = q[2];
+    };
+    auto add = [&](const T (&B)[9], const V (&p)[3], uint32_t lm) {
+      y0 = fma((V)B[2], p[2], fma((V)B[1], p[1], fma((V)B[0], p[0], y0)));
+      y1 = fma((V)B[5], p[2], fma((V)B[4], p[1], fma((V)B[3], p[0], y1)));
+      y2 = fma((V)B[8], p[2], fma((V)B[7], p[1], fma((V)B[6], p[0], y2)));
+      if (lm & 1) {
+        o[0] = (PV)y0;
+        o[1] = (PV)y1;
+        o[2] = (PV)y2;
+        o += 3;
+        y0 = y1 = y2 = V(0);
+      }
+    };
+    T B0[9];  // the first streamed block, on its way during the others
+    if (a.KS > 0) {
+#pragma unroll
+      for (int m = 0; m < 9; ++m) B0[m] = S[m * NT + tt];
+    }
+    V p[2][U][3];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < KR) read(word(u), p[0][u]);
+#pragma unroll
+    for (int k = 0; k < KR; k += U) {
+      if (k < K) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (k + U + u < KR) read(word(k + U + u), p[(k / U + 1) & 1][u]);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (k + u < KR) add(A[k + u], p[(k / U) & 1][u], word(k + u));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kResMaxTier; ++k)
+      if (k < a.KL) {
+        T B[9];
+        V q[3];
+        read(word(KR + k), q);
+#pragma unroll
+        for (int m = 0; m < 9; ++m) B[m] = L[(k * 9 + m) * NT + tt];
+        add(B, q, word(KR + k));
+      }
+    if (a.KS > 0) {
+      V q[3];
+      read(word(KR + kResMaxTier), q);
+      add(B0, q, word(KR + kResMaxTier));
+    }
+#pragma unroll
+    for (int k = 1; k < kResMaxTier; ++k)
+      if (k < a.KS) {
+        T B[9];
+        V q[3];
+        read(word(KR + kResMaxTier + k), q);
+#pragma unroll
+        for (int m = 0; m < 9; ++m) B[m] = S[(k * 9 + m) * NT + tt];
+        add(B, q, word(KR + kResMaxTier + k));
+      }
+    o[0] = (PV)y0;  // the open row's partial (or a slot that no row reads)
+    o[1] = (PV)y1;
+    o[2] = (PV)y2;
+  };
+
+  // the thread's row
+  const bool row = t < R;
+  const int v = v0 + t;
+  int s0 = 0, s1 = -1, fx = 7;
+  if (row) {
+    const int o0 = a.bptr[v] - b0, o1 = a.bptr[v + 1] - b0;
+    s0 = t + o0 / K;
+    s1 = t + (o1 - 1) / K;
+    fx = 0;
+    if (a.fixed) fx = (a.fixed[3 * v] ? 1 : 0) | (a.fixed[3 * v + 1] ? 2 : 0) | (a.fixed[3 * v + 2] ? 4 : 0);
+  }
+  auto rhs = [&](int q) { return (!row || ((fx >> q) & 1)) ? 0.0 : -a.g[3 * (int64_t)v + q]; };
+  auto row_sum = [&](PV (&y)[3]) {
+    // a row rarely spans more than kSpan threads: that many reads at once, then the rest
+    constexpr int kSpan = 5;
+    PV w[kSpan][3];
+#pragma unroll
+    for (int k = 0; k < kSpan; ++k)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[k][q] = part[3 * (s0 + k < s1 ? s0 + k : s1) + q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      y[q] = w[0][q];
+#pragma unroll
+      for (int k = 1; k < kSpan; ++k) y[q] += s0 + k <= s1 ? w[k][q] : PV(0);
+    }
+    for (int s = s0 + kSpan; s <= s1; ++s) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) y[q] += part[3 * s + q];
+    }
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if ((fx >> q) & 1) y[q] = PV(0);
+  };
+  // B^-1 of a vertex: read again each iteration rather than kept (the product needs the registers)
+  auto load_binv = [&](int64_t vertex, T (&B)[kBinv]) {
+#pragma unroll
+    for (int k = 0; k < kBinv; ++k) B[k] = a.binv[kBinv * vertex + k];
+  };
+  // z = B^-1 r and p = z + beta p, in one order of operations for owners and halos
+  auto precondition = [&](const T (&B)[kBinv], const T (&r)[3], T (&z)[3]) {
+    z[0] = fma(B[2], r[2], fma(B[1], r[1], B[0] * r[0]));
+    z[1] = fma(B[4], r[2], fma(B[3], r[1], B[1] * r[0]));
+    z[2] = fma(B[5], r[2], fma(B[4], r[1], B[2] * r[0]));
+  };
+  auto direction = [&](int l, const T (&B)[kBinv], const T (&r)[3], T beta) {
+    T z[3];
+    precondition(B, r, z);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) P[3 * l + q] = fma(beta, P[3 * l + q], z[q]);
+  };
+  // The exported rows' three values, staged in the rows' own partial slots, by all threads in word order
+  // (after a barrier).
+  auto put_exports = [&](auto tag, uint64_t* words, uint32_t epoch) {
+    using V = decltype(tag);
+    constexpr int VS = kVertStride<V>, VW = kVertWords<V>;
+    for (int j = t; j < E * VS; j += NT) {
+      const int w = j % VS;
+      if (w >= VW) continue;
+      const PV* src = part + 3 * EX[j / VS];
+      uint32_t u;
+      if constexpr (sizeof(V) == 8) u = reinterpret_cast<const uint32_t*>(src)[w];
+      else u = __float_as_uint((float)src[w]);
+      put_word(words + (size_t)x0 * VS + j, epoch, u);
+    }
+  };
+  for (int j = t; j < H; j += NT) HX[j] = a.halo[h0 + j];
+  for (int j = t; j < E; j += NT) EX[j] = a.exslot[x0 + j];
+  const int hv = t < H ? a.hvert[h0 + t] : 0;
+
+  // start: r = b, x = 0, p = z
+  double acc0[1] = {0.0};
+  if (row) {
+    T B[kBinv], r[3];
+    load_binv(v, B);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const double b = rhs(q);
+      acc0[0] += b * b;
+      r[q] = (T)b;
+      RL[3 * t + q] = r[q];
+      if (kMixed) XL[3 * t + q] = T(0);
+      else a.x[3 * (int64_t)v + q] = 0.0;
+      P[3 * t + q] = T(0);
+    }
+    direction(t, B, r, T(0));
+  }
+  for (int j = t; j < H; j += NT) {
+    const int64_t w = a.hvert[h0 + j];
+    T B[kBinv], r[3];
+    load_binv(w, B);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      r[q] = (a.fixed && a.fixed[3 * w + q]) ? T(0) : (T)-a.g[3 * w + q];
+      RL[3 * (R + j) + q] = r[q];
+      P[3 * (R + j) + q] = T(0);
+    }
+    direction(R + j, B, r, T(0));
+  }
+
+  Meet<NT> meet{s_red, s_tot, &s_bad, a.slots, a.G, 0, a.abort_flag, HX, H};
+  uint32_t epoch = a.epoch;
+  int iter = 0, done = 0, refines = 0;
+  double tol2 = 0.0, target = 0.0;
+  bool fresh = true;  // the tolerance starts from this residual
+  __syncthreads();
+  if (kMixed) {  // ||b||^2 in FP64
+    meet.template wave_sums<1>(acc0);
+    lds_barrier();
+    meet.template publish<1>(++epoch);
+    meet.template collect<1, T>(epoch, nullptr, nullptr);
+    lds_barrier();
+    meet.template totals<1>(acc0);
+    target = a.rtol2 * acc0[0];
+  }
+  const bool start = !kMixed || acc0[0] > 0.0;
+  if (!start) done = acc0[0] == 0.0 ? 1 : 3;
+  for (bool go = start && !s_bad; go;) {
+    product(P);
+    T B[kBinv], r[3], ap[3];
+    load_binv(row ? opaque(v) : 0, B);
+    lds_barrier();
+    double va[4] = {0.0, 0.0, 0.0, 0.0};
+    ++epoch;
+    if (row) {
+      PV y[3];
+      row_sum(y);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        ap[q] = (T)y[q];
+        part[3 * s0 + q] = (PV)ap[q];  // staged for put_exports in the row's own slot
+        r[q] = RL[3 * t + q];
+      }
+      T z[3], u[3];
+      precondition(B, r, z);
+      precondition(B, ap, u);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        va[0] += (double)P[3 * t + q] * (double)ap[q];
+        va[1] += (double)u[q] * (double)ap[q];
+        va[2] += (double)r[q] * (double)z[q];
+        va[3] += (double)r[q] * (double)r[q];
+      }
+    }
+    meet.template wave_sums<4>(va);
+    lds_barrier();
+    meet.template publish<4>(epoch);
+    put_exports(T(0), a.zx, epoch);
+    meet.template collect<4, T>(epoch, a.zx, reinterpret_cast<uint32_t*>(HA));
+    T BH[kBinv];
+    load_binv(row ? opaque(v) : 0, B);
+    load_binv(opaque(hv), BH);
+    double xg[3];
+    if (!kMixed && row) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) xg[q] = a.x[3 * (int64_t)opaque(v) + q];
+    }
+    lds_barrier();
+    if (s_bad) break;
+    meet.template totals<4>(va);
+    const double pAp = va[0], rz = va[2], rr = va[3];
+    if (fresh) tol2 = (kMixed ? a.inner_rtol2 : a.rtol2) * rr;
+    fresh = false;
+    if (!(isfinite(rr) && isfinite(rz))) {
+      done = 3;
+      break;
+    }
+    const bool conv = !(rr > tol2), limit = iter >= a.max_iter;
+    if (conv || limit) {
+      if constexpr (!kMixed) {
+        done = conv ? 1 : 0;
+        break;
+      } else {
+        // residual replacement: dx += x and r = b - A dx in FP64. p was formed from the old r; with the new
+        // one, z + beta p_before is z + (r.z / old r.z) (p - old z).
+        ++epoch;
+        ++refines;
+        if (row) {
+          double x64[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            double& dx = a.x[3 * (int64_t)v + q];
+            x64[q] = refines == 1 ? (double)XL[3 * t + q] : dx + (double)XL[3 * t + q];
+            dx = x64[q];
+            XL[3 * t + q] = T(0);
+            P64[3 * t + q] = x64[q];
+            part[3 * s0 + q] = x64[q];
+          }
+        }
+        lds_barrier();
+        put_exports(double(0), a.xx, epoch);
+        meet.template collect<0, double>(epoch, a.xx, reinterpret_cast<uint32_t*>(P64 + 3 * R));
+        lds_barrier();
+        if (s_bad) break;
+        product(P64);
+        lds_barrier();
+        double vb[2] = {0.0, 0.0};
+        ++epoch;
+        if (row) {
+          PV y[3];
+          row_sum(y);
+          T z[3];
+          load_binv(v, B);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const double rq = ((fx >> q) & 1) ? 0.0 : rhs(q) - (double)y[q];
+            vb[0] += rq * rq;
+            r[q] = (T)rq;
+            part[3 * s0 + q] = (PV)r[q];
+          }
+          precondition(B, r, z);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) vb[1] += (double)r[q] * (double)z[q];
+        }
+        meet.template wave_sums<2>(vb);
+        lds_barrier();
+        meet.template publish<2>(epoch);
+        put_exports(T(0), a.zx, epoch);
+        meet.template collect<2, T>(epoch, a.zx, reinterpret_cast<uint32_t*>(HA));
+        lds_barrier();
+        if (s_bad) break;
+        meet.template totals<2>(vb);
+        if (!(vb[0] > target) || refines >= a.max_refine || limit) {
+          done = vb[0] <= target ? 1 : isfinite(vb[0]) ? 0 : 3;
+          break;
+        }
+        const T ratio = (T)(vb[1] / rz);
+        auto replace = [&](int l, const T (&Bl)[kBinv], const T (&rn)[3]) {
+          T ro[3], zo[3], zn[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) ro[q] = RL[3 * l + q];
+          precondition(Bl, ro, zo);
+          precondition(Bl, rn, zn);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            P[3 * l + q] = fma(ratio, P[3 * l + q] - zo[q], zn[q]);
+            RL[3 * l + q] = rn[q];
+          }
+        };
+        if (row) replace(t, B, r);
+        for (int j = t; j < H; j += NT) {
+          const T hr[3] = {HA[3 * j], HA[3 * j + 1], HA[3 * j + 2]};
+          load_binv(a.hvert[h0 + j], BH);
+          replace(R + j, BH, hr);
+        }
+        fresh = true;
+        lds_barrier();
+        continue;
+      }
+    }
+    if (!(pAp > 0.0)) {
+      done = isfinite(pAp) ? 2 : 3;
+      break;
+    }
+    const double inv_pAp = 1.0 / pAp, inv_rz = 1.0 / rz;  // side by side
+    const T alpha = (T)(rz * inv_pAp);
+    // with alpha as rounded for the update: r.z of the residual that it leaves
+    const double al = (double)alpha, rz_next = al * al * va[1] - rz;
+    const T beta = (T)(rz_next > 0.0 ? rz_next * inv_rz : 0.0);
+    ++iter;
+    if (row) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        if (kMixed) XL[3 * t + q] = fma(alpha, P[3 * t + q], XL[3 * t + q]);
+        else a.x[3 * (int64_t)v + q] = fma((double)alpha, (double)P[3 * t + q], xg[q]);
+        r[q] = fma(-alpha, ap[q], RL[3 * t + q]);
+        RL[3 * t + q] = r[q];
+      }
+      direction(t, B, r, beta);
+    }
+    for (int j = t; j < H; j += NT) {
+      if (j != t) load_binv(a.hvert[h0 + j], BH);
+      T rh[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        rh[q] = fma(-alpha, HA[3 * j + q], RL[3 * (R + j) + q]);
+        RL[3 * (R + j) + q] = rh[q];
+      }
+      direction(R + j, BH, rh, beta);
+    }
+    lds_barrier();
+  }
+  __syncthreads();
+  if (s_bad) {
+    if (t == 0) {
+      __hip_atomic_store(a.abort_flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      a.host->aborted = 1;
+    }
+    return;
+  }
+  if (kMixed && row && refines == 0) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) a.x[3 * (int64_t)v + q] = 0.0;
+  }
+  if (blockIdx.x == 0 && t == 0) {
+    a.host->iter = iter;
+    a.host->done = done;
+    a.host->refines = refines;
+    a.host->epoch = epoch;
+  }
+}
+
+__global__ void resident_clear_kernel(int64_t n, uint64_t* p) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
+int clear_words(DevBuf<uint64_t>& b, hipStream_t st) {
+  if (b.n) resident_clear_kernel<<<grid_for((int64_t)b.n), kBlock, 0, st>>>((int64_t)b.n, b.p);
+  SK_HIP_CHECK(hipGetLastError());
+  return SK_OK;
+}
+
+// Dynamic LDS without the matrix tiers, and of one tier block per thread.
+size_t base_lds(bool fp32, int max_rows, int max_local, int max_halo) {
+  const int NT = fp32 ? kResNT32 : kResNT64;
+  const size_t v = fp32 ? 12 : 24;
+  return 24 * (size_t)(max_rows + NT + 1) + (fp32 ? 24 * (size_t)max_local + 12 * (size_t)max_rows : 0) +
+         2 * v * max_local + v * max_halo + 4 * (size_t)max_halo + 2 * (size_t)NT + 64;
+}
+size_t tier_lds(bool fp32) { return (fp32 ? kResNT32 : kResNT64) * (9 * (fp32 ? 4 : 8)) * (size_t)1; }
+
+struct Permits {
+  std::mutex mu;
+  std::condition_variable cv;
+  int used = 0, cus = -1;
+};
+Permits g_permits[64];
+
+}  // namespace
+
+ResidentState::~ResidentState() {
+  if (host) (void)hipHostFree(host);
+}
+
+bool ResidentPermit::acquire(int need, hipStream_t st) {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
+  // a stream restricted to some CUs
+  uint32_t mask[16] = {};
+  if (hipExtStreamGetCUMask(st, 16, mask) == hipSuccess) {
+    int n = 0;
+    for (uint32_t w : mask) n += __builtin_popcount(w);
+    if (n < need) return false;
+  } else {
+    (void)hipGetLastError();
+  }
+  Permits& P = g_permits[dev];
+  std::unique_lock<std::mutex> lock(P.mu);
+  if (P.cus < 0) {
+    int n = 0;
+    P.cus = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
+  }
+  if (need > P.cus) return false;
+  P.cv.wait(lock, [&] { return P.used + need <= P.cus; });
+  P.used += need;
+  dev_ = dev;
+  held_ = need;
+  st_ = st;
+  return true;
+}
+
+void ResidentPermit::release() {
+  if (!held_) return;
+  // a step that ends early (an error) may not have waited for the run yet
+  if (hipStreamQuery(st_) != hipSuccess) {
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(st_);
+  }
+  Permits& P = g_permits[dev_];
+  {
+    std::lock_guard<std::mutex> lock(P.mu);
+    P.used -= held_;
+  }
+  P.cv.notify_all();
+  held_ = 0;
+}
+
+int resident_parts(int64_t nv, int64_t nblk, bool fp32) {
+  const int NT = fp32 ? kResNT32 : kResNT64, KR = fp32 ? kResKR32 : kResKR64;
+  // at least enough workgroups that a row has a thread (with 10% for an uneven cut)
+  const int64_t need = (11 * nv + 10 * NT - 1) / (10 * (int64_t)NT);
+  int64_t G = nv <= NT ? 1 : need;
+  // and few blocks per thread
+  const int64_t target = (int64_t)NT * (KR < 8 ? KR : 8) / 2;
+  G = std::max(G, (nblk + target - 1) / target);
+  if (G > kResMaxParts) G = kResMaxParts;
+  if (nv > (int64_t)G * NT) return 0;
+  return (int)std::max<int64_t>(G, 1);
+}
+
+static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<int32_t>& parts, bool fp32, int* status) {
+  *status = SK_OK;
+  const int NT = fp32 ? kResNT32 : kResNT64, KR = fp32 ? kResKR32 : kResKR64;
+  const int G = (int)parts.size() - 1;
+  const int32_t *bptr = m->h_bptr.data(), *bcol = m->h_bcol.data();
+  auto p = std::make_shared<ResidentPlan>();
+  p->parts = parts;
+  p->fp32 = fp32;
+  p->G = G;
+  int max_nb = 0;
+  for (int g = 0; g < G; ++g) {
+    p->max_rows = std::max(p->max_rows, parts[g + 1] - parts[g]);
+    max_nb = std::max(max_nb, bptr[parts[g + 1]] - bptr[parts[g]]);
+  }
+  if (p->max_rows > NT) return nullptr;
+  p->K = std::max(1, (max_nb + NT - 1) / NT);
+  std::vector<int32_t> loc(m->nv, -1), halo_ptr(1, 0), halo;
+  std::vector<int16_t> place(m->nv, -1);
+  std::vector<int32_t> owner(m->nv), exp0(1, 0);
+  for (int g = 0; g < G; ++g)
+    for (int32_t r = parts[g]; r < parts[g + 1]; ++r) owner[r] = g;
+  std::vector<uint16_t> lcol(m->nblk), trow((size_t)G * NT);
+  std::vector<int32_t> mine;
+  for (int g = 0; g < G; ++g) {
+    const int32_t r0 = parts[g], r1 = parts[g + 1];
+    mine.clear();
+    for (int32_t b = bptr[r0]; b < bptr[r1]; ++b) {
+      const int32_t w = bcol[b];
+      if ((w < r0 || w >= r1) && loc[w] < 0) {
+        loc[w] = 0;
+        mine.push_back(w);
+      }
+    }
+    std::sort(mine.begin(), mine.end());
+    const int rows = r1 - r0, local = rows + (int)mine.size();
+    p->max_local = std::max(p->max_local, local);
+    p->max_halo = std::max(p->max_halo, (int)mine.size());
+    if (local > 32767) return nullptr;
+    for (size_t i = 0; i < mine.size(); ++i) {
+      loc[mine[i]] = rows + (int)i;
+      place[mine[i]] = 0;
+    }
+    int tk = 0;  // next thread whose first row is to be noted
+    for (int32_t r = r0; r < r1; ++r) {
+      for (int32_t b = bptr[r]; b < bptr[r + 1]; ++b) {
+        const int32_t w = bcol[b];
+        const int c = w >= r0 && w < r1 ? w - r0 : loc[w];
+        lcol[b] = (uint16_t)((c << 1) | (b + 1 == bptr[r + 1] ? 1 : 0));
+      }
+      for (; tk < NT && tk * p->K < bptr[r + 1] - bptr[r0]; ++tk) trow[(size_t)g * NT + tk] = (uint16_t)(r - r0);
+    }
+    for (; tk < NT; ++tk) trow[(size_t)g * NT + tk] = (uint16_t)rows;
+    for (int32_t w : mine) loc[w] = -1;
+    halo.insert(halo.end(), mine.begin(), mine.end());
+    halo_ptr.push_back((int32_t)halo.size());
+  }
+  // the exported vertices' places in their owners' lists, and the halos by them
+  for (int g = 0; g < G; ++g) {
+    int16_t e = 0;
+    for (int32_t r = parts[g]; r < parts[g + 1]; ++r)
+      if (place[r] >= 0) place[r] = e++;
+    exp0.push_back(exp0.back() + e);
+  }
+  p->n_exp = exp0.back();
+  std::vector<int32_t> where(std::max<size_t>(1, halo.size()), 0);
+  for (size_t i = 0; i < halo.size(); ++i) where[i] = exp0[owner[halo[i]]] + place[halo[i]];
+  std::vector<uint16_t> exslot(std::max(1, p->n_exp), 0);
+  for (int64_t v = 0; v < m->nv; ++v)
+    if (place[v] >= 0) {
+      const int32_t r0 = parts[owner[v]];
+      exslot[exp0[owner[v]] + place[v]] = (uint16_t)(v - r0 + (bptr[v] - bptr[r0]) / p->K);
+    }
+  const size_t base = base_lds(fp32, p->max_rows, p->max_local, p->max_halo) + kResStaticLds;
+  if (base > (size_t)kResLds) return nullptr;
+  const int rest = std::max(0, p->K - KR);
+  p->KL = (int)std::min<size_t>(std::min(rest, kResMaxTier), (kResLds - base) / tier_lds(fp32));
+  p->KS = rest - p->KL;
+  if (p->KS > kResMaxTier) return nullptr;
+  p->lds = base - kResStaticLds + p->KL * tier_lds(fp32);
+  // more than half of a CU's LDS: one workgroup per CU, so the runs spread over the chip
+  p->lds = std::max<size_t>(p->lds, kResLds / 2 + 1024);
+  std::vector<int32_t> row0(parts);
+  auto up = [&]() -> int {
+    SK_TRY(p->row0.upload(row0));
+    SK_TRY(p->lcol.upload(lcol));
+    SK_TRY(p->trow.upload(trow));
+    SK_TRY(p->halo_ptr.upload(halo_ptr));
+    SK_TRY(p->halo.upload(where));
+    SK_TRY(p->hvert.upload(halo));
+    SK_TRY(p->exp0.upload(exp0));
+    SK_TRY(p->exslot.upload(exslot));
+    return SK_OK;
+  };
+  *status = up();
+  return *status == SK_OK ? p : nullptr;
+}
+
+int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32) {
+  if (R.tried) return SK_OK;
+  R.tried = true;
+  std::vector<int32_t> parts = R.parts;
+  if (parts.empty()) {
+    const int G = resident_parts(m->nv, m->nblk, fp32);
+    if (G == 0) return SK_OK;
+    for (int g = 0; g <= G; ++g) parts.push_back((int32_t)(m->nv * g / G));
+  }
+  std::shared_ptr<ResidentPlan> plan;
+  {
+    std::lock_guard<std::mutex> lock(m->plan_mu);
+    for (auto& p : m->plans)
+      if (p->fp32 == fp32 && p->parts == parts) plan = p;
+    if (!plan) {
+      int s = SK_OK;
+      plan = build_plan(m, parts, fp32, &s);
+      if (s != SK_OK) return s;
+      if (plan) {
+        if (m->plans.size() >= 4) m->plans.erase(m->plans.begin());
+        m->plans.push_back(plan);
+      }
+    }
+  }
+  if (!plan) return SK_OK;
+  const int NT = fp32 ? kResNT32 : kResNT64;
+  SK_TRY(R.slots.alloc((size_t)kResCopies * kResCopyWords));
+  const size_t nx = std::max(1, plan->n_exp);
+  SK_TRY(R.zx.alloc(nx * (fp32 ? kVertStride<float> : kVertStride<double>)));
+  if (fp32) SK_TRY(R.xx.alloc(nx * kVertStride<double>));
+  SK_TRY(R.stream.alloc(std::max<size_t>(16, (size_t)plan->G * plan->KS * 9 * NT * (fp32 ? 4 : 8))));
+  SK_TRY(R.abort_flag.alloc(1));
+  SK_HIP_CHECK(hipMemset(R.slots.p, 0, R.slots.n * 8));
+  SK_HIP_CHECK(hipMemset(R.zx.p, 0, R.zx.n * 8));
+  if (fp32) SK_HIP_CHECK(hipMemset(R.xx.p, 0, R.xx.n * 8));
+  SK_HIP_CHECK(hipMemset(R.abort_flag.p, 0, sizeof(int)));
+  SK_HIP_CHECK(hipDeviceSynchronize());
+  SK_HIP_CHECK(hipHostMalloc((void**)&R.host, sizeof(ResidentResult), hipHostMallocCoherent));
+  *R.host = ResidentResult{};
+  R.epoch = 0;
+  R.plan = plan;
+  return SK_OK;
+}
+
+template <typename T, int NT, int KR, bool kMixed>
+static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st) {
+  const ResidentPlan& p = *R.plan;
+  ResidentArgs<T> a{p.G, p.K, p.KL, p.KS, p.row0.p, m->bptr.p, p.lcol.p, p.trow.p, m->sell_pos.p, (const T*)s.vals,
+                    (const T*)s.binv, s.fixed, s.g, s.dx, p.halo_ptr.p, p.hvert.p, p.halo.p, p.exp0.p, p.exslot.p, R.slots.p, R.zx.p,
+                    R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
+                    p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
+  resident_pcg_kernel<T, NT, KR, kMixed><<<p.G, NT, p.lds, st>>>(a);
+  SK_HIP_CHECK(hipGetLastError());
+  return SK_OK;
+}
+
+int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st) {
+  if (R.host->epoch > R.epoch) R.epoch = R.host->epoch;
+  if (R.epoch > 0x70000000u) {  // tags start over long before they wrap
+    SK_TRY(clear_words(R.slots, st));
+    SK_TRY(clear_words(R.zx, st));
+    SK_TRY(clear_words(R.xx, st));
+    R.epoch = 0;
+  }
+  *R.host = ResidentResult{0, 0, 0, 0, R.epoch};
+  return s.fp32 ? launch<float, kResNT32, kResKR32, true>(R, m, s, st)
+                : launch<double, kResNT64, kResKR64, false>(R, m, s, st);
+}
+
+
+}  // namespace sk
+
+using namespace sk;
+
+extern "C" {
+
+// Recursive coordinate bisection: vertices [lo, hi) of idx into parts [g0, g1).
+static void bisect(const double* X, const std::vector<float>& w, std::vector<int32_t>& idx, int64_t lo, int64_t hi,
+                   int g0, int g1, int32_t* ptr) {
+  if (g1 - g0 == 1) {
+    ptr[g0] = (int32_t)lo;
+    return;
+  }
+  double mn[3], mx[3];
+  for (int c = 0; c < 3; ++c) mn[c] = 1e300, mx[c] = -1e300;
+  double total = 0.0;
+  for (int64_t i = lo; i < hi; ++i) {
+    const double* x = X + 3 * (int64_t)idx[i];
+    total += w[idx[i]];
+    for (int c = 0; c < 3; ++c) {
+      mn[c] = std::min(mn[c], x[c]);
+      mx[c] = std::max(mx[c], x[c]);
+    }
+  }
+  int ax = 0;
+  for (int c = 1; c < 3; ++c)
+    if (mx[c] - mn[c] > mx[ax] - mn[ax]) ax = c;
+  const int a1 = (ax + 1) % 3, a2 = (ax + 2) % 3;
+  auto less = [&](int32_t p, int32_t q) {
+    const double *x = X + 3 * (int64_t)p, *y = X + 3 * (int64_t)q;
+    if (x[ax] != y[ax]) return x[ax] < y[ax];
+    if (x[a1] != y[a1]) return x[a1] < y[a1];
+    if (x[a2] != y[a2]) return x[a2] < y[a2];
+    return p < q;
+  };
+  const int gm = g0 + (g1 - g0) / 2;
+  // weighted selection of the cut; each side keeps at least one vertex per part
+  const double want = total * (gm - g0) / (g1 - g0);
+  int64_t a = lo + (gm - g0), b = hi - (g1 - gm);
+  int64_t l = lo, h = hi;
+  double acc = 0.0;
+  while (h - l > 1) {
+    const int64_t mid = (l + h) / 2;
+    std::nth_element(idx.begin() + l, idx.begin() + mid, idx.begin() + h, less);
+    double s = 0.0;
+    for (int64_t i = l; i < mid; ++i) s += w[idx[i]];
+    if (acc + s >= want) h = mid;
+    else acc += s, l = mid;
+  }
+  const int64_t cut = std::min(std::max(h, a), b);
+  std::nth_element(idx.begin() + lo, idx.begin() + cut, idx.begin() + hi, less);
+  bisect(X, w, idx, lo, cut, g0, gm, ptr);
+  bisect(X, w, idx, cut, hi, gm, g1, ptr);
+}
+
+int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
+                  int* n_parts, int32_t* part_ptr) {
+  SK_REQUIRE(X && T && order && n_parts && part_ptr, "sk_part_order: null argument");
+  SK_REQUIRE(precision == SK_PREC_FP64 || precision == SK_PREC_MIXED, "sk_part_order: bad precision");
+  SK_REQUIRE(nv > 0 && nt > 0, "sk_part_order: empty mesh");
+  for (int64_t k = 0; k < 4 * nt; ++k) SK_REQUIRE(T[k] >= 0 && T[k] < nv, "sk_part_order: tet index out of range");
+  *n_parts = 0;
+  std::vector<int32_t> deg;
+  vertex_degrees(T, nv, nt, deg);
+  int64_t nblk = 0;
+  for (int32_t d : deg) nblk += d;
+  const int G = resident_parts(nv, nblk, precision == SK_PREC_MIXED);
+  if (G == 0) {
+    degree_order(deg, order);
+    return SK_OK;
+  }
+  std::vector<float> w(nv);
+  const float mean = (float)nblk / (float)nv;
+  for (int64_t v = 0; v < nv; ++v) w[v] = (float)deg[v] + mean;
+  std::vector<int32_t> idx(nv);
+  std::iota(idx.begin(), idx.end(), 0);
+  bisect(X, w, idx, 0, nv, 0, G, part_ptr);
+  part_ptr[G] = (int32_t)nv;
+  for (int g = 0; g < G; ++g)
+    std::sort(idx.begin() + part_ptr[g], idx.begin() + part_ptr[g + 1], [&](int32_t p, int32_t q) {
+      return deg[p] != deg[q] ? deg[p] > deg[q] : p < q;
+    });
+  std::copy(idx.begin(), idx.end(), order);
+  *n_parts = G;
+  return SK_OK;
+}
+
+}  // extern "C"

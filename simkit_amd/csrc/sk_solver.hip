@@ -15,6 +15,7 @@
 // read, so every launch returns at once after convergence and the host reads
 // the struct once per chunk of enqueued iterations.
 #include "sk_coarse.h"
+#include "sk_resident.h"
 
 #include <cmath>
 
@@ -1606,12 +1607,19 @@ struct sk_sim {
   hipEvent_t ev[6] = {};
   bool have_events = false;
   sk::CoarseSpace coarse;  // two-level preconditioner (coarse.n_agg > 0 when enabled)
+  sk::ResidentState res;   // single-launch PCG on chip (sk_resident.h)
   bool mixed() const { return prm.precision == SK_PREC_MIXED; }
   bool two_level() const { return coarse.n_agg > 0; }
   // The mixed path keeps the classic form: its FP64 residual replacement breaks the pipelined
   // recurrences' identity p.Ap = delta - beta gamma / alpha_prev in FP32 (the replaced residual is
   // no longer r_prev - alpha s_prev to the recurrences' accuracy; a numpy emulation of the FP32 run
   // breaks down at the second replacement).
+  // The resident PCG serves the classic block-Jacobi form with the library's own launch shape; a caller
+  // that sets the launch widths or the chunk length asks for the launches.
+  bool may_be_resident() const {
+    return !res.off && (prm.pcg_variant == 0 || mixed()) && !two_level() && prm.spmv_blocks == 0 && prm.update_blocks == 0 &&
+           prm.pcg_chunk == 0;
+  }
   bool pipelined() const { return prm.pcg_variant == 1 && !two_level() && !mixed(); }
 };
 
@@ -2036,6 +2044,17 @@ int sk_sim_set_order(sk_sim* S, const int32_t* order_host) {
   return S->order.upload(h);
 }
 
+int sk_sim_set_parts(sk_sim* S, int n, const int32_t* ptr) {
+  SK_REQUIRE(S && (n == 0 || ptr), "sk_sim_set_parts: null argument");
+  SK_REQUIRE(n >= 0 && n <= kResMaxParts, "sk_sim_set_parts: 0..256 parts");
+  for (int g = 0; g < n; ++g) SK_REQUIRE(ptr[g] < ptr[g + 1], "sk_sim_set_parts: parts must be non-empty ranges");
+  SK_REQUIRE(n == 0 || (ptr[0] == 0 && ptr[n] == S->mesh->nv), "sk_sim_set_parts: parts must cover the vertices");
+  S->res.parts.assign(ptr, ptr + (n ? n + 1 : 0));
+  S->res.plan.reset();
+  S->res.tried = false;
+  return SK_OK;
+}
+
 int sk_sim_coarse_info(const sk_sim* S, int* n_agg, int* nc, int* built, double* build_ms) {
   SK_REQUIRE(S, "sk_sim_coarse_info: null simulator");
   if (n_agg) *n_agg = S->coarse.n_agg;
@@ -2133,10 +2152,28 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
       else SK_TRY(form_precond_matrix<double>(S, S->vals.p, S->binv.p, S->vhat.p, st));
     }
     if (P.timing) SK_HIP_CHECK(hipEventRecord(S->ev[1], st));
-    // Newton direction: H dx = -g on the free DOFs. The RHS is negated in place.
-    axpy_kernel<<<grid_for(n3), kBlock, 0, st>>>(n3, -2.0, S->g.p, S->g.p);
+    // Newton direction: H dx = -g on the free DOFs.
     int64_t it = 0;
     int done = 0, refines = 0;
+    bool resident = false;
+    ResidentPermit permit;
+    if (S->may_be_resident()) {
+      SK_TRY(resident_prepare(S->res, m, mixed));
+      if (S->res.plan && permit.acquire(S->res.plan->G, st)) {
+        ResidentSolve rs{S->vals.p, S->binv.p, fixed, S->g.p, S->dx.p, P.pcg_rtol, P.inner_rtol, P.pcg_max_iter,
+                         P.max_refine, mixed};
+        if (mixed) {
+          rs.vals = S->vals32.p;
+          rs.binv = S->binv32.p;
+        }
+        SK_TRY(resident_launch(S->res, m, rs, st));
+        resident = true;
+      }
+    }
+  launches:
+    if (!resident) {
+    // The RHS is negated in place.
+    axpy_kernel<<<grid_for(n3), kBlock, 0, st>>>(n3, -2.0, S->g.p, S->g.p);
     // The FP64 solve is not waited for: the slope's launches follow it in the
     // stream and its result is read after the slope's readback.
     if (mixed) SK_TRY(run_mixed_solve(S, st, &it, &refines, &done));
@@ -2145,11 +2182,25 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
                                   nullptr, nullptr));
     else SK_TRY(run_block_pcg<double>(S, bufs64(S), S->g.p, P.pcg_rtol, P.pcg_max_iter, st, nullptr, nullptr));
     axpy_kernel<<<grid_for(n3), kBlock, 0, st>>>(n3, -2.0, S->g.p, S->g.p);
+    }
     if (P.timing) SK_HIP_CHECK(hipEventRecord(S->ev[2], st));
     dot_kernel<<<grid_for(n3), kBlock, 0, st>>>(n3, S->g.p, S->dx.p, m->red.partials.p);
     finalize_sum_kernel<1><<<1, kBlock, 0, st>>>(m->red.partials.p, grid_for(n3), m->red.result.p);
     SK_TRY(read_scalars(m, m->red.result.p, 1, st));
-    if (!mixed) pcg_result(S, &it, &done);
+    if (resident) {
+      permit.release();
+      const volatile ResidentResult* h = S->res.host;
+      if (h->aborted) {  // the run gave up waiting for a workgroup: solve by launches, now and later
+        S->res.off = true;
+        resident = false;
+        goto launches;
+      }
+      it = h->iter;
+      done = h->done;
+      refines = h->refines;
+    } else if (!mixed) {
+      pcg_result(S, &it, &done);
+    }
     inf.pcg_iters += it;
     inf.refine_steps += refines;
     if (done == 2) inf.status = SK_ERR_PCG_BREAKDOWN;

@@ -85,18 +85,29 @@ class BackwardEulerSim:
         coarse_vertices = self.coarse_vertices
         # internal vertex order: order[t] = caller's vertex at internal position t
         self._order = self._pos = None
+        parts = None
         if renumber:
             order = np.empty(self.nv, np.int32)
             Tc = np.ascontiguousarray(T, dtype=np.int32)
-            _lib.call("sk_sell_order", Tc.ctypes.data_as(ctypes.c_void_p), int(self.nv), int(self.nt),
-                      order.ctypes.data_as(ctypes.c_void_p))
             if preconditioner == "two_level":
+                _lib.call("sk_sell_order", Tc.ctypes.data_as(ctypes.c_void_p), int(self.nv), int(self.nt),
+                          order.ctypes.data_as(ctypes.c_void_p))
                 # aggregate by aggregate, each aggregate's vertices in the sliced-ELL order (descending
                 # block count, ties by index), so that a SELL chunk's rows are mostly consecutive
                 rank = np.empty(self.nv, np.int64)
                 rank[order] = np.arange(self.nv)
                 key = np.repeat(np.arange(len(agg_ptr) - 1, dtype=np.int64), np.diff(agg_ptr)) * self.nv
                 order[:] = agg_order[np.argsort(key + rank[agg_order], kind="stable")]
+            else:
+                Xc = np.ascontiguousarray(X, dtype=np.float64)
+                n_parts, ptr_ = ctypes.c_int(), np.empty(257, np.int32)
+                _lib.call("sk_part_order", Xc.ctypes.data_as(ctypes.c_void_p), Tc.ctypes.data_as(ctypes.c_void_p),
+                          int(self.nv), int(self.nt),
+                          {"fp64": _lib.SK_PREC_FP64, "mixed": _lib.SK_PREC_MIXED}[precision],
+                          order.ctypes.data_as(ctypes.c_void_p), ctypes.byref(n_parts),
+                          ptr_.ctypes.data_as(ctypes.c_void_p))
+                if n_parts.value:
+                    parts = ptr_[:n_parts.value + 1]
             if not np.array_equal(order, np.arange(self.nv)):
                 pos = np.empty_like(order)
                 pos[order] = np.arange(self.nv, dtype=np.int32)
@@ -164,6 +175,8 @@ class BackwardEulerSim:
             # states cross the boundary in the caller's numbering; the library permutes them
             oc = np.ascontiguousarray(self._order, dtype=np.int32)
             _lib.call("sk_sim_set_order", self._h, oc.ctypes.data_as(ctypes.c_void_p))
+        if parts is not None:
+            _lib.call("sk_sim_set_parts", self._h, len(parts) - 1, parts.ctypes.data_as(ctypes.c_void_p))
         self.X_dev = dev(X.reshape(-1))
         self.preconditioner = preconditioner
         if preconditioner == "two_level":
