@@ -15,8 +15,8 @@ constexpr int kResMaxParts = 256;     // workgroups at most (the CUs of an MI355
 constexpr int kResLds = 160 * 1024;   // LDS a workgroup may use
 constexpr int kResStaticLds = 2048;   // bound on the kernel's static LDS
 // Threads per workgroup and blocks per thread held in registers, by precision.
-constexpr int kResNT64 = 512, kResKR64 = 8;
-constexpr int kResNT32 = 512, kResKR32 = 14;
+constexpr int kResNT64 = 512, kResKR64 = 8, kResShort64 = 5;
+constexpr int kResNT32 = 512, kResKR32 = 12, kResShort32 = 6;
 constexpr int kResMaxTier = 4;        // blocks per thread in LDS, and streamed from L2, at most (each)
 
 // Cut of a mesh's rows into contiguous ranges, one per workgroup, with the
@@ -24,11 +24,12 @@ constexpr int kResMaxTier = 4;        // blocks per thread in LDS, and streamed 
 struct ResidentPlan {
   std::vector<int32_t> parts;      // [G + 1] the cut (the cache key, with fp32)
   bool fp32 = false;
-  int G = 0, K = 0, KL = 0, KS = 0;  // blocks per thread: K = registers (up to KR) + LDS (KL) + streamed (KS)
+  int G = 0, K = 0, KR = 0, KL = 0, KS = 0;  // blocks per thread: K = registers (up to KR) + LDS (KL) + streamed (KS)
   int max_rows = 0, max_local = 0, max_halo = 0, n_exp = 0;
   size_t lds = 0;                  // dynamic LDS bytes
   DevBuf<int32_t> row0;            // [G + 1]
-  DevBuf<uint16_t> lcol;           // [nblk] (local column << 1) | last block of its row
+  DevBuf<uint16_t> lcol;           // [nblk] LDS byte offset of the block's column
+  DevBuf<uint32_t> tflag;          // [G NT] which of a thread's blocks end a row
   DevBuf<uint16_t> trow;           // [G NT] local row of each thread's first block (rows: none)
   // The halo of a part: the vertices of other parts that its rows couple to (hvert, ascending; halo_ptr[G + 1]),
   // and their places among all exported vertices (ResidentArgs::halo, exp0, exslot).

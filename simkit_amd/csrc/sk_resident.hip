@@ -57,7 +57,8 @@ struct ResidentArgs {
   int G, K, KL, KS;
   const int32_t* row0;
   const int32_t* bptr;
-  const uint16_t* lcol;
+  const uint16_t* lcol;       // [nblk] LDS byte offset of the block's column in a T vector
+  const uint32_t* tflag;      // [G NT] bit k: the thread's k-th block is the last of its row
   const uint16_t* trow;
   const int32_t* sell_pos;
   const T* vals;
@@ -257,15 +258,22 @@ struct Meet {
       }
     }
   }
-  // Totals over all workgroups (after the barrier that follows collect).
+  // Totals over all workgroups (after the barrier that follows collect): lane
+  // 8 k + w takes wave w's sum of value k.
   template <int NV>
   __device__ __forceinline__ void totals(double (&v)[NV]) const {
+    static_assert(nw == 8, "eight waves");
+    const int lane = threadIdx.x % kWave;
+    double s = tot[lane < NV * nw ? lane : 0];
+    s = dpp_add<0xB1, 0xf>(s);   // quad_perm [1, 0, 3, 2]
+    s = dpp_add<0x4E, 0xf>(s);   // quad_perm [2, 3, 0, 1]
+    s = dpp_add<0x141, 0xf>(s);  // row_half_mirror: the other half of the eight lanes
 #pragma unroll
     for (int k = 0; k < NV; ++k) {
-      double s = 0.0;
-#pragma unroll
-      for (int w = 0; w < nw; ++w) s += tot[k * nw + w];
-      v[k] = s;
+      const uint64_t u = (uint64_t)__double_as_longlong(s);
+      const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, k * nw);
+      const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), k * nw);
+      v[k] = __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
     }
   }
 };
@@ -301,10 +309,13 @@ struct Meet {
 // Why: the two-launch form reads 107 MB (FP64) of values per iteration and
 // pays two launch boundaries; 256 CUs hold 128 MB in registers and 40 MB in
 // LDS, so nothing but the halo has to move. Measured per iteration over a
-// whole step, launches then this kernel: 48^3 FP64 30.8 -> 11.3 us, mixed 20.9
-// -> 8.4; 32^3 mixed 12.6 -> 6.4; 10^3 FP64 11.9 -> 6.0 us. What bounds it is
-// the meeting (about 3.5 us at 256 workgroups, 1.5 us at 8) and the latency of
-// the phases between barriers.
+// whole step, launches then this kernel: 48^3 FP64 30.8 -> 10.7 us, mixed 20.9
+// -> 8.2; 32^3 mixed 12.6 -> 5.6; 10^3 FP64 11.9 -> 5.4 us. What bounds it is
+// the meeting (about 2.2 us at 256 workgroups, 1.5 us at 8) and the latency of
+// the phases between barriers; in FP64 at 48^3 also the product (2.9 us, two of
+// a thread's twelve blocks streamed from L2). Exchanging B^-1 A p instead of
+// A p, so that the halo needs neither r nor B^-1, was slower: the owner's x and
+// r then leave LDS (FP64 10.7 -> 12.7 us, mixed equal).
 template <typename T, int NT, int KR, bool kMixed>
 __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs<T> a) {
   extern __shared__ double dyn[];
@@ -320,19 +331,19 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   const int h0 = a.halo_ptr[me], H = a.halo_ptr[me + 1] - h0;
   const int x0 = a.exp0[me], E = a.exp0[me + 1] - x0;
   const int K = a.K;
-  PV* part = reinterpret_cast<PV*>(dyn);                              // [max_rows + NT + 1][3]
-  double* P64 = reinterpret_cast<double*>(part + 3 * (a.max_rows + NT + 1));  // [max_local][3] (kMixed)
-  T* P = reinterpret_cast<T*>(P64 + (kMixed ? 3 * a.max_local : 0));  // [max_local][3]
+  T* P = reinterpret_cast<T*>(dyn);                                   // [max_local][3], at a constant address
   T* RL = P + 3 * a.max_local;                                        // [max_local][3] r
   T* HA = RL + 3 * a.max_local;                                       // [max_halo][3] what the halo's owners sent
   T* XL = HA + 3 * a.max_halo;                                        // [max_rows][3] x (kMixed; else in a.x)
-  T* L = XL + (kMixed ? 3 * a.max_rows : 0);                          // [KL][9][NT]
+  PV* part = reinterpret_cast<PV*>(XL + (kMixed ? 3 * a.max_rows + (a.max_halo + a.max_rows) % 2 : 0));
+  double* P64 = reinterpret_cast<double*>(part + 3 * (a.max_rows + NT + 1));  // [max_local][3] (kMixed)
+  T* L = reinterpret_cast<T*>(P64 + (kMixed ? 3 * a.max_local : 0));  // [KL][9][NT]
   int32_t* HX = reinterpret_cast<int32_t*>(L + (size_t)9 * NT * a.KL);  // [max_halo] places of the halo vertices
   uint16_t* EX = reinterpret_cast<uint16_t*>(HX + a.max_halo);        // [NT] partial slots of the exported rows
   T* S = a.stream + (size_t)me * a.KS * 9 * NT;
   if (t == 0) s_bad = 0;
 
-  // the thread's blocks and their words (local column << 1 | last of its row)
+  // the thread's blocks, their columns' byte offsets and which of them end a row
   T A[KR][9];
   uint32_t meta[(KR + 2 * kResMaxTier + 1) / 2];
 #pragma unroll
@@ -368,6 +379,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
 #pragma unroll
       for (int m = 0; m < 9; ++m) S[(k * 9 + m) * NT + t] = B[m];
     }
+  const uint32_t flags = a.tflag[me * NT + t];
   const int slot0 = (int)a.trow[me * NT + t] + t;
 
   // y = A src for the workgroup's rows, as partials. The source entries of the
@@ -381,17 +393,18 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     const int tt = opaque(t);
     V y0 = 0, y1 = 0, y2 = 0;
     PV* o = part + 3 * slot0;
-    auto read = [&](uint32_t lm, V (&p)[3]) {
-      const V* q = src + 3 * (lm >> 1);
+    const uint32_t fl = (uint32_t)opaque((int)flags);
+    auto read = [&](uint32_t off, V (&p)[3]) {  // offsets are those of T vectors
+      const V* q = reinterpret_cast<const V*>(reinterpret_cast<const char*>(src) + off * (sizeof(V) / sizeof(T)));
       p[0] = q[0];
       p[1] = q[1];
       p[2] = q[2];
     };
-    auto add = [&](const T (&B)[9], const V (&p)[3], uint32_t lm) {
+    auto add = [&](const T (&B)[9], const V (&p)[3], uint32_t last) {
       y0 = fma((V)B[2], p[2], fma((V)B[1], p[1], fma((V)B[0], p[0], y0)));
       y1 = fma((V)B[5], p[2], fma((V)B[4], p[1], fma((V)B[3], p[0], y1)));
       y2 = fma((V)B[8], p[2], fma((V)B[7], p[1], fma((V)B[6], p[0], y2)));
-      if (lm & 1) {
+      if (last) {
         o[0] = (PV)y0;
         o[1] = (PV)y1;
         o[2] = (PV)y2;
@@ -416,7 +429,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
           if (k + U + u < KR) read(word(k + U + u), p[(k / U + 1) & 1][u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-          if (k + u < KR) add(A[k + u], p[(k / U) & 1][u], word(k + u));
+          if (k + u < KR) add(A[k + u], p[(k / U) & 1][u], fl & (1u << (k + u)));
       }
     }
 #pragma unroll
@@ -427,12 +440,12 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         read(word(KR + k), q);
 #pragma unroll
         for (int m = 0; m < 9; ++m) B[m] = L[(k * 9 + m) * NT + tt];
-        add(B, q, word(KR + k));
+        add(B, q, fl & (1u << (KR + k)));
       }
     if (a.KS > 0) {
       V q[3];
       read(word(KR + kResMaxTier), q);
-      add(B0, q, word(KR + kResMaxTier));
+      add(B0, q, fl & (1u << (KR + kResMaxTier)));
     }
 #pragma unroll
     for (int k = 1; k < kResMaxTier; ++k)
@@ -442,7 +455,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         read(word(KR + kResMaxTier + k), q);
 #pragma unroll
         for (int m = 0; m < 9; ++m) B[m] = S[(k * 9 + m) * NT + tt];
-        add(B, q, word(KR + kResMaxTier + k));
+        add(B, q, fl & (1u << (KR + kResMaxTier + k)));
       }
     o[0] = (PV)y0;  // the open row's partial (or a slot that no row reads)
     o[1] = (PV)y1;
@@ -505,14 +518,22 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   auto put_exports = [&](auto tag, uint64_t* words, uint32_t epoch) {
     using V = decltype(tag);
     constexpr int VS = kVertStride<V>, VW = kVertWords<V>;
-    for (int j = t; j < E * VS; j += NT) {
-      const int w = j % VS;
-      if (w >= VW) continue;
-      const PV* src = part + 3 * EX[j / VS];
-      uint32_t u;
-      if constexpr (sizeof(V) == 8) u = reinterpret_cast<const uint32_t*>(src)[w];
-      else u = __float_as_uint((float)src[w]);
-      put_word(words + (size_t)x0 * VS + j, epoch, u);
+    constexpr int U = sizeof(V) == 8 ? 2 : 4;
+    for (int j0 = t; j0 < E * VS; j0 += U * NT) {  // U words' LDS reads under way together
+      const int w = j0 % VS < VW ? j0 % VS : 0;
+      uint32_t u[U];
+      int e[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) e[k] = EX[j0 + k * NT < E * VS ? (j0 + k * NT) / VS : 0];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const PV* src = part + 3 * e[k];
+        if constexpr (sizeof(V) == 8) u[k] = reinterpret_cast<const uint32_t*>(src)[w];
+        else u[k] = __float_as_uint((float)src[w]);
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k)
+        if (j0 % VS < VW && j0 + k * NT < E * VS) put_word(words + (size_t)x0 * VS + j0 + k * NT, epoch, u[k]);
     }
   };
   for (int j = t; j < H; j += NT) HX[j] = a.halo[h0 + j];
@@ -574,20 +595,21 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     double va[4] = {0.0, 0.0, 0.0, 0.0};
     ++epoch;
     if (row) {
+      const int l = opaque(t);
       PV y[3];
       row_sum(y);
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
         ap[q] = (T)y[q];
         part[3 * s0 + q] = (PV)ap[q];  // staged for put_exports in the row's own slot
-        r[q] = RL[3 * t + q];
+        r[q] = RL[3 * l + q];
       }
       T z[3], u[3];
       precondition(B, r, z);
       precondition(B, ap, u);
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        va[0] += (double)P[3 * t + q] * (double)ap[q];
+        va[0] += (double)P[3 * l + q] * (double)ap[q];
         va[1] += (double)u[q] * (double)ap[q];
         va[2] += (double)r[q] * (double)z[q];
         va[3] += (double)r[q] * (double)r[q];
@@ -709,18 +731,19 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     const double al = (double)alpha, rz_next = al * al * va[1] - rz;
     const T beta = (T)(rz_next > 0.0 ? rz_next * inv_rz : 0.0);
     ++iter;
+    const int l = opaque(t);
     if (row) {
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        if (kMixed) XL[3 * t + q] = fma(alpha, P[3 * t + q], XL[3 * t + q]);
-        else a.x[3 * (int64_t)v + q] = fma((double)alpha, (double)P[3 * t + q], xg[q]);
-        r[q] = fma(-alpha, ap[q], RL[3 * t + q]);
-        RL[3 * t + q] = r[q];
+        if (kMixed) XL[3 * l + q] = fma(alpha, P[3 * l + q], XL[3 * l + q]);
+        else a.x[3 * (int64_t)(v0 + l) + q] = fma((double)alpha, (double)P[3 * l + q], xg[q]);
+        r[q] = fma(-alpha, ap[q], RL[3 * l + q]);
+        RL[3 * l + q] = r[q];
       }
-      direction(t, B, r, beta);
+      direction(l, B, r, beta);
     }
-    for (int j = t; j < H; j += NT) {
-      if (j != t) load_binv(a.hvert[h0 + j], BH);
+    for (int j = l; j < H; j += NT) {
+      if (j != l) load_binv(a.hvert[h0 + j], BH);
       T rh[3];
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
@@ -828,21 +851,32 @@ void ResidentPermit::release() {
 }
 
 int resident_parts(int64_t nv, int64_t nblk, bool fp32) {
-  const int NT = fp32 ? kResNT32 : kResNT64, KR = fp32 ? kResKR32 : kResKR64;
+  const int NT = fp32 ? kResNT32 : kResNT64;
   // at least enough workgroups that a row has a thread (with 10% for an uneven cut)
   const int64_t need = (11 * nv + 10 * NT - 1) / (10 * (int64_t)NT);
   int64_t G = nv <= NT ? 1 : need;
-  // and few blocks per thread
-  const int64_t target = (int64_t)NT * (KR < 8 ? KR : 8) / 2;
+  // and about one block per thread: the product's latency costs more than the meeting of more workgroups
+  // (per iteration, at 4 / 2 / 1 blocks per thread: 10^3 FP64 5.8 / 5.7 / 5.4 us, a 29 x 13 x 21 box 7.5 /
+  // 7.1 / 6.9, 32^3 mixed 5.9 / 5.6 / 5.6)
+  const int64_t target = NT;
   G = std::max(G, (nblk + target - 1) / target);
+  if (G > 8) G = (G + 7) / 8 * 8;  // the same number of workgroups on every XCD
   if (G > kResMaxParts) G = kResMaxParts;
   if (nv > (int64_t)G * NT) return 0;
   return (int)std::max<int64_t>(G, 1);
 }
 
+// Blocks per thread in registers: the short variant where all of a thread's
+// blocks fit it (no register spilled: 10^3 FP64 5.8 us an iteration against
+// 6.5 us with the long one), else the long one.
+static int resident_kr(bool fp32, int K) {
+  if (fp32) return K <= kResShort32 ? kResShort32 : kResKR32;
+  return K <= kResShort64 ? kResShort64 : kResKR64;
+}
+
 static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<int32_t>& parts, bool fp32, int* status) {
   *status = SK_OK;
-  const int NT = fp32 ? kResNT32 : kResNT64, KR = fp32 ? kResKR32 : kResKR64;
+  const int NT = fp32 ? kResNT32 : kResNT64;
   const int G = (int)parts.size() - 1;
   const int32_t *bptr = m->h_bptr.data(), *bcol = m->h_bcol.data();
   auto p = std::make_shared<ResidentPlan>();
@@ -856,12 +890,16 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   }
   if (p->max_rows > NT) return nullptr;
   p->K = std::max(1, (max_nb + NT - 1) / NT);
+  p->KR = resident_kr(fp32, p->K);
+  const int KR = p->KR;
   std::vector<int32_t> loc(m->nv, -1), halo_ptr(1, 0), halo;
   std::vector<int16_t> place(m->nv, -1);
   std::vector<int32_t> owner(m->nv), exp0(1, 0);
   for (int g = 0; g < G; ++g)
     for (int32_t r = parts[g]; r < parts[g + 1]; ++r) owner[r] = g;
   std::vector<uint16_t> lcol(m->nblk), trow((size_t)G * NT);
+  std::vector<int32_t> tlast;
+  tlast.reserve(m->nv);
   std::vector<int32_t> mine;
   for (int g = 0; g < G; ++g) {
     const int32_t r0 = parts[g], r1 = parts[g + 1];
@@ -877,7 +915,7 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
     const int rows = r1 - r0, local = rows + (int)mine.size();
     p->max_local = std::max(p->max_local, local);
     p->max_halo = std::max(p->max_halo, (int)mine.size());
-    if (local > 32767) return nullptr;
+    if (local * (fp32 ? 12 : 24) > 65535) return nullptr;
     for (size_t i = 0; i < mine.size(); ++i) {
       loc[mine[i]] = rows + (int)i;
       place[mine[i]] = 0;
@@ -887,8 +925,9 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
       for (int32_t b = bptr[r]; b < bptr[r + 1]; ++b) {
         const int32_t w = bcol[b];
         const int c = w >= r0 && w < r1 ? w - r0 : loc[w];
-        lcol[b] = (uint16_t)((c << 1) | (b + 1 == bptr[r + 1] ? 1 : 0));
+        lcol[b] = (uint16_t)(c * (fp32 ? 12 : 24));
       }
+      tlast.push_back(bptr[r + 1] - 1 - bptr[r0]);  // the row's last block in the workgroup's list
       for (; tk < NT && tk * p->K < bptr[r + 1] - bptr[r0]; ++tk) trow[(size_t)g * NT + tk] = (uint16_t)(r - r0);
     }
     for (; tk < NT; ++tk) trow[(size_t)g * NT + tk] = (uint16_t)rows;
@@ -918,6 +957,14 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   p->KL = (int)std::min<size_t>(std::min(rest, kResMaxTier), (kResLds - base) / tier_lds(fp32));
   p->KS = rest - p->KL;
   if (p->KS > kResMaxTier) return nullptr;
+  // the threads' row-end bits: registers, the LDS tier (kResMaxTier bits), the streamed tier
+  static_assert(kResKR32 + 2 * kResMaxTier <= 32 && kResKR64 + 2 * kResMaxTier <= 32, "one bit per block");
+  std::vector<uint32_t> tflag((size_t)G * NT, 0);
+  for (int g = 0; g < G; ++g)
+    for (int32_t r = parts[g]; r < parts[g + 1]; ++r) {
+      const int th = tlast[r] / p->K, k = tlast[r] % p->K;
+      tflag[(size_t)g * NT + th] |= 1u << (k < KR + p->KL ? k : KR + kResMaxTier + (k - KR - p->KL));
+    }
   p->lds = base - kResStaticLds + p->KL * tier_lds(fp32);
   // more than half of a CU's LDS: one workgroup per CU, so the runs spread over the chip
   p->lds = std::max<size_t>(p->lds, kResLds / 2 + 1024);
@@ -925,6 +972,7 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   auto up = [&]() -> int {
     SK_TRY(p->row0.upload(row0));
     SK_TRY(p->lcol.upload(lcol));
+    SK_TRY(p->tflag.upload(tflag));
     SK_TRY(p->trow.upload(trow));
     SK_TRY(p->halo_ptr.upload(halo_ptr));
     SK_TRY(p->halo.upload(where));
@@ -984,7 +1032,7 @@ int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32) {
 template <typename T, int NT, int KR, bool kMixed>
 static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st) {
   const ResidentPlan& p = *R.plan;
-  ResidentArgs<T> a{p.G, p.K, p.KL, p.KS, p.row0.p, m->bptr.p, p.lcol.p, p.trow.p, m->sell_pos.p, (const T*)s.vals,
+  ResidentArgs<T> a{p.G, p.K, p.KL, p.KS, p.row0.p, m->bptr.p, p.lcol.p, p.tflag.p, p.trow.p, m->sell_pos.p, (const T*)s.vals,
                     (const T*)s.binv, s.fixed, s.g, s.dx, p.halo_ptr.p, p.hvert.p, p.halo.p, p.exp0.p, p.exslot.p, R.slots.p, R.zx.p,
                     R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
                     p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
@@ -1002,8 +1050,11 @@ int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStr
     R.epoch = 0;
   }
   *R.host = ResidentResult{0, 0, 0, 0, R.epoch};
-  return s.fp32 ? launch<float, kResNT32, kResKR32, true>(R, m, s, st)
-                : launch<double, kResNT64, kResKR64, false>(R, m, s, st);
+  if (s.fp32)
+    return R.plan->KR == kResShort32 ? launch<float, kResNT32, kResShort32, true>(R, m, s, st)
+                                     : launch<float, kResNT32, kResKR32, true>(R, m, s, st);
+  return R.plan->KR == kResShort64 ? launch<double, kResNT64, kResShort64, false>(R, m, s, st)
+                                   : launch<double, kResNT64, kResKR64, false>(R, m, s, st);
 }
 
 
