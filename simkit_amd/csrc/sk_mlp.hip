@@ -17,19 +17,21 @@
 //                      refreshed after every update.
 // Rounding to BF16 is round-to-nearest-even.
 //
-// Every GEMM runs 64 x 64 output tiles per workgroup (4 waves, 32 x 32 each:
-// 2 x 2 tiles of v_mfma_f32_16x16x32_bf16), stepping K by 32: the workgroup
-// stages the A and B tiles in LDS with 16-byte loads along whichever operand
-// dimension is contiguous in memory (so transposed operands cost the same),
-// storing both k-contiguous; lane l then reads its fragments with one 16-byte
-// LDS load each: A[l % 16][8 (l / 16) + 0..7] and B[8 (l / 16) + 0..7][l % 16],
-// and receives D[4 (l / 16) + 0..3][l % 16]. Feature and batch dimensions are
-// padded to multiples of 16 with zeros; a K tail of 16 is zero-filled in LDS.
+// Every GEMM runs 32 x 32 or 64 x 64 output tiles per workgroup (4 waves, a
+// quarter each, in 16 x 16 tiles of v_mfma_f32_16x16x32_bf16), stepping K by 64:
+// the workgroup stages the A and B tiles in LDS with 16-byte loads along
+// whichever operand dimension is contiguous in memory (so transposed operands
+// cost the same), storing both k-contiguous; lane l then reads its fragments
+// with one 16-byte LDS load each: A[l % 16][8 (l / 16) + 0..7] and
+// B[8 (l / 16) + 0..7][l % 16], and receives D[4 (l / 16) + 0..3][l % 16].
+// Feature and batch dimensions are padded to multiples of 16 with zeros; a K
+// tail is zero-filled in LDS.
 #include "sk_internal.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <vector>
 
 typedef float sk_v4f __attribute__((ext_vector_type(4)));
@@ -72,88 +74,130 @@ struct GemmArgs {
   uint16_t* Cbf;                    // bf16(act(C)), row stride ldcb (may be null)
   int64_t ldcb;
   int gelu_act;                     // 1: Cbf holds GELU(C)
+  const float* Zgrad;               // non-null: C and Cbf hold acc * GELU'(Zgrad(m, n)), row stride ldc
 };
-
-constexpr int kGT = 64;           // workgroup output tile, M and N
-constexpr int kGK = 32;           // K step (one 16x16x32 MFMA)
-constexpr int kGP = kGK + 8;      // LDS row pitch in BF16 (80 bytes: 16-byte aligned, rows on different banks)
 
 typedef __bf16 sk_bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t sk_u4 __attribute__((ext_vector_type(4)));
 
-// S[r][c] = P[(r0 + r) srow + (k0 + c) sk] for r < 64, c < 32 (zero outside
-// R x K). 256 threads, 8 elements each: 16-byte loads along k (sk == 1) or
-// along r (srow == 1) when the addresses allow, else element by element.
-// K is a multiple of 16, so an aligned run of 8 along k is all inside or all
-// outside.
-__device__ __forceinline__ void stage_tile(const uint16_t* __restrict__ P, int64_t srow, int64_t sk, int r0, int R,
-                                           int k0, int K, bool vec_k, bool vec_r, uint16_t (*S)[kGP]) {
-  const int t = threadIdx.x;
-  if (vec_k) {
-    const int r = t / 4, c = (t % 4) * 8;
-    sk_u4 v = {0u, 0u, 0u, 0u};
-    if (r0 + r < R && k0 + c < K) v = *reinterpret_cast<const sk_u4*>(P + (int64_t)(r0 + r) * srow + (k0 + c));
-    *reinterpret_cast<sk_u4*>(&S[r][c]) = v;
-  } else if (vec_r) {
-    const int c = t / 8, r = (t % 8) * 8;
-    sk_u4 v = {0u, 0u, 0u, 0u};
-    if (r0 + r < R && k0 + c < K) v = *reinterpret_cast<const sk_u4*>(P + (int64_t)(k0 + c) * sk + (r0 + r));
-    const uint16_t* h = reinterpret_cast<const uint16_t*>(&v);
+// A tile of TR rows x KS columns of P in registers, 16-byte runs of 8 along k
+// (sk == 1) or along r (srow == 1) when the addresses allow, else element by
+// element: thread t holds the NQ runs t, t + 256, ... P(r, c) =
+// P[(r0 + r) srow + (k0 + c) sk], zero outside R x K. K is a multiple of 16, so
+// an aligned run of 8 along k is all inside or all outside.
+template <int TR, int KS>
+struct StagedTile {
+  static constexpr int NQ = TR * KS / 8 / kBlock;
+  static constexpr int kPitch = KS + 8;  // LDS row pitch (16-byte aligned, rows on different banks)
+  sk_u4 v[NQ];
+
+  __device__ __forceinline__ void load(const uint16_t* __restrict__ P, int64_t srow, int64_t sk, int r0, int R,
+                                       int k0, int K, bool vec_k, bool vec_r) {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) S[r + q][c] = h[q];
-  } else {
+    for (int q = 0; q < NQ; ++q) {
+      const int e = threadIdx.x + q * kBlock;
+      v[q] = sk_u4{0u, 0u, 0u, 0u};
+      if (vec_r) {
+        const int c = e / (TR / 8), r = (e % (TR / 8)) * 8;
+        if (r0 + r < R && k0 + c < K) v[q] = *reinterpret_cast<const sk_u4*>(P + (int64_t)(k0 + c) * sk + (r0 + r));
+      } else {
+        const int r = e / (KS / 8), c = (e % (KS / 8)) * 8;
+        if (r0 + r >= R || k0 + c >= K) continue;
+        const uint16_t* src = P + (int64_t)(r0 + r) * srow + (int64_t)(k0 + c) * sk;
+        if (vec_k) {
+          v[q] = *reinterpret_cast<const sk_u4*>(src);
+        } else {
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int e = t * 8 + q, r = e / kGK, c = e % kGK;
-      S[r][c] = (r0 + r < R && k0 + c < K) ? P[(int64_t)(r0 + r) * srow + (int64_t)(k0 + c) * sk] : (uint16_t)0;
+          for (int h = 0; h < 4; ++h)
+            v[q][h] = (uint32_t)src[(2 * h) * sk] | (uint32_t)src[(2 * h + 1) * sk] << 16;
+        }
+      }
     }
   }
-}
+  __device__ __forceinline__ void store(uint16_t (*S)[kPitch], bool vec_r) const {
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+      const int e = threadIdx.x + q * kBlock;
+      if (vec_r) {
+        const int c = e / (TR / 8), r = (e % (TR / 8)) * 8;
+#pragma unroll
+        for (int h = 0; h < 8; ++h) S[r + h][c] = (uint16_t)(v[q][h / 2] >> (16 * (h & 1)));
+      } else {
+        const int r = e / (KS / 8), c = (e % (KS / 8)) * 8;
+        *reinterpret_cast<sk_u4*>(&S[r][c]) = v[q];
+      }
+    }
+  }
+};
 
+// Tile x Tile outputs per workgroup (4 waves, a quarter each), K in steps of 64
+// with the next step's tiles on their way from memory while this one is
+// multiplied. At the network's usual sizes (256 x 256 x 256) a product is the
+// latency of its K steps on a few workgroups, not bandwidth or matrix rate: 64 x
+// 64 tiles with 32-wide steps and no prefetch (16 workgroups, 8 steps) took 7.9
+// us back to back, 32 x 32 tiles this way 4.0 us. The accumulation order over k
+// is the same for every tile size.
+constexpr int kGK = 64;
+template <int Tile>
 __global__ __launch_bounds__(kBlock) void gemm_bf16_kernel(GemmArgs g) {
-  __shared__ __align__(16) uint16_t As[kGT][kGP];  // [m][k]
-  __shared__ __align__(16) uint16_t Bs[kGT][kGP];  // [n][k]
-  const int tiles_n = (g.N + kGT - 1) / kGT;
-  const int m0 = (blockIdx.x / tiles_n) * kGT, n0 = (blockIdx.x % tiles_n) * kGT;
+  using Staged = StagedTile<Tile, kGK>;
+  constexpr int NT = Tile / 32;  // 16 x 16 tiles per wave and direction
+  __shared__ __align__(16) uint16_t As[Tile][Staged::kPitch];  // [m][k]
+  __shared__ __align__(16) uint16_t Bs[Tile][Staged::kPitch];  // [n][k]
+  const int tiles_n = (g.N + Tile - 1) / Tile;
+  const int m0 = (blockIdx.x / tiles_n) * Tile, n0 = (blockIdx.x % tiles_n) * Tile;
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-  const int wm = (wid / 2) * 32, wn = (wid % 2) * 32;
+  const int wm = (wid / 2) * (Tile / 2), wn = (wid % 2) * (Tile / 2);
   const int i = lane % 16, kq = lane / 16;
   // 16-byte staging needs 8-element runs at 16-byte aligned addresses
   auto aligned = [](const uint16_t* p, int64_t s) { return ((uintptr_t)p % 16 == 0) && (s % 8 == 0); };
   const bool a_k = g.sak == 1 && aligned(g.A, g.sam), a_r = !a_k && g.sam == 1 && aligned(g.A, g.sak);
   const bool b_k = g.sbk == 1 && aligned(g.B, g.sbn), b_r = !b_k && g.sbn == 1 && aligned(g.B, g.sbk);
-  sk_v4f acc[2][2];
+  sk_v4f acc[NT][NT];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NT; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = sk_v4f{0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < NT; ++b) acc[a][b] = sk_v4f{0.f, 0.f, 0.f, 0.f};
+  Staged sa, sb;
+  sa.load(g.A, g.sam, g.sak, m0, g.M, 0, g.K, a_k, a_r);
+  sb.load(g.B, g.sbn, g.sbk, n0, g.N, 0, g.K, b_k, b_r);
   for (int k0 = 0; k0 < g.K; k0 += kGK) {
-    stage_tile(g.A, g.sam, g.sak, m0, g.M, k0, g.K, a_k, a_r, As);
-    stage_tile(g.B, g.sbn, g.sbk, n0, g.N, k0, g.K, b_k, b_r, Bs);
+    sa.store(As, a_r);
+    sb.store(Bs, b_r);
     __syncthreads();
-    sk_bf16x8 af[2], bfr[2];
+    if (k0 + kGK < g.K) {
+      sa.load(g.A, g.sam, g.sak, m0, g.M, k0 + kGK, g.K, a_k, a_r);
+      sb.load(g.B, g.sbn, g.sbk, n0, g.N, k0 + kGK, g.K, b_k, b_r);
+    }
 #pragma unroll
-    for (int a = 0; a < 2; ++a) af[a] = *reinterpret_cast<const sk_bf16x8*>(&As[wm + 16 * a + i][8 * kq]);
+    for (int kk = 0; kk < kGK; kk += 32) {
+      if (k0 + kk >= g.K) break;
+      sk_bf16x8 af[NT], bfr[NT];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) bfr[b] = *reinterpret_cast<const sk_bf16x8*>(&Bs[wn + 16 * b + i][8 * kq]);
+      for (int a = 0; a < NT; ++a) af[a] = *reinterpret_cast<const sk_bf16x8*>(&As[wm + 16 * a + i][kk + 8 * kq]);
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+      for (int b = 0; b < NT; ++b) bfr[b] = *reinterpret_cast<const sk_bf16x8*>(&Bs[wn + 16 * b + i][kk + 8 * kq]);
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+      for (int a = 0; a < NT; ++a)
+#pragma unroll
+        for (int b = 0; b < NT; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[a], bfr[b], acc[a][b], 0, 0, 0);
+    }
     __syncthreads();
   }
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
+  for (int b = 0; b < NT; ++b) {
     const int n = n0 + wn + 16 * b + i;
     if (n >= g.N) continue;
     const float bn = g.bias ? g.bias[n] : 0.f;
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < NT; ++a)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t m = m0 + wm + 16 * a + 4 * kq + r;
         if (m >= g.M) continue;
-        const float z = acc[a][b][r] + bn;
+        float z = acc[a][b][r] + bn;
+        if (g.Zgrad) z *= gelu_grad(g.Zgrad[m * g.ldc + n]);
         if (g.C) g.C[m * g.ldc + n] = z;
         if (g.Cbf) g.Cbf[m * g.ldcb + n] = f2bf(g.gelu_act ? gelu(z) : z);
       }
@@ -163,8 +207,13 @@ __global__ __launch_bounds__(kBlock) void gemm_bf16_kernel(GemmArgs g) {
 int launch_gemm(const GemmArgs& g, hipStream_t st) {
   SK_REQUIRE(g.M % kTile == 0 && g.N % kTile == 0 && g.K % kTile == 0 && g.M > 0 && g.N > 0 && g.K > 0,
              "bf16 GEMM: dimensions must be positive multiples of 16");
-  const int64_t blocks = (int64_t)((g.M + kGT - 1) / kGT) * ((g.N + kGT - 1) / kGT);
-  gemm_bf16_kernel<<<(unsigned)blocks, kBlock, 0, st>>>(g);
+  // 32 x 32 tiles until there are two 64 x 64 ones for each of the 256 CUs; both
+  // measured, 32 against 64: 256 large tiles 5.9 / 8.1 us (1024 x 1024, K = 256)
+  // and 12.6 / 17.6 us (K = 1024), 512 large tiles 14.4 / 12.6 us (4096 x 512, K
+  // = 512), 1024 large tiles 74.5 / 60.6 us (2048 cubed).
+  auto blocks = [&](int t) { return (int64_t)((g.M + t - 1) / t) * ((g.N + t - 1) / t); };
+  if (blocks(64) < 512) gemm_bf16_kernel<32><<<(unsigned)blocks(32), kBlock, 0, st>>>(g);
+  else gemm_bf16_kernel<64><<<(unsigned)blocks(64), kBlock, 0, st>>>(g);
   SK_HIP_CHECK(hipGetLastError());
   return SK_OK;
 }
@@ -228,22 +277,25 @@ __global__ __launch_bounds__(kBlock) void mse_grad_kernel(int rows, int cols, in
   store_block_partials<1>(v, partials);
 }
 
-// dZ = dA * GELU'(Z) and its BF16 copy.
-__global__ void gelu_backward_kernel(int64_t n, const float* dA, const float* Z, float* dZ, uint16_t* dZbf) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n) return;
-  const float d = dA[e] * gelu_grad(Z[e]);
-  dZ[e] = d;
-  dZbf[e] = f2bf(d);
-}
-
-// db[n] = sum_b dZ[b][n] in batch order.
-__global__ void colsum_kernel(int prow, int pcol, const float* dZ, float* db) {
-  const int n = blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= pcol) return;
+// db[n] = sum_b dZ[b][n]: 32 columns per workgroup, eight row lanes each, the
+// lanes' sums added in order. One thread per column walked the batch in 55 us at
+// 256 x 256, a chain of 256 dependent loads; this takes 3.2 us.
+constexpr int kColRows = kBlock / 32;
+__global__ __launch_bounds__(kBlock) void colsum_kernel(int prow, int pcol, const float* dZ, float* db) {
+  __shared__ float part[kColRows][32];
+  const int c = threadIdx.x % 32, r = threadIdx.x / 32, n = blockIdx.x * 32 + c;
   float s = 0.f;
-  for (int b = 0; b < prow; ++b) s += dZ[(int64_t)b * pcol + n];
-  db[n] = s;
+  if (n < pcol) {
+#pragma unroll 4
+    for (int b = r; b < prow; b += kColRows) s += dZ[(int64_t)b * pcol + n];
+  }
+  part[r][c] = s;
+  __syncthreads();
+  if (r == 0 && n < pcol) {
+#pragma unroll
+    for (int q = 1; q < kColRows; ++q) s += part[q][c];
+    db[n] = s;
+  }
 }
 
 __global__ void adam_kernel(int64_t n, float* w, const float* g, float* m, float* v, uint16_t* wbf, float lr,
@@ -281,9 +333,11 @@ struct sk_mlp {
   std::vector<DevBuf<uint16_t>> Wbf;
   std::vector<DevBuf<uint16_t>> Abf;  // layer inputs [pbatch][pdims[l]], l = 0..L-1
   std::vector<DevBuf<float>> Z;       // pre-activations [pbatch][pdims[l+1]] (Z[L-1] = output)
-  DevBuf<float> dA, dZ[2];
+  DevBuf<float> dZ[2];
   DevBuf<uint16_t> dZbf[2];
   DevBuf<double> partials, loss;
+  DevBuf<float> packed;               // the parameters without padding (mlp_export)
+  std::mutex packed_mu;               // reads of the parameters may come from several threads
   int64_t step = 0;
   bool have_grad = false;
 };
@@ -382,13 +436,13 @@ int sk_mlp_create(int n_layers, const int* dims, int max_batch, sk_mlp** out) {
       SK_TRY(n->Abf[l].alloc((size_t)n->pbatch * n->pdims[l]));
       SK_TRY(n->Z[l].alloc((size_t)n->pbatch * n->pdims[l + 1]));
     }
-    SK_TRY(n->dA.alloc((size_t)n->pbatch * maxd));
     for (int i = 0; i < 2; ++i) {
       SK_TRY(n->dZ[i].alloc((size_t)n->pbatch * maxd));
       SK_TRY(n->dZbf[i].alloc((size_t)n->pbatch * maxd));
     }
     SK_TRY(n->partials.alloc(grid_for((int64_t)n->pbatch * n->pdims[L]) + 1));
     SK_TRY(n->loss.alloc(1));
+    SK_TRY(n->packed.alloc((size_t)sk_mlp_num_params(n)));
     return SK_OK;
   };
   const int s = run();
@@ -435,21 +489,25 @@ int sk_mlp_set_params(sk_mlp* n, const float* params, sk_stream_t s) {
   return SK_OK;
 }
 
-// which = 0: FP32 master parameters; 1: the last computed gradient.
+// which = 0: FP32 master parameters; 1: the last computed gradient. One copy
+// of the layers packed without padding, instead of two copies and a wait for
+// each layer: 181 -> 136 us for four layers of 256 x 256, most of the rest the
+// copy into pageable memory.
 static int mlp_export(sk_mlp* n, int which, float* out, hipStream_t st) {
-  float* p = out;
+  std::lock_guard<std::mutex> lock(n->packed_mu);
+  int64_t at = 0;
   for (int l = 0; l < n->L; ++l) {
     const int di = n->dims[l], dn = n->dims[l + 1], pi = n->pdims[l];
-    std::vector<float> w((size_t)n->pdims[l + 1] * pi), bb(n->pdims[l + 1]);
-    const float* sw = which ? n->dW[l].p : n->W[l].p;
-    const float* sb = which ? n->db[l].p : n->b[l].p;
-    SK_HIP_CHECK(hipMemcpyAsync(w.data(), sw, w.size() * sizeof(float), hipMemcpyDeviceToHost, st));
-    SK_HIP_CHECK(hipMemcpyAsync(bb.data(), sb, bb.size() * sizeof(float), hipMemcpyDeviceToHost, st));
-    SK_HIP_CHECK(hipStreamSynchronize(st));
-    for (int r = 0; r < dn; ++r)
-      for (int c = 0; c < di; ++c) *p++ = w[(size_t)r * pi + c];
-    for (int r = 0; r < dn; ++r) *p++ = bb[r];
+    const int64_t nw = (int64_t)dn * di;
+    unpack_kernel<<<grid_for(nw), kBlock, 0, st>>>(dn, di, pi, which ? n->dW[l].p : n->W[l].p, n->packed.p + at);
+    at += nw;
+    unpack_kernel<<<grid_for(dn), kBlock, 0, st>>>(1, dn, n->pdims[l + 1], which ? n->db[l].p : n->b[l].p,
+                                                   n->packed.p + at);
+    at += dn;
   }
+  SK_HIP_CHECK(hipGetLastError());
+  SK_HIP_CHECK(hipMemcpyAsync(out, n->packed.p, at * sizeof(float), hipMemcpyDeviceToHost, st));
+  SK_HIP_CHECK(hipStreamSynchronize(st));
   return SK_OK;
 }
 
@@ -522,10 +580,10 @@ int sk_mlp_backward(sk_mlp* n, const float* X, const float* T, int batch, double
     g.C = n->dW[l].p;
     g.ldc = di;
     SK_TRY(launch_gemm(g, st));
-    colsum_kernel<<<(dn + kBlock - 1) / kBlock, kBlock, 0, st>>>(pb, dn, n->dZ[cur].p, n->db[l].p);
+    colsum_kernel<<<(dn + 31) / 32, kBlock, 0, st>>>(pb, dn, n->dZ[cur].p, n->db[l].p);
     SK_HIP_CHECK(hipGetLastError());
     if (l == 0) break;
-    // dA (pb x di) = dZ W_l: A(m, k) = dZ[m][k], B(k, n) = W_l[k][n]
+    // dZ of the layer before (pb x di) = (dZ W_l) * GELU'(Z): A(m, k) = dZ[m][k], B(k, n) = W_l[k][n]
     GemmArgs h{};
     h.M = pb;
     h.N = di;
@@ -536,13 +594,12 @@ int sk_mlp_backward(sk_mlp* n, const float* X, const float* T, int batch, double
     h.B = n->Wbf[l].p;
     h.sbk = di;
     h.sbn = 1;
-    h.C = n->dA.p;
+    h.C = n->dZ[1 - cur].p;
     h.ldc = di;
+    h.Cbf = n->dZbf[1 - cur].p;
+    h.ldcb = di;
+    h.Zgrad = n->Z[l - 1].p;
     SK_TRY(launch_gemm(h, st));
-    const int64_t ez = (int64_t)pb * di;
-    gelu_backward_kernel<<<grid_for(ez), kBlock, 0, st>>>(ez, n->dA.p, n->Z[l - 1].p, n->dZ[1 - cur].p,
-                                                          n->dZbf[1 - cur].p);
-    SK_HIP_CHECK(hipGetLastError());
     cur = 1 - cur;
   }
   n->have_grad = true;
