@@ -57,9 +57,12 @@ struct DevBuf {
   }
 };
 
-// Upper-triangle 3x3-block index of local pair (i <= j) of a tet: 0..9. The
-// blocks of one local row i are consecutive.
-__host__ __device__ constexpr int ublock(int i, int j) { return i * (7 - i) / 2 + j; }
+// Staged block of corners i <= j of a tet, the corners in ascending vertex
+// order: 0..5 for i < j, in the order (0,1) (0,2) (0,3) (2,3) (1,2) (1,3), so that
+// the blocks of one matrix row are together, and 6 + i on the diagonal.
+__host__ __device__ constexpr int kst_block(int i, int j) {
+  return i == j ? 6 + i : i == 0 ? j - 1 : i == 2 ? 3 : 2 + j;
+}
 
 // The inverse of a vertex's masked diagonal block (the block-Jacobi
 // preconditioner) is symmetric: the simulator stores its upper triangle
@@ -80,18 +83,11 @@ __device__ __forceinline__ void binv_load(const T* __restrict__ binv, int64_t v,
   B[8] = u2.y;
 }
 
-// Staged element stiffness: the 10 upper 3x3 blocks of K_e. Block u (ublock)
-// of element e sits at R-unit offset kKstR<R> e + kBlkStride<R> u. FP64
-// blocks are padded to 10 doubles (the padding is never written) so that the
-// gather reads them with five 16-byte loads; FP32 blocks stay at 9 floats
-// (padded to 12 the extra bytes cost more than the wider loads saved).
-// Records are not padded to whole cache lines: at 48^3 that wrote 5% more
-// bytes and took 6% longer in FP64.
-template <typename R>
-constexpr int kBlkStride = sizeof(R) == 8 ? 10 : 9;
-template <typename R>
-constexpr int kKstR = 10 * kBlkStride<R>;
-constexpr int kKst = 100;  // staging doubles per element (the larger of the two layouts)
+// Staged element stiffness K_e (symmetric): element e's record of kKst values
+// holds the six blocks above the diagonal (kst_block u, row-major, at 9 u), then
+// the upper triangles of the four diagonal blocks (block 6 + i at kKstDiag + 6 i,
+// in the order of kBinvPQ).
+constexpr int kKst = 78, kKstDiag = 54;
 constexpr int kSellC = 16;       // rows per SELL chunk
 constexpr int kSellLanes = 4;    // lanes per row in the SELL SpMV (kSellC * kSellLanes = wave size)
 constexpr int kFst = 12;  // staged doubles per element: f_e = vol P D
@@ -122,8 +118,11 @@ struct sk_mesh {
   sk::DevBuf<int32_t> bcol;   // [nblk] sorted neighbour vertex per block
   sk::DevBuf<int32_t> brow;   // [nblk] row vertex per block
   sk::DevBuf<int32_t> emap;   // [16][nt] block of local pair (i, j)
-  sk::DevBuf<int32_t> cptr;   // [nblk+1] contribution list per block
-  sk::DevBuf<int32_t> clist;  // [16 nt] (e << 4) | (4 i + j), e ascending per block
+  // The blocks the Hessian gather sums: the nv diagonal ones, then the (nblk - nv) / 2 above the diagonal in row
+  // order. gmeta[n] = (block, its transpose, first and end of its contributions in glist); a contribution is
+  // e << 5 | u << 1 for staged block u (kst_block) of element e, e ascending per block.
+  sk::DevBuf<int4> gmeta;
+  sk::DevBuf<uint32_t> glist;
   sk::DevBuf<int32_t> vptr;   // [nv+1] element incidences per vertex
   sk::DevBuf<int32_t> vlist;  // [4 nt] (e << 2) | i, e ascending per vertex
   // Sliced-ELL (SELL-C-sigma) layout of the simulator's matrix: rows sorted by

@@ -2,16 +2,14 @@
 //
 // Assembly is atomic-free and sort-free at run time. Set-up (host, once per
 // mesh) builds the sorted vertex-pair block pattern, the element -> block map
-// and, per block, the list of (element, local pair) contributions in
+// and, per block on or above the diagonal, the list of its contributions in
 // ascending element order. Each Hessian evaluation is then two launches:
 //   1. element pass: one lane per tet computes F, the 9x9 Hessian, its
-//      vol-weighted PSD projection and the 10 upper 3x3 blocks of
-//      K_e = B_e^T H+ B_e, staged per element (kKstR values, blocks padded
-//      to 16 bytes);
-//   2. block gather: one lane per CSR block sums its contributions in list
-//      order and writes the 3 row segments of the block. No two lanes write the
-//      same value and the summation order is fixed, so values are
-//      bit-reproducible.
+//      vol-weighted PSD projection and the upper triangle of
+//      K_e = B_e^T H+ B_e, staged per element (kKst values);
+//   2. block gather: sums each block's contributions in a fixed order and
+//      writes the 3 row segments of the block and of its transpose. No two
+//      lanes write the same value, so values are bit-reproducible.
 #include "sk_elem.h"
 #include "sk_internal.h"
 #include "sk_materials.h"
@@ -153,6 +151,9 @@ __device__ __forceinline__ void wave_count(bool flag, unsigned long long* count)
   if (flag && (int)__lane_id() == __ffsll((long long)m) - 1) atomicAdd(count, (unsigned long long)__popcll(m));
 }
 
+// Orders a wave's LDS accesses among its lanes (the wave's own accesses are in order).
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // kMode 0: Hessian, vol weight and 9x9 Jacobi PSD projection for every
 // element. kMode 1 (densities with a closed-form eigensystem, PSD on): the
 // eigenvalue modification from that eigensystem; elements it declines are
@@ -161,60 +162,153 @@ __device__ __forceinline__ void wave_count(bool flag, unsigned long long* count)
 // closed-form kernel's registers (and occupancy) free of the 9x9 Jacobi's.
 template <template <typename> class M, int PSD, typename R, int kMode = 0>
 __global__ __launch_bounds__(kBlock) void elem_hess_kernel(ElemArgs a) {
+  __shared__ __align__(16) R stage[kBlock / kWave][kWave * 18];
   const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= a.m.nt) return;
-  if (a.active && !a.active[a.pid[a.m.T[e]]]) return;
-  if (kMode == 2 && !a.flags[e]) return;
-  int32_t v[4];
-  double Dd[12], xe[12], F[9];
-  load_elem(a.m, e, v, Dd);
-  gather_x(a.x, v, xe);
-  make_F(xe, Dd, F);
-  add_F0(a.F0, e, F);
-  R H[45];
-  if constexpr (kMode == 1) {
-    R Fr[9];
+  bool live = e < a.m.nt && !(a.active && !a.active[a.pid[a.m.T[e]]]) && !(kMode == 2 && !a.flags[e]);
+  R H[45], D[12];
+  if (live) {
+    int32_t v[4];
+    double Dd[12], xe[12], F[9];
+    load_elem(a.m, e, v, Dd);
+    gather_x(a.x, v, xe);
+    make_F(xe, Dd, F);
+    add_F0(a.F0, e, F);
+    if constexpr (kMode == 1) {
+      R Fr[9];
 #pragma unroll
-    for (int k = 0; k < 9; ++k) Fr[k] = (R)F[k];
-    const bool ok = M<R>::hessian_psd_analytic(Fr, (R)a.mu[e], a.lam ? (R)a.lam[e] : R(0), (R)a.vol[e], PSD,
-                                               R(1e-6), H);
-    a.flags[e] = ok ? 0 : 1;
-    if (!ok) return;
-  } else {
-    const bool fp64_polar = elem_hessian_eval<M, R>(F, a.mu[e], a.lam ? a.lam[e] : 0.0, H);
-    if (sizeof(R) == 4 && M<R>::kPolar && a.fp64_count) wave_count(fp64_polar, a.fp64_count);
-    const R vol = (R)a.vol[e];
+      for (int k = 0; k < 9; ++k) Fr[k] = (R)F[k];
+      live = M<R>::hessian_psd_analytic(Fr, (R)a.mu[e], a.lam ? (R)a.lam[e] : R(0), (R)a.vol[e], PSD, R(1e-6), H);
+      a.flags[e] = live ? 0 : 1;
+    } else {
+      const bool fp64_polar = elem_hessian_eval<M, R>(F, a.mu[e], a.lam ? a.lam[e] : 0.0, H);
+      if (sizeof(R) == 4 && M<R>::kPolar && a.fp64_count) wave_count(fp64_polar, a.fp64_count);
+      const R vol = (R)a.vol[e];
 #pragma unroll
-    for (int k = 0; k < 45; ++k) H[k] *= vol;
-    if (PSD != SK_PSD_NONE) psd_project_sym<9, R>(H, PSD, R(1e-6));
+      for (int k = 0; k < 45; ++k) H[k] *= vol;
+      if (PSD != SK_PSD_NONE) psd_project_sym<9, R>(H, PSD, R(1e-6));
+    }
+#pragma unroll
+    for (int k = 0; k < 12; ++k) D[k] = (R)Dd[k];
+    // the corners in ascending vertex order
+    int32_t key[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) key[k] = 4 * v[k] + k;
+    auto order = [&](int i, int j) {
+      const bool swap = key[i] > key[j];
+      const int32_t ki = key[i];
+      key[i] = swap ? key[j] : ki;
+      key[j] = swap ? ki : key[j];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const R di = D[4 * c + i], dj = D[4 * c + j];
+        D[4 * c + i] = swap ? dj : di;
+        D[4 * c + j] = swap ? di : dj;
+      }
+    };
+    order(0, 1);
+    order(2, 3);
+    order(0, 2);
+    order(1, 3);
+    order(1, 2);
   }
-  R D[12];
+  // K_e[3i+p][3j+q] = sum_{c,c'} D[c][i] H[3p+c][3q+c'] D[c'][j], a few values of the wave's elements at a
+  // time through LDS, so that neighbouring lanes store neighbouring words: a record written by its own lane
+  // reached L2 as 8- and 16-byte pieces, whose number and not their bytes took the time (48^3 with PSD, FP64
+  // 254 -> 136 us, FP32 95 -> 88 us).
+  const uint64_t lives = __ballot(live);
+  if (!lives) return;
+  const int lane = threadIdx.x % kWave;
+  R* mine = stage[threadIdx.x / kWave];
+  R* out = reinterpret_cast<R*>(a.Kst) + (int64_t)kKst * (e - lane);
+  using W = std::conditional_t<sizeof(R) == 8, double2, float3>;  // what a lane stores at once
+  constexpr int kW = sizeof(W) / sizeof(R);
+  // the NV values of every lane at mine[NV lane] to its record's offset `at`
+  auto flush = [&](auto nv, int at) {
+    constexpr int NV = decltype(nv)::value, kPer = NV / kW;
+    wave_lds_fence();
 #pragma unroll
-  for (int k = 0; k < 12; ++k) D[k] = (R)Dd[k];
-  // K_e[3i+p][3j+q] = sum_{c,c'} D[c][i] H[3p+c][3q+c'] D[c'][j], upper blocks i <= j,
-  // written one local row i at a time: row i's blocks are consecutive in the
-  // record, so its cache lines are complete before the next row starts
-  R* out = reinterpret_cast<R*>(a.Kst) + (int64_t)kKstR<R> * e;
+    for (int k = 0; k < kPer; ++k) {
+      const int n = k * kWave + lane, el = n / kPer;
+      if (lives >> el & 1)
+        *reinterpret_cast<W*>(out + (int64_t)kKst * el + at + n % kPer * kW) = reinterpret_cast<const W*>(mine)[n];
+    }
+    wave_lds_fence();
+  };
+  using Pair = std::integral_constant<int, 18>;
+  using Diag = std::integral_constant<int, 6>;
+  R w[3][9];  // w[p][3q+c'] = sum_c D[c][i] H[3p+c][3q+c']
+  auto left = [&](int i) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int p = 0; p < 3; ++p) {
-      R w[9];  // w[3q+c'] = sum_c D[c][i] H[3p+c][3q+c']
+    for (int p = 0; p < 3; ++p)
 #pragma unroll
       for (int m = 0; m < 9; ++m)
-        w[m] = D[i] * H[Sym<9>::idx(3 * p, m)] + D[4 + i] * H[Sym<9>::idx(3 * p + 1, m)] +
-               D[8 + i] * H[Sym<9>::idx(3 * p + 2, m)];
+        w[p][m] = D[i] * H[Sym<9>::idx(3 * p, m)] + D[4 + i] * H[Sym<9>::idx(3 * p + 1, m)] +
+                  D[8 + i] * H[Sym<9>::idx(3 * p + 2, m)];
+  };
+  auto entry = [&](int j, int p, int q) { return w[p][3 * q] * D[j] + w[p][3 * q + 1] * D[4 + j] + w[p][3 * q + 2] * D[8 + j]; };
+  auto block = [&](int j, R* o) {
 #pragma unroll
-      for (int j = i; j < 4; ++j)
+    for (int p = 0; p < 3; ++p)
 #pragma unroll
-        for (int q = 0; q < 3; ++q)
-          out[ublock(i, j) * kBlkStride<R> + 3 * p + q] = w[3 * q] * D[j] + w[3 * q + 1] * D[4 + j] + w[3 * q + 2] * D[8 + j];
+      for (int q = 0; q < 3; ++q) o[3 * p + q] = entry(j, p, q);
+  };
+  auto diagonal = [&](int i) {
+    if (live) {
+#pragma unroll
+      for (int u = 0; u < 6; ++u) mine[6 * lane + u] = entry(i, kBinvPQ[u][0], kBinvPQ[u][1]);
     }
+    flush(Diag{}, kKstDiag + 6 * i);
+  };
+  R b03[9];
+  if (live) {
+    left(0);
+    block(1, mine + 18 * lane);
+    block(2, mine + 18 * lane + 9);
+    block(3, b03);
+  }
+  flush(Pair{}, 0);
+  diagonal(0);
+  if (live) {
+    left(2);
+#pragma unroll
+    for (int m = 0; m < 9; ++m) mine[18 * lane + m] = b03[m];
+    block(3, mine + 18 * lane + 9);
+  }
+  flush(Pair{}, 18);
+  diagonal(2);
+  if (live) {
+    left(1);
+    block(2, mine + 18 * lane);
+    block(3, mine + 18 * lane + 9);
+  }
+  flush(Pair{}, 36);
+  diagonal(1);
+  if (live) left(3);
+  diagonal(3);
 }
 
 // ---------------------------------------------------------------------------
 // Gathers
 // ---------------------------------------------------------------------------
+// Sum over the four lanes of a quad, in each of them: (x0 + x1) + (x2 + x3).
+template <int kPerm>
+__device__ __forceinline__ float quad_perm(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), kPerm, 0xf, 0xf, true));
+}
+template <int kPerm>
+__device__ __forceinline__ double quad_perm(double x) {
+  const uint64_t u = (uint64_t)__double_as_longlong(x);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kPerm, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kPerm, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <typename R>
+__device__ __forceinline__ R quad_sum(R x) {
+  x += quad_perm<0xB1>(x);         // [1, 0, 3, 2]
+  return x + quad_perm<0x4E>(x);   // [2, 3, 0, 1]
+}
+constexpr int kQuad = 4;
+
 struct GatherGArgs {
   int64_t nv;
   const int32_t* vptr;
@@ -230,13 +324,19 @@ struct GatherGArgs {
   double* partials;
 };
 
+// Four lanes per vertex: lane s sums the incidences s, s + 4, ... of the list,
+// then lane c writes DOF c. A lane per vertex was a chain of up to 32 dependent
+// loads on few waves: 10^3 22.5 -> 5.7 us, a 29 x 13 x 21 box 20 -> 11.5; at 48^3
+// the reads themselves bound it (42 -> 41 us).
 __global__ __launch_bounds__(kBlock) void gather_grad_kernel(GatherGArgs a) {
-  const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const int s = threadIdx.x % kQuad;
   double nrm = 0.0;
-  if (v < a.nv) {
+  for (int64_t v = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kQuad; v < a.nv;
+       v += (int64_t)gridDim.x * (kBlock / kQuad)) {
     double acc[3] = {0.0, 0.0, 0.0};
-    const int32_t k0 = a.vptr[v], k1 = a.vptr[v + 1];
-    for (int32_t k = k0; k < k1; ++k) {
+    const int32_t k1 = a.vptr[v + 1];
+#pragma unroll 2
+    for (int32_t k = a.vptr[v] + s; k < k1; k += kQuad) {
       const int32_t pk = a.vlist[k];
       const double* f = a.fst + (int64_t)kFst * (pk >> 2) + 3 * (pk & 3);
       acc[0] += f[0];
@@ -244,9 +344,10 @@ __global__ __launch_bounds__(kBlock) void gather_grad_kernel(GatherGArgs a) {
       acc[2] += f[2];
     }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const int64_t k = 3 * v + c;
-      double gk = acc[c];
+    for (int c = 0; c < 3; ++c) acc[c] = quad_sum(acc[c]);
+    if (s < 3) {
+      const int64_t k = 3 * v + s;
+      double gk = s == 0 ? acc[0] : s == 1 ? acc[1] : acc[2];
       if (a.mass) {
         gk += a.mass[k] * (a.x[k] - a.xt[k]) * a.inv_h2;
         if (a.fext) gk -= a.fext[k];
@@ -263,12 +364,13 @@ __global__ __launch_bounds__(kBlock) void gather_grad_kernel(GatherGArgs a) {
 }
 
 struct GatherHArgs {
-  int64_t nblk;
+  int64_t nv;
+  int64_t noff;             // off-diagonal blocks above the diagonal
+  int64_t dgrid;            // workgroups of the diagonal blocks
+  const int4* gmeta;        // [nv + noff]
+  const uint32_t* glist;
   const int32_t* bptr;
-  const int32_t* bcol;
   const int32_t* brow;
-  const int32_t* cptr;
-  const int32_t* clist;
   const void* Kst;
   void* values;
   const double* mass;
@@ -283,103 +385,139 @@ struct GatherHArgs {
   const int32_t* pid;
 };
 
-// A staged block: FP64 in five 16-byte loads (16-byte aligned, padded to 10),
-// FP32 in nine 4-byte loads.
+// A staged block above the diagonal (9 values) or on it (its upper triangle, 6).
+typedef double sk_d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float sk_f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_staged(const double* __restrict__ s, double (&B)[9]) {
+  const sk_d2u* v = reinterpret_cast<const sk_d2u*>(s);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const sk_d2u d = v[t];
+    B[2 * t] = d.x;
+    B[2 * t + 1] = d.y;
+  }
+  B[8] = s[8];
+}
+__device__ __forceinline__ void load_staged(const float* __restrict__ s, float (&B)[9]) {
+  const sk_f4u a = *reinterpret_cast<const sk_f4u*>(s), b = *reinterpret_cast<const sk_f4u*>(s + 4);
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    B[t] = a[t];
+    B[4 + t] = b[t];
+  }
+  B[8] = s[8];
+}
 template <typename R>
-__device__ __forceinline__ void load_staged_block(const R* __restrict__ s, R (&B)[kBlkStride<R>]) {
-  if constexpr (sizeof(R) == 8) {
-    const double2* v = reinterpret_cast<const double2*>(s);
+__device__ __forceinline__ void load_staged_diag(const R* __restrict__ s, R (&B)[6]) {
+  using R2 = std::conditional_t<sizeof(R) == 8, double2, float2>;
+  const R2* v = reinterpret_cast<const R2*>(s);
 #pragma unroll
-    for (int t = 0; t < 5; ++t) {
-      const double2 d = v[t];
-      B[2 * t] = d.x;
-      B[2 * t + 1] = d.y;
-    }
-  } else {
-#pragma unroll
-    for (int m = 0; m < 9; ++m) B[m] = s[m];
+  for (int t = 0; t < 3; ++t) {
+    const R2 d = v[t];
+    B[2 * t] = d.x;
+    B[2 * t + 1] = d.y;
   }
 }
 
-// Contributions loaded per pass of the gather loop. Measured at 48^3 as the
-// FP64 Hessian phase per Newton iteration (element pass + gather): 1 per pass
-// 0.780 ms, 2 per pass 0.710 ms, 4 per pass 0.725 ms.
-constexpr int kGatherU = 2;
-
-// One lane per block: sums the staged contributions in list order (precision
-// R), adds the lumped mass / h^2 on diagonal blocks, writes the block in CSR,
-// BSR or a sliced order and, for diagonal blocks, the inverse of the
-// fixed-DOF-masked block (inverse of diag(f) A diag(f) + diag(1 - f), masked to
-// the free DOFs).
+// Sums the staged contributions of a block (precision R), adds the lumped mass
+// / h^2 on diagonal blocks, writes the block in CSR, BSR or a sliced order and,
+// for diagonal blocks, the inverse of the fixed-DOF-masked block (inverse of
+// diag(f) A diag(f) + diag(1 - f), masked to the free DOFs).
+//
+// The matrix is symmetric: only blocks on and above the diagonal are summed,
+// an off-diagonal one by one lane that also writes its transpose. Diagonal
+// blocks have several times the contributions of the others (on a grid of five
+// tets per cell 32 or 8 against 4 to 6), so four lanes share one, lane s taking
+// contributions s, s + 4, ..., and workgroups hold either diagonal or
+// off-diagonal blocks. Workgroups of one XCD take consecutive rows, the diagonal
+// ones among the others, for the records they share. Bound by the scattered
+// reads of the records (80 to 216 bytes at a time) and writes of the blocks. One
+// lane per block in row order, every off-diagonal block read twice, took 314 us
+// at 48^3 (FP64, CSR order), this 241 us; 10^3 19.9 -> 9.4 us, FP32 at 48^3 193 -> 160 us.
+// Two contributions at a time: one or four took 70 and 15 us more.
 template <typename R>
 __global__ __launch_bounds__(kBlock) void gather_hess_kernel(GatherHArgs a) {
-  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= a.nblk) return;
-  if (a.active && !a.active[a.pid[a.brow[b]]]) return;
+  // workgroup `wg` in matrix order: an eighth of the list per XCD, the diagonal workgroups spread evenly
+  const int64_t eighth = gridDim.x / 8, wg = blockIdx.x < 8 * eighth ? blockIdx.x % 8 * eighth + blockIdx.x / 8 : blockIdx.x;
+  const int64_t d0 = wg * a.dgrid / gridDim.x, d1 = (wg + 1) * a.dgrid / gridDim.x;  // diagonal ones before it, and with it
+  const bool diag = d1 > d0;
+  const int64_t at = (diag ? d0 : wg - d0) * kBlock + threadIdx.x;
+  const int64_t n = diag ? at / kQuad : at;
+  if (n >= (diag ? a.nv : a.noff)) return;
+  const int4 gm = a.gmeta[diag ? n : a.nv + n];  // block, its transpose, contributions [z, w)
+  const int32_t v = a.brow[gm.x], w = a.brow[gm.y];
+  if (a.active && !a.active[a.pid[v]]) return;
   const R* __restrict__ Kst = reinterpret_cast<const R*>(a.Kst);
+  auto record = [&](uint32_t c) { return Kst + kKst * (int64_t)(c >> 5); };
   R acc[9];
 #pragma unroll
   for (int k = 0; k < 9; ++k) acc[k] = R(0);
-  // the staged upper block (min(i,j), max(i,j)) of contribution pk, used
-  // transposed when i > j: one load path for every lane, the transpose by selects
-  auto source = [&](int32_t pk, bool& tr) {
-    const int i = (pk >> 2) & 3, j = pk & 3;
-    tr = i > j;
-    return Kst + kKstR<R> * (int64_t)(pk >> 4) + kBlkStride<R> * ublock(tr ? j : i, tr ? i : j);
-  };
-  auto accumulate = [&](const R (&B)[kBlkStride<R>], bool tr) {
-    acc[0] += B[0];
-    acc[4] += B[4];
-    acc[8] += B[8];
-    acc[1] += tr ? B[3] : B[1];
-    acc[3] += tr ? B[1] : B[3];
-    acc[2] += tr ? B[6] : B[2];
-    acc[6] += tr ? B[2] : B[6];
-    acc[5] += tr ? B[7] : B[5];
-    acc[7] += tr ? B[5] : B[7];
-  };
-  const int32_t k0 = a.cptr[b], k1 = a.cptr[b + 1];
-  int32_t k = k0;
-  // kGatherU contributions per pass: their blocks' loads in flight together, summed in list order
-  constexpr int U = kGatherU;
-  for (; k + U <= k1; k += U) {
-    bool t[U];
-    R B[U][kBlkStride<R>];
+  if (diag) {
+    const int s = threadIdx.x % kQuad;
+#pragma unroll 2
+    for (int32_t k = gm.z + s; k < gm.w; k += kQuad) {
+      const uint32_t c = a.glist[k], u = c >> 1 & 15;
+      if (u >= 6) {
+        R B[6];
+        load_staged_diag(record(c) + kKstDiag + 6 * (u - 6), B);
 #pragma unroll
-    for (int u = 0; u < U; ++u) load_staged_block<R>(source(a.clist[k + u], t[u]), B[u]);
+        for (int m = 0; m < 6; ++m) acc[3 * kBinvPQ[m][0] + kBinvPQ[m][1]] += B[m];
+      } else {  // a tet that has the vertex twice: K_ij + K_ji, half of the sum for each of the two entries
+        R B[9];
+        load_staged(record(c) + 9 * u, B);
 #pragma unroll
-    for (int u = 0; u < U; ++u) accumulate(B[u], t[u]);
+        for (int m = 0; m < 6; ++m) {
+          const int p = kBinvPQ[m][0], q = kBinvPQ[m][1];
+          acc[3 * p + q] += R(0.5) * (B[3 * p + q] + B[3 * q + p]);
+        }
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+      const int p = kBinvPQ[m][0], q = kBinvPQ[m][1];
+      acc[3 * q + p] = acc[3 * p + q] = quad_sum(acc[3 * p + q]);
+    }
+    if (s != 0) return;
+  } else {
+#pragma unroll 2
+    for (int32_t k = gm.z; k < gm.w; ++k) {
+      const uint32_t c = a.glist[k];
+      R B[9];
+      load_staged(record(c) + 9 * (c >> 1 & 15), B);
+#pragma unroll
+      for (int m = 0; m < 9; ++m) acc[m] += B[m];
+    }
   }
-  for (; k < k1; ++k) {
-    bool t0;
-    R B0[kBlkStride<R>];
-    load_staged_block<R>(source(a.clist[k], t0), B0);
-    accumulate(B0, t0);
-  }
-  const int32_t v = a.brow[b], w = a.bcol[b];
-  const int32_t b0 = a.bptr[v], deg = a.bptr[v + 1] - b0, r = (int32_t)(b - b0);
-  if (v == w && a.mass) {
+  if (diag && a.mass) {
 #pragma unroll
     for (int p = 0; p < 3; ++p) acc[4 * p] += (R)(a.mass[3 * (int64_t)v + p] * a.inv_h2);
   }
   R* values = reinterpret_cast<R*>(a.values);
-  if (a.sell_pos) {
-    const int64_t q = a.sell_pos[b];
+  auto write = [&](int64_t b, int32_t row, const R (&B)[9]) {
+    if (a.sell_pos) {
+      const int64_t q = a.sell_pos[b];
 #pragma unroll
-    for (int m = 0; m < 9; ++m)
-      values[a.quad ? slot_index<kQuadC, kQuadVW>(q, m) : slot_index<kSellC, 1>(q, m)] = acc[m];
-  } else if (a.bsr) {
-    R* out = values + 9 * b;
+      for (int m = 0; m < 9; ++m)
+        values[a.quad ? slot_index<kQuadC, kQuadVW>(q, m) : slot_index<kSellC, 1>(q, m)] = B[m];
+    } else if (a.bsr) {
+      R* out = values + 9 * b;
 #pragma unroll
-    for (int m = 0; m < 9; ++m) out[m] = acc[m];
-  } else {
-    R* out = values + 9 * (int64_t)b0 + 3 * r;
+      for (int m = 0; m < 9; ++m) out[m] = B[m];
+    } else {
+      const int32_t b0 = a.bptr[row], deg = a.bptr[row + 1] - b0;
+      R* out = values + 9 * (int64_t)b0 + 3 * (b - b0);
 #pragma unroll
-    for (int p = 0; p < 3; ++p)
+      for (int p = 0; p < 3; ++p)
 #pragma unroll
-      for (int q = 0; q < 3; ++q) out[3 * p * deg + q] = acc[3 * p + q];
+        for (int q = 0; q < 3; ++q) out[3 * p * deg + q] = B[3 * p + q];
+    }
+  };
+  write(gm.x, v, acc);
+  if (!diag) {
+    const R t[9] = {acc[0], acc[3], acc[6], acc[1], acc[4], acc[7], acc[2], acc[5], acc[8]};
+    write(gm.y, w, t);
   }
-  if (v == w && a.binv) {
+  if (diag && a.binv) {
     R f[3];
 #pragma unroll
     for (int p = 0; p < 3; ++p) f[p] = (a.fixed && a.fixed[3 * (int64_t)v + p]) ? R(0) : R(1);
@@ -568,10 +706,39 @@ int launch_count_inverted(sk_mesh* m, const double* x, double* result, hipStream
 int launch_gather_grad(sk_mesh* m, double* g, const double* mass, const double* x, const double* xt,
                        const double* fext, const uint8_t* fixed, double inv_h2, hipStream_t st) {
   GatherGArgs a{m->nv, m->vptr.p, m->vlist.p, m->fst.p, g, mass, x, xt, fext, fixed, inv_h2, m->red.partials.p};
-  const int gr = grid_for(m->nv);
-  SK_REQUIRE(gr <= Reducer::kMaxBlocks, "mesh too large for the gradient reduction");
+  SK_REQUIRE(grid_for(m->nv) <= Reducer::kMaxBlocks, "mesh too large for the gradient reduction");
+  const int gr = std::min(grid_for(kQuad * m->nv), 2048);  // eight workgroups per CU, then several vertices a quad
   gather_grad_kernel<<<gr, kBlock, 0, st>>>(a);
   if (mass) finalize_sum_kernel<1><<<1, kBlock, 0, st>>>(m->red.partials.p, gr, m->red.result.p);
+  SK_HIP_CHECK(hipGetLastError());
+  return SK_OK;
+}
+
+static GatherHArgs gather_args(const sk_mesh* m, void* values, const double* mass, double inv_h2, const uint8_t* fixed,
+                               void* binv, const int* active, const int32_t* pid) {
+  GatherHArgs a{};
+  a.nv = m->nv;
+  a.noff = (m->nblk - m->nv) / 2;
+  a.dgrid = grid_for(kQuad * m->nv);
+  a.gmeta = m->gmeta.p;
+  a.glist = m->glist.p;
+  a.bptr = m->bptr.p;
+  a.brow = m->brow.p;
+  a.Kst = m->Kst.p;
+  a.values = values;
+  a.mass = mass;
+  a.inv_h2 = inv_h2;
+  a.fixed = fixed;
+  a.binv = binv;
+  a.active = active;
+  a.pid = pid;
+  return a;
+}
+
+static int run_gather_hess(const GatherHArgs& a, bool fp32, hipStream_t st) {
+  const unsigned g = (unsigned)(a.dgrid + (a.noff ? grid_for(a.noff) : 0));
+  if (fp32) gather_hess_kernel<float><<<g, kBlock, 0, st>>>(a);
+  else gather_hess_kernel<double><<<g, kBlock, 0, st>>>(a);
   SK_HIP_CHECK(hipGetLastError());
   return SK_OK;
 }
@@ -580,13 +747,10 @@ int launch_gather_hess(sk_mesh* m, void* values, const double* mass, double inv_
                        void* binv, int layout, bool fp32, hipStream_t st, const int* active, const int32_t* pid) {
   SK_REQUIRE(layout == kLayoutCSR || layout == kLayoutSELL || layout == kLayoutBSR, "invalid value layout");
   SK_REQUIRE(!active == !pid, "launch_gather_hess: active and pid go together");
-  GatherHArgs a{m->nblk, m->bptr.p, m->bcol.p, m->brow.p, m->cptr.p, m->clist.p, m->Kst.p,
-                values, mass, inv_h2, fixed, binv, layout == kLayoutSELL ? m->sell_pos.p : nullptr, 0,
-                nullptr, layout == kLayoutBSR ? 1 : 0, active, pid};
-  if (fp32) gather_hess_kernel<float><<<grid_for(m->nblk), kBlock, 0, st>>>(a);
-  else gather_hess_kernel<double><<<grid_for(m->nblk), kBlock, 0, st>>>(a);
-  SK_HIP_CHECK(hipGetLastError());
-  return SK_OK;
+  GatherHArgs a = gather_args(m, values, mass, inv_h2, fixed, binv, active, pid);
+  a.sell_pos = layout == kLayoutSELL ? m->sell_pos.p : nullptr;
+  a.bsr = layout == kLayoutBSR ? 1 : 0;
+  return run_gather_hess(a, fp32, st);
 }
 
 int launch_gather_hess_quad(sk_mesh* m, void* values, const double* mass, double inv_h2, const uint8_t* fixed,
@@ -595,12 +759,11 @@ int launch_gather_hess_quad(sk_mesh* m, void* values, const double* mass, double
   SK_REQUIRE(pos && (!binv || row_pos), "launch_gather_hess_quad: missing slot map");
   SK_REQUIRE(fp32, "launch_gather_hess_quad: the quad layout holds FP32 values");
   SK_REQUIRE(!active == !pid, "launch_gather_hess_quad: active and pid go together");
-  GatherHArgs a{m->nblk, m->bptr.p, m->bcol.p, m->brow.p, m->cptr.p, m->clist.p, m->Kst.p,
-                values, mass, inv_h2, fixed, binv, pos, 1, row_pos, 0, active, pid};
-  if (fp32) gather_hess_kernel<float><<<grid_for(m->nblk), kBlock, 0, st>>>(a);
-  else gather_hess_kernel<double><<<grid_for(m->nblk), kBlock, 0, st>>>(a);
-  SK_HIP_CHECK(hipGetLastError());
-  return SK_OK;
+  GatherHArgs a = gather_args(m, values, mass, inv_h2, fixed, binv, active, pid);
+  a.sell_pos = pos;
+  a.quad = 1;
+  a.binv_pos = row_pos;
+  return run_gather_hess(a, fp32, st);
 }
 
 int read_scalars(sk_mesh* m, const double* dev, int n, hipStream_t st) {
@@ -675,7 +838,7 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
   for (auto& c : cols) nblk += (int64_t)c.size();
   SK_REQUIRE(9 * nblk < (int64_t(1) << 31), "sk_mesh_create: nnz exceeds int32 indexing");
   std::partial_sum(bptr.begin(), bptr.end(), bptr.begin());
-  std::vector<int32_t> bcol(nblk), brow(nblk), emap(16 * nt), cptr(nblk + 1, 0), clist(16 * nt);
+  std::vector<int32_t> bcol(nblk), brow(nblk), emap(16 * nt), cnt(nblk, 0);
   ranges([&](int k, int64_t v0, int64_t v1) {
     std::copy(cols[k].begin(), cols[k].end(), bcol.begin() + bptr[v0]);
     std::vector<int32_t> at(nv);  // block of the current row at each of its columns
@@ -690,21 +853,60 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
         for (int j = 0; j < 4; ++j) {
           const int32_t b = at[T[4 * e + j]];
           emap[(4 * i + j) * nt + e] = b;
-          cptr[b + 1]++;
+          cnt[b]++;
         }
       }
     }
   });
-  std::partial_sum(cptr.begin(), cptr.end(), cptr.begin());
+  // The blocks that the gather sums, diagonal ones first, then those above the diagonal row by row, and their
+  // contribution lists in that order.
+  const int64_t noff = (nblk - nv) / 2;
+  std::vector<int4> gmeta(nv + noff);
+  std::vector<int32_t> goff(nv + 1, 0);  // off-diagonal blocks of the rows before
+  for (int64_t v = 0; v < nv; ++v)
+    goff[v + 1] = goff[v] + (int32_t)(bcol.begin() + bptr[v + 1] -
+                                      std::upper_bound(bcol.begin() + bptr[v], bcol.begin() + bptr[v + 1], (int32_t)v));
   ranges([&](int, int64_t v0, int64_t v1) {
-    std::vector<int32_t> fill(cptr.begin() + bptr[v0], cptr.begin() + bptr[v1]);
-    for (int64_t v = v0; v < v1; ++v)
+    for (int64_t v = v0; v < v1; ++v) {
+      int32_t o = goff[v];
+      for (int32_t b = bptr[v]; b < bptr[v + 1]; ++b) {
+        const int32_t w = bcol[b];
+        if (w == v) gmeta[v] = make_int4(b, b, 0, cnt[b]);
+        if (w <= v) continue;
+        const auto r = bcol.begin() + bptr[w];
+        const int32_t t = (int32_t)(std::lower_bound(r, bcol.begin() + bptr[w + 1], (int32_t)v) - bcol.begin());
+        gmeta[nv + o++] = make_int4(b, t, 0, cnt[b]);
+      }
+    }
+  });
+  int32_t nlist = 0;
+  for (int4& g : gmeta) {
+    g.z = nlist;
+    nlist += g.w;
+    g.w = nlist;
+  }
+  std::vector<uint32_t> glist(nlist);
+  ranges([&](int, int64_t v0, int64_t v1) {
+    std::vector<int32_t> fill(nv);  // next entry of the current row's block at each of its columns w >= v
+    for (int64_t v = v0; v < v1; ++v) {
+      fill[v] = gmeta[v].z;
+      for (int32_t o = goff[v]; o < goff[v + 1]; ++o) fill[bcol[gmeta[nv + o].x]] = gmeta[nv + o].z;
       for (int32_t q = vptr[v]; q < vptr[v + 1]; ++q) {
         const int64_t e = vlist[q] >> 2;
         const int i = vlist[q] & 3;
-        for (int j = 0; j < 4; ++j)
-          clist[fill[emap[(4 * i + j) * nt + e] - bptr[v0]]++] = (int32_t)((e << 4) | (4 * i + j));
+        const int32_t* c = T + 4 * e;
+        auto place = [&](int j) {  // of corner j in ascending vertex order
+          int r = 0;
+          for (int k = 0; k < 4; ++k) r += c[k] < c[j] || (c[k] == c[j] && k < j);
+          return r;
+        };
+        for (int j = 0; j < 4; ++j) {
+          if (c[j] < v) continue;
+          const int pi = place(i), pj = place(j);
+          glist[fill[c[j]]++] = (uint32_t)e << 5 | (uint32_t)kst_block(std::min(pi, pj), std::max(pi, pj)) << 1;
+        }
       }
+    }
   });
   // SELL-C-sigma layout: rows sorted by block count (descending, stable, so
   // rows of equal degree keep their spatial order), chunks of kSellC rows.
@@ -786,8 +988,8 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
   SK_TRY(m->bcol.upload(bcol));
   SK_TRY(m->brow.upload(brow));
   SK_TRY(m->emap.upload(emap));
-  SK_TRY(m->cptr.upload(cptr));
-  SK_TRY(m->clist.upload(clist));
+  SK_TRY(m->gmeta.upload(gmeta));
+  SK_TRY(m->glist.upload(glist));
   SK_TRY(m->vptr.upload(vptr));
   SK_TRY(m->vlist.upload(vlist));
   SK_TRY(m->sell_row.upload(sell_row));
