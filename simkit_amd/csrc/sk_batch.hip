@@ -28,6 +28,8 @@
 // reads the active flags on the device; it is captured once in a hipGraph
 // and replayed. Workgroup size and rows-per-lane layout of the per-problem
 // kernels are chosen by sk_batch_autotune (timed on the batch itself).
+// One launch shape (512 threads, one lane per row, vectors in LDS) has a PCG
+// kernel and an order of the values of its own: batch_pcg_even_kernel.
 #include "sk_coarse.h"
 #include "sk_elem.h"
 #include "sk_internal.h"
@@ -723,6 +725,577 @@ __global__ __launch_bounds__(NT) void batch_pcg_kernel(BatchArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// The same PCG with the matrix blocks dealt evenly to the threads: the shape 512
+// threads, one lane per row, vectors in LDS, wherever a problem's data fit.
+//
+// The problem's blocks, in row order, are dealt K consecutive ones to a thread;
+// the gather writes them in that order (block k of thread t at slot k kEvenNT + t
+// of the problem, quad layout), so that every load of a wave is one contiguous
+// run. The first kEvenKR stay in registers, the next KL in the LDS the vectors
+// leave over, and the rest are streamed, kEvenDepth blocks under way. A product
+// leaves one partial per (row, thread) pair at slot row + thread (consecutive for
+// a row), which the row's thread adds in order; the residual replacement runs the
+// same product in FP64. Threads own rows t, t + kEvenNT, ...; a wave's rows lie in
+// one aggregate. The coarse inverse is read four columns per load, a thread's
+// first rows of it on their way while x and r are updated.
+//
+// Why: with a lane per row every sweep of rows is a chain of 5 to 8 dependent
+// batches of loads on 8 waves, lanes of short rows idle, and the coarse inverse
+// comes in 4-byte loads. The 512-beam batch (8 to 64 cells long, 960 rows and
+// 10,000 blocks on average, 50 to 100 iterations) took 5,467 us per launch and
+// 1.6 TB/s over the chip; this takes 2,400 us. What bounds it now is the latency of
+// the phases between barriers: of 13.5 us per iteration at 950 rows the product is
+// 3.8, the update of x and r 2.3, the coarse product 5.5 (at 1,625 rows 7.5, 3.5 and
+// 6.8 of 20.6).
+// ---------------------------------------------------------------------------
+constexpr int kEvenNT = 512;          // threads per workgroup
+constexpr int kEvenKR = 8;            // blocks per thread in registers
+constexpr int kEvenMaxKL = 6;         // and in LDS, at most
+constexpr int kEvenSweeps = 4;        // rows per thread, at most
+constexpr int kEvenLds = 156 * 1024;  // dynamic LDS of the launch (the static part is below 1 KB)
+constexpr int kEvenDepth = 4;         // streamed blocks under way
+constexpr int kEvenE = 12;            // rows of the coarse inverse a thread reads ahead
+constexpr int kEvenGroups = 16;       // row groups of the coarse product, at most
+
+__host__ __device__ constexpr int even_up(int n) { return (n + 1) & ~1; }
+
+// Where a problem's data lie in LDS (floats) and how its blocks are held.
+struct EvenShape {
+  int K, KL, KS;              // blocks per thread; in LDS; streamed
+  int rw, cd, bi, p, r, x, part, tier;
+  bool fits;
+};
+__host__ __device__ inline EvenShape even_shape(int rows, int nblk, bool kc, int scratch) {
+  EvenShape s;
+  s.K = nblk > 0 ? (nblk + kEvenNT - 1) / kEvenNT : 1;
+  s.rw = scratch;
+  s.cd = s.rw + even_up(rows + 1);
+  s.bi = s.cd + (kc ? even_up(3 * rows) : 0);
+  s.p = s.bi + 6 * rows;
+  s.r = s.p + even_up(3 * rows);
+  s.x = s.r + even_up(3 * rows);
+  s.part = s.x + even_up(3 * rows);
+  // FP64 partials start at r
+  const int end32 = s.part + 3 * (rows + kEvenNT), end64 = s.r + 6 * (rows + kEvenNT);
+  const int endc = kc ? s.part + 2 * 4 * kEvenNT : 0;  // four FP64 columns per thread of the coarse product
+  int end = end32 > end64 ? end32 : end64;
+  end = end > endc ? end : endc;
+  s.tier = (end + 3) / 4 * 4;
+  const int room = kEvenLds / 4 - s.tier, rest = s.K > kEvenKR ? s.K - kEvenKR : 0;
+  s.fits = room >= 0 && rows <= kEvenSweeps * kEvenNT;
+  s.KL = rest < kEvenMaxKL ? rest : kEvenMaxKL;
+  if (s.KL > room / (9 * kEvenNT)) s.KL = room < 0 ? 0 : room / (9 * kEvenNT);
+  s.KS = rest - s.KL;
+  return s;
+}
+
+struct EvenArgs {
+  const int32_t* order;   // [P] problems by descending block count
+  const int64_t* slot0;   // [P] first slot of each problem (a multiple of kEvenNT)
+  const float* vals;      // the dealt blocks
+  const uint16_t* word;   // [slots] 12 column | (1: the row's last block); 0 where a thread has no block
+  const int32_t* bptr;    // the mesh's block rows
+  const int32_t* wrow;    // slot of each vertex's inverse in the sliced layout
+  int scratch;            // floats of the coarse scratch, at the start of the dynamic LDS
+};
+
+// Slot of every block (pos) and the word of every slot.
+__global__ void even_map_kernel(int64_t nblk, const int32_t* brow, const int32_t* bcol, const int32_t* bptr,
+                                const int32_t* pid, const int32_t* vstart, const int64_t* slot0, int32_t* pos,
+                                uint16_t* word) {
+  const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nblk) return;
+  const int32_t v = brow[b], p = pid[v], v0 = vstart[p], b0 = bptr[v0], n = bptr[vstart[p + 1]] - b0;
+  const int32_t K = (n + kEvenNT - 1) / kEvenNT, l = (int32_t)b - b0;
+  const int64_t q = slot0[p] + (int64_t)(l % K) * kEvenNT + l / K;
+  pos[b] = (int32_t)q;
+  word[q] = (uint16_t)(12 * (bcol[b] - v0) + (b + 1 == bptr[v + 1] ? 1 : 0));
+}
+
+// Totals of NV values in every thread; one barrier (two buffers take turns).
+template <int NV>
+__device__ __forceinline__ void even_sum(double (&v)[NV], double (*lds)[2 * (kEvenNT / kWave)], int& turn) {
+  constexpr int nw = kEvenNT / kWave;
+  double* b = lds[turn ^= 1];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const double s = wave_sum_last(v[k]);
+    if (threadIdx.x % kWave == kWave - 1) b[k * nw + threadIdx.x / kWave] = s;
+  }
+  lds_barrier();
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < nw; ++w) s += b[k * nw + w];
+    v[k] = s;
+  }
+}
+
+template <bool KC>
+__global__ __launch_bounds__(kEvenNT) void batch_pcg_even_kernel(BatchArgs a, EvenArgs ev) {
+  constexpr int NT = kEvenNT, KR = kEvenKR, nw = NT / kWave, SW = kEvenSweeps;
+  extern __shared__ double dyn_d[];
+  __shared__ double s_sum[2][2 * nw];
+  float* dyn = reinterpret_cast<float*>(dyn_d);
+  const int p = ev.order[blockIdx.x];
+  if (!block_read(a.active + p)) return;
+  const int t = threadIdx.x, lane = t % kWave, wid = t / kWave;
+  const int64_t v0 = a.vstart[p];
+  const int R = (int)(a.vstart[p + 1] - v0);
+  const int b0 = ev.bptr[v0], nbk = ev.bptr[v0 + R] - b0;
+  const EvenShape sh = even_shape(R, nbk, KC, ev.scratch);
+  const int K = sh.K, KL = sh.KL, KS = sh.KS;
+  int32_t* RW = reinterpret_cast<int32_t*>(dyn + sh.rw);  // [R + 1] first block of each row
+  float *CD = dyn + sh.cd, *BI = dyn + sh.bi, *P = dyn + sh.p, *Rv = dyn + sh.r, *X = dyn + sh.x;
+  float* part32 = dyn + sh.part;
+  double* part64 = reinterpret_cast<double*>(dyn + sh.r);
+  float* L = dyn + sh.tier;
+  const int64_t q0 = ev.slot0[p];
+  const float* V0 = ev.vals + 9 * q0;
+  const uint16_t* W0 = ev.word + q0;
+  CoarseLds cl{};
+  if (KC) cl = coarse_lds(dyn, a);
+  int nagg = 0, g0 = 0, cb = 0, nc = 0;
+  for (int i = t; i <= R; i += NT) RW[i] = ev.bptr[v0 + i] - b0;
+  if (KC) {
+    g0 = a.cagg0[p];
+    nagg = a.cagg0[p + 1] - g0;
+    cb = a.ccol[g0];
+    nc = a.ccol[g0 + nagg] - cb;
+    for (int i = t; i < nagg * (a.agg_rows / kWave) * 6; i += NT) cl.raw[i] = 0.f;
+    for (int i = t; i < 3 * R; i += NT) CD[i] = a.cdv[3 * v0 + i];
+  }
+  __syncthreads();
+
+  // the thread's blocks
+  float A[KR][9];
+  uint32_t meta[(KR + kEvenMaxKL + 1) / 2];
+#pragma unroll
+  for (int k = 0; k < (KR + kEvenMaxKL + 1) / 2; ++k) meta[k] = 0;
+  auto load_block = [&](int k, int th, float (&B)[9]) -> uint32_t {
+    load_slot<float, kQuadC, kQuadVW>(V0, k * NT + (th & ~(kWave - 1)), th & (kWave - 1), B);
+    return W0[k * NT + th];
+  };
+  auto word = [&](int k) { return (meta[k / 2] >> (16 * (k & 1))) & 0xffffu; };
+#pragma unroll
+  for (int k = 0; k < KR; ++k) {
+#pragma unroll
+    for (int m = 0; m < 9; ++m) A[k][m] = 0.f;
+    if (k < K) meta[k / 2] |= load_block(k, t, A[k]) << (16 * (k & 1));
+  }
+#pragma unroll
+  for (int k = 0; k < kEvenMaxKL; ++k)
+    if (k < KL) {
+      float B[9];
+      meta[(KR + k) / 2] |= load_block(KR + k, t, B) << (16 * ((KR + k) & 1));
+#pragma unroll
+      for (int m = 0; m < 9; ++m) L[(k * 9 + m) * NT + t] = B[m];
+    }
+  int row;  // of the thread's first block: the last one that starts at or before it
+  {
+    int lo = 0, hi = R;
+    while (hi - lo > 1) {
+      const int m = (lo + hi) / 2;
+      if (RW[m] <= t * K) lo = m;
+      else hi = m;
+    }
+    row = t * K < nbk ? lo : R;
+  }
+  const int slot0 = row + t;
+
+  // A src as partials (src: LDS in FP32 or the global FP64 correction)
+  auto product = [&](const auto* __restrict__ src, auto* __restrict__ part) {
+    using V = std::remove_cv_t<std::remove_reference_t<decltype(src[0])>>;
+#pragma unroll
+    for (int k = 0; k < (KR + kEvenMaxKL + 1) / 2; ++k) meta[k] = (uint32_t)opaque((int)meta[k]);
+    const int tt = opaque(t);
+    V y0 = 0, y1 = 0, y2 = 0;
+    V* o = part + 3 * slot0;
+    auto read = [&](uint32_t w, V (&s)[3]) {
+      const V* q = reinterpret_cast<const V*>(reinterpret_cast<const char*>(src) + (w & ~3u) * (sizeof(V) / 4));
+      s[0] = q[0];
+      s[1] = q[1];
+      s[2] = q[2];
+    };
+    auto add = [&](const float (&B)[9], const V (&s)[3], uint32_t w) {
+      y0 = fma((V)B[2], s[2], fma((V)B[1], s[1], fma((V)B[0], s[0], y0)));
+      y1 = fma((V)B[5], s[2], fma((V)B[4], s[1], fma((V)B[3], s[0], y1)));
+      y2 = fma((V)B[8], s[2], fma((V)B[7], s[1], fma((V)B[6], s[0], y2)));
+      if (w & 1u) {
+        o[0] = y0;
+        o[1] = y1;
+        o[2] = y2;
+        o += 3;
+        y0 = y1 = y2 = V(0);
+      }
+    };
+    constexpr int D = kEvenDepth;
+    float u[D][9];
+    uint32_t uw[D];
+    auto fetch = [&](int d, int k) {
+      if (k < KS) uw[d] = load_block(KR + KL + k, tt, u[d]);
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) fetch(d, d);
+    constexpr int U = 2;
+    V s[2][U][3];
+#pragma unroll
+    for (int k = 0; k < U; ++k) read(word(k), s[0][k]);
+#pragma unroll
+    for (int k = 0; k < KR; k += U) {
+      if (k < K) {
+#pragma unroll
+        for (int h = 0; h < U; ++h)
+          if (k + U + h < KR) read(word(k + U + h), s[(k / U + 1) & 1][h]);
+#pragma unroll
+        for (int h = 0; h < U; ++h) add(A[k + h], s[(k / U) & 1][h], word(k + h));
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < kEvenMaxKL; ++k)
+      if (k < KL) {
+        float B[9];
+        V q[3];
+        read(word(KR + k), q);
+#pragma unroll
+        for (int m = 0; m < 9; ++m) B[m] = L[(k * 9 + m) * NT + tt];
+        add(B, q, word(KR + k));
+      }
+    for (int k0 = 0; k0 < KS; k0 += D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d)
+        if (k0 + d < KS) {
+          V q[3];
+          read(uw[d], q);
+          add(u[d], q, uw[d]);
+          fetch(d, k0 + d + D);
+        }
+    }
+    o[0] = y0;  // the open row's partial (or a slot that no row reads)
+    o[1] = y1;
+    o[2] = y2;
+  };
+
+  // the thread's rows: slots of the partials (first | last << 16) and fixed DOFs; B^-1 goes to LDS
+  uint32_t span[SW];
+  int fx[SW];
+#pragma unroll
+  for (int s = 0; s < SW; ++s) {
+    const int r = s * NT + t;
+    span[s] = 0;
+    fx[s] = 7;
+    if (r < R) {
+      span[s] = (uint32_t)(r + RW[r] / K) | (uint32_t)(r + (RW[r + 1] - 1) / K) << 16;
+      const int64_t k = 3 * (v0 + r);
+      fx[s] = a.fixed ? (a.fixed[k] ? 1 : 0) | (a.fixed[k + 1] ? 2 : 0) | (a.fixed[k + 2] ? 4 : 0) : 0;
+      const int w = ev.wrow[v0 + r];
+      float B[9];
+      load_slot<float, kQuadC, kQuadVW>(a.binv, w & ~(kQuadC - 1), w & (kQuadC - 1), B);
+#pragma unroll
+      for (int m = 0; m < 6; ++m) BI[6 * r + m] = B[3 * kBinvPQ[m][0] + kBinvPQ[m][1]];
+    }
+  }
+  auto row_sum = [&](const auto* __restrict__ part, int s, auto (&y)[3]) {
+    const uint32_t sp = (uint32_t)opaque((int)span[s]);
+    const int s0 = (int)(sp & 0xffffu), s1 = (int)(sp >> 16);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) y[q] = part[3 * s0 + q];
+    for (int k = s0 + 1; k <= s1; ++k)
+#pragma unroll
+      for (int q = 0; q < 3; ++q) y[q] += part[3 * k + q];
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if ((fx[s] >> q) & 1) y[q] = 0;
+  };
+  auto precondition = [&](int i, const float (&r)[3], float (&z)[3]) {
+    const float* B = BI + 6 * i;
+    z[0] = B[0] * r[0] + B[1] * r[1] + B[2] * r[2];
+    z[1] = B[1] * r[0] + B[3] * r[1] + B[4] * r[2];
+    z[2] = B[2] * r[0] + B[4] * r[1] + B[5] * r[2];
+  };
+  // the wave's share of W^T r for sweep s
+  auto restrict_rows = [&](int s, const float (&r)[3], bool has) {
+    float v[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const int row0 = s * NT + wid * kWave, l = row0 / a.agg_rows;
+    if (l >= nagg) return;  // the same for the whole wave
+    if (has) restrict_terms(CD + 3 * (s * NT + opaque(t)), r, v);
+    const int at = (l * (a.agg_rows / kWave) + row0 % a.agg_rows / kWave) * 6;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      const float w = wave_sum_last(v[q]);
+      if (lane == kWave - 1) cl.raw[at + q] = w;
+    }
+  };
+  // the thread's coarse unknown (aggregate ag, motion am), its basis column and row
+  const int ag = t / 6, am = t % 6;
+  float tcol[6], trow[6];
+  int c0 = 0, ck = 0;
+#pragma unroll
+  for (int q = 0; q < 6; ++q) tcol[q] = trow[q] = 0.f;
+  if (KC && ag < nagg) {
+    c0 = a.ccol[g0 + ag] - cb;
+    ck = a.ccol[g0 + ag + 1] - a.ccol[g0 + ag];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) {
+      tcol[q] = a.ctm[36 * (int64_t)(g0 + ag) + 6 * q + am];
+      trow[q] = a.ctm[36 * (int64_t)(g0 + ag) + 6 * am + q];
+    }
+  }
+  int turn = 0;
+  // E^-1 (symmetric, rows nc apart): the thread's four columns and its rows ej, ej + groups, ...
+  const int n4 = (nc + 3) / 4, groups = KC && n4 ? (NT / n4 < kEvenGroups ? NT / n4 : kEvenGroups) : 1;
+  const int ei0 = KC && n4 ? t % n4 : 0, ej0 = KC && n4 && t / n4 < groups ? t / n4 : nc;
+  const float* Einv = KC ? a.einv + a.einv_off[p] : nullptr;
+  typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+  f4u e[kEvenE];
+  auto fetch_coarse = [&]() {
+    const int j0 = opaque(ej0);
+    const float* E = Einv + 4 * opaque(ei0);
+#pragma unroll
+    for (int u = 0; u < kEvenE; ++u) {
+      const int j = j0 + u * groups;
+      e[u] = f4u{0.f, 0.f, 0.f, 0.f};
+      if (j < nc) e[u] = *reinterpret_cast<const f4u*>(E + j * nc);
+    }
+  };
+  // From the waves' shares (before the preceding barrier): y = E^-1 W^T r, the rigid motions; returns c.y.
+  // The partials' LDS holds the row groups' shares of E^-1 c.
+  auto coarse = [&]() -> double {
+    const int t = opaque(threadIdx.x), ej = opaque(ej0), ei = opaque(ei0);
+    if (ag < nagg && am < ck) {
+      const int slots = a.agg_rows / kWave;
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        float rq = 0.f;
+        for (int w = 0; w < slots; ++w) rq += cl.raw[(ag * slots + w) * 6 + q];
+        s += (double)tcol[q] * (double)rq;
+      }
+      cl.c[c0 + am] = s;
+    }
+    lds_barrier();
+    const float* E = Einv + 4 * ei;
+    double* red = reinterpret_cast<double*>(part32);
+    double y[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add_row = [&](const f4u& x, double c) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) y[m] += (double)x[m] * c;
+    };
+#pragma unroll
+    for (int u = 0; u < kEvenE; ++u) {
+      const int j = ej + u * groups;
+      add_row(e[u], cl.c[j < nc ? j : 0]);  // e is 0 past the last row
+    }
+    for (int j = ej + kEvenE * groups; j < nc; j += groups) add_row(*reinterpret_cast<const f4u*>(E + j * nc), cl.c[j]);
+    if (ej < nc) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) red[(ej * n4 + ei) * 4 + m] = y[m];
+    }
+    lds_barrier();
+    double cy[1] = {0.0};
+    if (t < nc) {
+      const int rows = groups < nc ? groups : nc;
+      double s = 0.0;
+#pragma unroll 4
+      for (int w = 0; w < rows; ++w) s += red[w * 4 * n4 + t];
+      cl.y[t] = s;
+      cy[0] = cl.c[t] * s;
+    }
+    lds_barrier();
+    if (ag < nagg) {
+      double s = 0.0;
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+        if (q < ck) s += (double)trow[q] * cl.y[c0 + q];
+      cl.uw[t] = s;
+    }
+    even_sum<1>(cy, s_sum, turn);  // its barrier also publishes uw
+    return cy[0];
+  };
+  // P = z + coarse part + beta P
+  auto direction = [&](float beta, bool first) {
+#pragma unroll
+    for (int s = 0; s < SW; ++s) {
+      const int r = s * NT + opaque(t);
+      if (r < R) {
+        float z[3], zc[3] = {0.f, 0.f, 0.f};
+        const float rv[3] = {Rv[3 * r], Rv[3 * r + 1], Rv[3 * r + 2]};
+        precondition(r, rv, z);
+        if (KC) coarse_term(a, cl, CD + 3 * r, r, fx[s], zc);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) P[3 * r + q] = first ? z[q] + zc[q] : z[q] + zc[q] + beta * P[3 * r + q];
+      }
+    }
+    lds_barrier();
+  };
+  const double* g = a.g + 3 * v0;
+  double* dx = a.dx + 3 * v0;
+
+  // x = 0, r = b = -g (free), z, p = M^-1 r
+  double acc[2] = {0.0, 0.0};
+  if (KC) fetch_coarse();
+#pragma unroll
+  for (int s = 0; s < SW; ++s) {
+    const int i = s * NT + t;
+    float r[3] = {0.f, 0.f, 0.f};
+    if (i < R) {
+      float z[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const double b = ((fx[s] >> q) & 1) ? 0.0 : -g[3 * i + q];
+        dx[3 * i + q] = 0.0;
+        r[q] = (float)b;
+        Rv[3 * i + q] = r[q];
+        X[3 * i + q] = 0.f;
+        acc[1] += b * b;
+      }
+      precondition(i, r, z);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        acc[0] += (double)r[q] * (double)z[q];
+      }
+    }
+    if (KC) restrict_rows(s, r, i < R);
+  }
+  even_sum<2>(acc, s_sum, turn);
+  double rz = acc[0];
+  const double bb = acc[1];
+  if (KC) rz += coarse();
+  direction(0.f, true);
+  const double target = a.pcg_rtol2 * bb;
+  double seg_rr = bb;
+  int it = 0, refines = 0, st = SK_OK;
+  bool done = !(bb > 0.0);
+  if (!isfinite(bb)) {
+    st = SK_ERR_NONFINITE;
+    done = true;
+  }
+  while (!done && it < a.pcg_max_iter) {
+    product(P, part32);
+    lds_barrier();
+    double d1[1] = {0.0};
+    float ap[SW][3];
+#pragma unroll
+    for (int s = 0; s < SW; ++s) {
+      const int i = s * NT + opaque(t);
+      if (i < R) {
+        row_sum(part32, s, ap[s]);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) d1[0] += (double)P[3 * i + q] * (double)ap[s][q];
+      }
+    }
+    even_sum<1>(d1, s_sum, turn);
+    const double pAp = d1[0];
+    if (!(pAp > 0.0)) {
+      st = isfinite(pAp) ? SK_ERR_PCG_BREAKDOWN : SK_ERR_NONFINITE;
+      break;
+    }
+    const float alpha = (float)(rz / pAp);
+    double d2[2] = {0.0, 0.0};
+    if (KC) fetch_coarse();
+#pragma unroll
+    for (int s = 0; s < SW; ++s) {
+      const int i = s * NT + opaque(t);
+      float r[3] = {0.f, 0.f, 0.f};
+      if (i < R) {
+        float z[3];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          X[3 * i + q] += alpha * P[3 * i + q];
+          r[q] = Rv[3 * i + q] - alpha * ap[s][q];
+          Rv[3 * i + q] = r[q];
+          d2[0] += (double)r[q] * (double)r[q];
+        }
+        precondition(i, r, z);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          d2[1] += (double)r[q] * (double)z[q];
+        }
+      }
+      if (KC) restrict_rows(s, r, i < R);
+    }
+    even_sum<2>(d2, s_sum, turn);
+    ++it;
+    if (!isfinite(d2[0])) {
+      st = SK_ERR_NONFINITE;
+      break;
+    }
+    if (d2[0] <= a.inner_rtol2 * seg_rr || d2[0] <= target) {
+      // residual replacement: dx += x (FP64), r = b - A dx, x = 0
+#pragma unroll
+      for (int s = 0; s < SW; ++s) {
+        const int i = s * NT + opaque(t);
+        if (i < R) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) dx[3 * i + q] += (double)X[3 * i + q];
+        }
+      }
+      __syncthreads();  // dx is in memory, and x has been read
+      product(const_cast<const double*>(dx), part64);
+      lds_barrier();
+      double y[SW][3];
+#pragma unroll
+      for (int s = 0; s < SW; ++s)
+        if (s * NT + opaque(t) < R) row_sum(part64, s, y[s]);
+      lds_barrier();  // before r and x are written over the partials
+      double d3[2] = {0.0, 0.0};
+      if (KC) fetch_coarse();
+#pragma unroll
+      for (int s = 0; s < SW; ++s) {
+        const int i = s * NT + opaque(t);
+        float r[3] = {0.f, 0.f, 0.f};
+        if (i < R) {
+          float z[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const double e = ((fx[s] >> q) & 1) ? 0.0 : -g[3 * i + q] - y[s][q];
+            r[q] = (float)e;
+            Rv[3 * i + q] = r[q];
+            X[3 * i + q] = 0.f;
+            d3[0] += e * e;
+          }
+          precondition(i, r, z);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            d3[1] += (double)r[q] * (double)z[q];
+          }
+        }
+        if (KC) restrict_rows(s, r, i < R);
+      }
+      even_sum<2>(d3, s_sum, turn);
+      ++refines;
+      if (d3[0] <= target) break;
+      seg_rr = d3[0];
+      d2[1] = d3[1];
+    }
+    const double rz_new = d2[1] + (KC ? coarse() : 0.0);
+    const float beta = (float)(rz_new / rz);
+    rz = rz_new;
+    direction(beta, false);
+  }
+  if (it >= a.pcg_max_iter && st == SK_OK) {
+    // iteration limit: the FP64 correction so far is used as the direction
+#pragma unroll
+    for (int s = 0; s < SW; ++s) {
+      const int i = s * NT + opaque(t);
+      if (i < R) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) dx[3 * i + q] += (double)X[3 * i + q];
+      }
+    }
+  }
+  if (t == 0 && a.count_pcg) {
+    a.pcg_iters[p] += it;
+    a.refines[p] += refines;
+    if (st != SK_OK) {
+      a.status[p] = st;
+      a.active[p] = 0;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Per-problem Armijo line search in difference form:
 //   dE(t) = sum_e vol (psi(x + t dx) - psi(x)) + sum_free [c/(2h^2) m ((x1-xt)^2 - (x0-xt)^2) - f (x1 - x0)]
 // accepted at the first t in {1, beta, beta^2, ...} with dE <= alpha t g.dx + threshold.
@@ -898,6 +1471,12 @@ struct sk_batch {
   DevBuf<int64_t> einv_off;
   DevBuf<double> cE;
   DevBuf<int> cbad;
+  // the evenly dealt PCG (batch_pcg_even_kernel): 1 in use, 0 not (yet looked for: -1)
+  int even = -1;
+  DevBuf<int32_t> even_order, even_pos;
+  DevBuf<int64_t> even_slot0;
+  DevBuf<uint16_t> even_word;
+  DevBuf<float> even_vals;
   bool coarse() const { return agg_rows > 0; }
   BatchArgs args() const;
 };
@@ -982,6 +1561,57 @@ size_t pcg_lds_bytes(const sk_batch* B) { return pcg_shm_bytes(B, 1); }
 // 1024 threads), within the 160 KiB a workgroup may use.
 bool pcg_lds_fits(const sk_batch* B) { return B->max_rows > 0 && pcg_lds_bytes(B) <= 150 * 1024; }
 
+// Floats of the coarse scratch.
+int coarse_scratch(const sk_batch* B) {
+  return B->coarse() ? coarse_raw_floats(B->max_agg, B->agg_rows) + 2 * (2 * B->max_nc + 6 * B->max_agg) : 0;
+}
+// Whether a launch shape runs the evenly dealt PCG: whenever it fits. It holds a CU to one workgroup, yet was the
+// faster one at every size tried (a step, lane per row against dealt evenly): 512 beams of 8 to 64 cells block-Jacobi
+// 77.1 / 44.0 ms, of 36 to 46 two-level 20.5 / 14.1, of 16 to 24 13.0 / 8.7, of 4 to 10 7.0 / 5.3, 64 beams of 4 to
+// 10 3.6 / 2.4, 2,048 of 4 to 10 20.7 / 16.2.
+bool pcg_even(const sk_batch* B, int block, int lanes, int lds) {
+  return B->even == 1 && block == kEvenNT && lanes == 1 && lds;
+}
+// Before the first launch (and never within a captured one): decides whether
+// the evenly dealt PCG can serve the batch and allocates what it streams.
+int prepare_even(sk_batch* B) {
+  if (B->even >= 0) return SK_OK;
+  B->even = 0;
+  if (!pcg_lds_fits(B)) return SK_OK;
+  std::vector<int32_t> vs(B->P + 1), order(B->P);
+  SK_HIP_CHECK(hipMemcpy(vs.data(), B->vstart.p, vs.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+  const std::vector<int32_t>& bptr = B->mesh->h_bptr;
+  auto blocks = [&](int q) { return bptr[vs[q + 1]] - bptr[vs[q]]; };
+  std::vector<int64_t> slot0(B->P);
+  int64_t slots = 0;
+  for (int q = 0; q < B->P; ++q) {
+    const EvenShape s = even_shape(vs[q + 1] - vs[q], blocks(q), B->coarse(), coarse_scratch(B));
+    if (!s.fits) return SK_OK;
+    slot0[q] = slots;
+    slots += (int64_t)s.K * kEvenNT;
+    order[q] = q;
+  }
+  if (slots > INT32_MAX) return SK_OK;
+  std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blocks(x) > blocks(y); });
+  const sk_mesh* m = B->mesh;
+  if (B->even_vals.alloc(9 * slots) || B->even_word.alloc(slots) || B->even_pos.alloc(m->nblk) ||
+      B->even_order.upload(order) || B->even_slot0.upload(slot0)) {
+    (void)hipGetLastError();  // no memory for it: the lane-per-row kernel needs none
+    for (DevBuf<int32_t>* b : {&B->even_order, &B->even_pos}) b->release();
+    B->even_vals.release();
+    B->even_word.release();
+    B->even_slot0.release();
+    return SK_OK;
+  }
+  SK_HIP_CHECK(hipMemsetAsync(B->even_vals.p, 0, B->even_vals.n * sizeof(float), B->st));  // slots without a block
+  SK_HIP_CHECK(hipMemsetAsync(B->even_word.p, 0, B->even_word.n * sizeof(uint16_t), B->st));
+  even_map_kernel<<<grid_for(m->nblk), kBlock, 0, B->st>>>(m->nblk, m->brow.p, m->bcol.p, m->bptr.p, B->pid.p,
+                                                           B->vstart.p, B->even_slot0.p, B->even_pos.p, B->even_word.p);
+  SK_HIP_CHECK(hipGetLastError());
+  B->even = 1;
+  return SK_OK;
+}
+
 int launch_pcg(const sk_batch* B, const BatchArgs& a, int block, int lanes, int lds) {
   const int g = B->grid;
   const size_t shm = pcg_shm_bytes(B, lds);
@@ -990,6 +1620,14 @@ int launch_pcg(const sk_batch* B, const BatchArgs& a, int block, int lanes, int 
   BatchArgs a2 = a;
   a2.vec_floats = pcg_vec_floats(B, lds);
   const bool kc = B->coarse();
+  if (pcg_even(B, block, lanes, lds)) {
+    a2.vec_floats = 0;
+    const EvenArgs ev{B->even_order.p, B->even_slot0.p, B->even_vals.p, B->even_word.p,
+                      B->mesh->bptr.p, B->wrow.p, coarse_scratch(B)};
+    if (kc) batch_pcg_even_kernel<true><<<B->P, kEvenNT, kEvenLds, B->st>>>(a2, ev);
+    else batch_pcg_even_kernel<false><<<B->P, kEvenNT, kEvenLds, B->st>>>(a2, ev);
+    return SK_OK;
+  }
 #define SK_PCG_CASE(NT, L)                                                         \
   if (block == NT && lanes == L) {                                                 \
     if (kc) {                                                                      \
@@ -1033,7 +1671,8 @@ struct GalerkinBatchArgs {
   const int32_t* vstart;
   const int32_t* bptr;
   const int32_t* bcol;
-  const int32_t* wpos;     // slot of each block in the sliced FP32 values
+  const int32_t* brow;
+  const int32_t* wpos;     // slot of each block in the FP32 values
   const float* vals;
   const uint8_t* fixed;
   const float* cdv;
@@ -1063,13 +1702,19 @@ __device__ __forceinline__ void rigid_row_f(const float* d, int p, double (&out)
 
 // Workgroup g (aggregate): E_q blocks (g, J) = T_g^T (sum over blocks (v, w),
 // v in g, w in J, of R_v^T M_v A_vw M_w R_w) T_J for every adjacent J, with
-// fixed-order block sums.
+// fixed-order block sums. Threads take the aggregate's blocks in turn, and 36 of
+// them an entry of the result each: with a thread per row (64 of 256 at work) and
+// one thread for all 36 entries the 512-beam batch (7,900 aggregates) took 2,970
+// us, this way 534 us.
 __global__ __launch_bounds__(kBlock) void batch_galerkin_kernel(GalerkinBatchArgs a) {
-  __shared__ double lds[36 * kBlock / kWave];
-  const int g = blockIdx.x, q = a.cagg_prob[g];
+  constexpr int nw = kBlock / kWave;
+  __shared__ double s_wave[36][nw], s_acc[36];
+  __shared__ float s_t[2][36];  // T_g, T_J
+  const int g = blockIdx.x, q = a.cagg_prob[g], t = threadIdx.x;
   const int64_t v0 = a.vstart[q], v1 = a.vstart[q + 1];
   const int g0 = a.cagg0[q], l = g - g0;
   const int64_t r0 = v0 + (int64_t)l * a.agg_rows, r1 = std::min<int64_t>(v1, r0 + a.agg_rows);
+  const int32_t b0 = a.bptr[r0], b1 = a.bptr[r1];
   const int cb = a.ccol[g0], nq = a.cnq[q];
   const int cI = a.ccol[g] - cb, kI = a.ccol[g + 1] - a.ccol[g];
   for (int jj = a.cadj_ptr[g]; jj < a.cadj_ptr[g + 1]; ++jj) {
@@ -1078,83 +1723,157 @@ __global__ __launch_bounds__(kBlock) void batch_galerkin_kernel(GalerkinBatchArg
     double acc[36];
 #pragma unroll
     for (int k = 0; k < 36; ++k) acc[k] = 0.0;
-    for (int64_t v = r0 + threadIdx.x; v < r1; v += blockDim.x) {
-      for (int32_t b = a.bptr[v]; b < a.bptr[v + 1]; ++b) {
-        const int64_t w = a.bcol[b];
-        if (g0 + (int)((w - v0) / a.agg_rows) != J) continue;
-        double A[9];
-        const int64_t q = a.wpos[b];
+    for (int32_t b = b0 + t; b < b1; b += kBlock) {
+      const int64_t v = a.brow[b], w = a.bcol[b];
+      if (g0 + (int)((w - v0) / a.agg_rows) != J) continue;
+      double A[9];
+      const int64_t q = a.wpos[b];
 #pragma unroll
-        for (int m = 0; m < 9; ++m) {
-          const bool fr = !(a.fixed && (a.fixed[3 * v + m / 3] || a.fixed[3 * w + m % 3]));
-          A[m] = fr ? (double)a.vals[slot_index<kQuadC, kQuadVW>(q, m)] : 0.0;
-        }
-        double Rw[3][6], AR[3][6];
+      for (int m = 0; m < 9; ++m) {
+        const bool fr = !(a.fixed && (a.fixed[3 * v + m / 3] || a.fixed[3 * w + m % 3]));
+        A[m] = fr ? (double)a.vals[slot_index<kQuadC, kQuadVW>(q, m)] : 0.0;
+      }
+      double Rw[3][6], AR[3][6];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) rigid_row_f(a.cdv + 3 * w, p, Rw[p]);
+      for (int p = 0; p < 3; ++p) rigid_row_f(a.cdv + 3 * w, p, Rw[p]);
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
+      for (int p = 0; p < 3; ++p)
 #pragma unroll
-          for (int c = 0; c < 6; ++c) AR[p][c] = A[3 * p] * Rw[0][c] + A[3 * p + 1] * Rw[1][c] + A[3 * p + 2] * Rw[2][c];
+        for (int c = 0; c < 6; ++c) AR[p][c] = A[3 * p] * Rw[0][c] + A[3 * p + 1] * Rw[1][c] + A[3 * p + 2] * Rw[2][c];
 #pragma unroll
-        for (int p = 0; p < 3; ++p) {
-          double Rv[6];
-          rigid_row_f(a.cdv + 3 * v, p, Rv);
+      for (int p = 0; p < 3; ++p) {
+        double Rv[6];
+        rigid_row_f(a.cdv + 3 * v, p, Rv);
 #pragma unroll
-          for (int r = 0; r < 6; ++r)
+        for (int r = 0; r < 6; ++r)
 #pragma unroll
-            for (int c = 0; c < 6; ++c) acc[6 * r + c] += Rv[r] * AR[p][c];
-        }
+          for (int c = 0; c < 6; ++c) acc[6 * r + c] += Rv[r] * AR[p][c];
       }
     }
-    block_sum<36>(acc, lds);
-    if (threadIdx.x == 0) {
-      const float* TI = a.ctm + 36 * (int64_t)g;
-      const float* TJ = a.ctm + 36 * (int64_t)J;
-      double* E = a.E + a.einv_off[q];
-      for (int j = 0; j < kI; ++j)
-        for (int m = 0; m < kJ; ++m) {
-          double s = 0.0;
-          for (int r = 0; r < 6; ++r)
-            for (int c = 0; c < 6; ++c) s += (double)TI[6 * r + j] * acc[6 * r + c] * (double)TJ[6 * c + m];
-          E[(int64_t)(cI + j) * nq + cJ + m] = s;
-        }
+#pragma unroll
+    for (int k = 0; k < 36; ++k) {
+      const double w = wave_sum_last(acc[k]);
+      if (t % kWave == kWave - 1) s_wave[k][t / kWave] = w;
+    }
+    if (t < 72) s_t[t / 36][t % 36] = a.ctm[36 * (int64_t)(t < 36 ? g : J) + t % 36];
+    __syncthreads();
+    if (t < 36) {
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < nw; ++w) s += s_wave[t][w];
+      s_acc[t] = s;
+    }
+    __syncthreads();
+    if (t < 36 && t / 6 < kI && t % 6 < kJ) {
+      const int j = t / 6, m = t % 6;
+      double s = 0.0;
+#pragma unroll
+      for (int r = 0; r < 6; ++r)
+#pragma unroll
+        for (int c = 0; c < 6; ++c) s += (double)s_t[0][6 * r + j] * s_acc[6 * r + c] * (double)s_t[1][6 * c + m];
+      a.E[a.einv_off[q] + (int64_t)(cI + j) * nq + cJ + m] = s;
     }
     __syncthreads();
   }
 }
 
-// Workgroup q: Gauss-Jordan inversion of E_q in place (symmetric positive
-// definite, no pivoting), then E_q^-1 symmetrised into FP32. A non-positive
-// or non-finite pivot sets bad[q] and stops that problem's elimination.
-constexpr int kGjBlock = 1024;
+// Workgroup q: Gauss-Jordan inversion of E_q (symmetric positive definite, no
+// pivoting), then E_q^-1 symmetrised into FP32. A non-positive or non-finite
+// pivot sets bad[q] and stops that problem's elimination.
+//
+// Up to kGjReg unknowns the matrix stays in registers: thread (ti, tj) of a 32 x
+// 32 grid holds the entries (ti + 32 a, tj + 32 b), and a step passes the pivot's
+// row and column through LDS (two buffers take turns: one barrier per step).
+// Larger ones are eliminated in memory. In memory, with a division per entry and
+// step, the 512-beam batch (36 to 156 unknowns) took 3,240 us; in registers 302
+// us, bound by the barrier and LDS latency of the steps.
+constexpr int kGjBlock = 1024, kGjSide = 32, kGjTiles = 5, kGjReg = kGjSide * kGjTiles;
 
 __global__ __launch_bounds__(kGjBlock) void batch_gj_kernel(double* E, const int64_t* off, const int32_t* nq_arr,
                                                             float* einv, int* bad) {
+  __shared__ double s_row[2][kGjReg], s_col[2][kGjReg];
   __shared__ double s_piv;
   const int q = blockIdx.x, n = nq_arr[q];
   double* A = E + off[q];
-  for (int k = 0; k < n; ++k) {
-    if (threadIdx.x == 0) s_piv = A[(int64_t)k * n + k];
-    __syncthreads();
-    const double piv = s_piv;
-    if (!(piv > 0.0) || !isfinite(piv)) {
-      if (threadIdx.x == 0) bad[q] = 1;
-      return;  // uniform: every thread read the same pivot
-    }
-    for (int64_t idx = threadIdx.x; idx < (int64_t)n * n; idx += blockDim.x) {
-      const int i = (int)(idx / n), j = (int)(idx % n);
-      if (i != k && j != k) A[idx] -= A[(int64_t)i * n + k] * A[(int64_t)k * n + j] / piv;
-    }
-    __syncthreads();
-    for (int idx = threadIdx.x; idx < 2 * n; idx += blockDim.x) {
-      if (idx < n) {
-        A[(int64_t)k * n + idx] = (idx == k) ? 1.0 / piv : A[(int64_t)k * n + idx] / piv;
-      } else if (idx - n != k) {
-        A[(int64_t)(idx - n) * n + k] = -A[(int64_t)(idx - n) * n + k] / piv;
+  if (n <= kGjReg) {
+    const int ti = threadIdx.x / kGjSide, tj = threadIdx.x % kGjSide;
+    double M[kGjTiles][kGjTiles];
+#pragma unroll
+    for (int x = 0; x < kGjTiles; ++x)
+#pragma unroll
+      for (int y = 0; y < kGjTiles; ++y) {
+        const int i = ti + kGjSide * x, j = tj + kGjSide * y;
+        M[x][y] = i < n && j < n ? A[(int64_t)i * n + j] : 0.0;
       }
-    }
+#pragma unroll
+    for (int kb = 0; kb < kGjTiles; ++kb)
+      for (int kk = 0; kk < kGjSide; ++kk) {
+        const int k = kGjSide * kb + kk;
+        if (k >= n) break;
+        double *row = s_row[k & 1], *col = s_col[k & 1];
+        const bool mine_r = ti == kk, mine_c = tj == kk;
+        if (mine_r) {
+#pragma unroll
+          for (int y = 0; y < kGjTiles; ++y) row[tj + kGjSide * y] = M[kb][y];
+        }
+        if (mine_c) {
+#pragma unroll
+          for (int x = 0; x < kGjTiles; ++x) col[ti + kGjSide * x] = M[x][kb];
+        }
+        __syncthreads();
+        const double piv = row[k];
+        if (!(piv > 0.0) || !isfinite(piv)) {
+          if (threadIdx.x == 0) bad[q] = 1;
+          return;  // uniform: every thread read the same pivot
+        }
+        const double inv = 1.0 / piv;
+        double r[kGjTiles], c[kGjTiles];
+#pragma unroll
+        for (int y = 0; y < kGjTiles; ++y) {
+          r[y] = row[tj + kGjSide * y];
+          c[y] = col[ti + kGjSide * y] * inv;
+        }
+#pragma unroll
+        for (int x = 0; x < kGjTiles; ++x)
+#pragma unroll
+          for (int y = 0; y < kGjTiles; ++y) {
+            double m = M[x][y] - c[x] * r[y];
+            if (x == kb && mine_r) m = r[y] * inv;
+            if (y == kb && mine_c) m = x == kb && mine_r ? inv : -c[x];
+            M[x][y] = m;
+          }
+      }
+#pragma unroll
+    for (int x = 0; x < kGjTiles; ++x)
+#pragma unroll
+      for (int y = 0; y < kGjTiles; ++y) {
+        const int i = ti + kGjSide * x, j = tj + kGjSide * y;
+        if (i < n && j < n) A[(int64_t)i * n + j] = M[x][y];
+      }
     __syncthreads();
+  } else {
+    for (int k = 0; k < n; ++k) {
+      if (threadIdx.x == 0) s_piv = A[(int64_t)k * n + k];
+      __syncthreads();
+      const double piv = s_piv;
+      if (!(piv > 0.0) || !isfinite(piv)) {
+        if (threadIdx.x == 0) bad[q] = 1;
+        return;  // uniform: every thread read the same pivot
+      }
+      for (int64_t idx = threadIdx.x; idx < (int64_t)n * n; idx += blockDim.x) {
+        const int i = (int)(idx / n), j = (int)(idx % n);
+        if (i != k && j != k) A[idx] -= A[(int64_t)i * n + k] * A[(int64_t)k * n + j] / piv;
+      }
+      __syncthreads();
+      for (int idx = threadIdx.x; idx < 2 * n; idx += blockDim.x) {
+        if (idx < n) {
+          A[(int64_t)k * n + idx] = (idx == k) ? 1.0 / piv : A[(int64_t)k * n + idx] / piv;
+        } else if (idx - n != k) {
+          A[(int64_t)(idx - n) * n + k] = -A[(int64_t)(idx - n) * n + k] / piv;
+        }
+      }
+      __syncthreads();
+    }
   }
   for (int64_t idx = threadIdx.x; idx < (int64_t)n * n; idx += blockDim.x) {
     const int i = (int)(idx / n), j = (int)(idx % n);
@@ -1162,13 +1881,14 @@ __global__ __launch_bounds__(kGjBlock) void batch_gj_kernel(double* E, const int
   }
 }
 
-int hessian_phase(sk_batch* B, bool only_active);
+int hessian_phase(sk_batch* B, bool only_active, bool even);
 
 // Forms and inverts every problem's coarse operator from the system assembled
 // at the batch's current positions (synchronises the batch stream).
-int build_coarse(sk_batch* B) {
-  SK_TRY(hessian_phase(B, false));
-  GalerkinBatchArgs g{B->vstart.p, B->mesh->bptr.p, B->mesh->bcol.p, B->wpos.p, B->vals32.p, B->fixed.p,
+int build_coarse(sk_batch* B, bool even) {
+  SK_TRY(hessian_phase(B, false, even));
+  GalerkinBatchArgs g{B->vstart.p, B->mesh->bptr.p, B->mesh->bcol.p, B->mesh->brow.p, even ? B->even_pos.p : B->wpos.p,
+                      even ? B->even_vals.p : B->vals32.p, B->fixed.p,
                       B->cdv.p, B->ctm.p, B->cagg0.p, B->ccol.p, B->cagg_prob.p, B->cadj_ptr.p, B->cadj.p,
                       B->cnq.p, B->einv_off.p, B->cE.p, B->agg_rows};
   SK_HIP_CHECK(hipMemsetAsync(B->cE.p, 0, B->cE.n * sizeof(double), B->st));
@@ -1195,24 +1915,26 @@ int gradient_phase(sk_batch* B) {
                             1.0 / (B->prm.h * B->prm.h), B->st);
 }
 
-// Element Hessian + FP32 gather into the sliced layout. only_active: skip the elements and
+// Element Hessian + FP32 gather into the sliced layout, or with `even` into the
+// order of the evenly dealt PCG. only_active: skip the elements and
 // blocks of problems whose active flag (read on the device) is 0 (their
 // values are not read until they are assembled again); else every problem.
-int hessian_phase(sk_batch* B, bool only_active) {
+int hessian_phase(sk_batch* B, bool only_active, bool even) {
   sk_mesh* m = B->mesh;
   const int* act = only_active ? B->active.p : nullptr;
   const int32_t* pid = only_active ? B->pid.p : nullptr;
   SK_TRY(launch_elem_hess(m, B->prm.material, B->x.p, nullptr, B->mu.p, B->lam.p, B->vol.p, B->prm.psd, true,
                           B->st, act, pid, nullptr, true));
-  return launch_gather_hess_quad(m, B->vals32.p, B->mass.p, 1.0 / (B->prm.h * B->prm.h), B->fixed.p,
-                                 B->binv32.p, B->wpos.p, B->wrow.p, true, B->st, act, pid);
+  return launch_gather_hess_quad(m, even ? B->even_vals.p : B->vals32.p, B->mass.p, 1.0 / (B->prm.h * B->prm.h),
+                                 B->fixed.p, B->binv32.p, even ? B->even_pos.p : B->wpos.p, B->wrow.p, true, B->st,
+                                 act, pid);
 }
 
 // One Newton iteration of every active problem (no host synchronization).
 int newton_iteration(sk_batch* B, int block, int lanes, int lds) {
   const BatchArgs a = B->args();
   const int64_t n3 = 3 * B->mesh->nv;
-  SK_TRY(hessian_phase(B, true));
+  SK_TRY(hessian_phase(B, true, pcg_even(B, block, lanes, lds)));
   SK_TRY(launch_pcg(B, a, block, lanes, lds));
   SK_TRY(launch_ls(B, a, block));
   batch_update_kernel<<<grid_for(n3), kBlock, 0, B->st>>>(n3, a);
@@ -1437,9 +2159,10 @@ int sk_batch_step(sk_batch* B, const double* x_curr, const double* x_prev, const
   SK_HIP_CHECK(hipEventRecord(B->ev_in, caller));
   SK_HIP_CHECK(hipStreamWaitEvent(B->st, B->ev_in, 0));
   const int block = batch_block(B), lanes = batch_lanes(B), lds = batch_lds(B);
+  SK_TRY(prepare_even(B));
   SK_TRY(start_step(B, x_curr, x_prev, x_bc));
   if (B->coarse() && (!B->coarse_built || (B->coarse_period > 0 && B->steps_since_coarse >= B->coarse_period))) {
-    SK_TRY(build_coarse(B));
+    SK_TRY(build_coarse(B, pcg_even(B, block, lanes, lds)));
     B->steps_since_coarse = 0;
   }
   ++B->steps_since_coarse;
@@ -1496,6 +2219,7 @@ int sk_batch_set_coarse(sk_batch* B, const double* X, int agg_rows, int period) 
   B->graph = nullptr;
   B->agg_rows = B->n_agg = B->max_agg = B->max_nc = 0;
   B->coarse_built = false;
+  B->even = -1;  // the coarse scratch changes what fits
   for (DevBuf<float>* b : {&B->cdv, &B->ctm, &B->einv}) b->release();
   for (DevBuf<int32_t>* b : {&B->cagg0, &B->ccol, &B->cagg_prob, &B->cadj_ptr, &B->cadj, &B->cnq}) b->release();
   B->einv_off.release();
@@ -1581,7 +2305,7 @@ int sk_batch_set_coarse(sk_batch* B, const double* X, int agg_rows, int period) 
   if ((s = B->cdv.upload(dv32)) || (s = B->ctm.upload(tm32)) || (s = B->cagg0.upload(cagg0)) ||
       (s = B->ccol.upload(ccol)) || (s = B->cagg_prob.upload(cagg_prob)) || (s = B->cadj_ptr.upload(adj_ptr)) ||
       (s = B->cadj.upload(adj)) || (s = B->cnq.upload(cnq)) || (s = B->einv_off.upload(einv_off)) ||
-      (s = B->cE.alloc(etot)) || (s = B->einv.alloc(etot)) || (s = B->cbad.alloc(P)))
+      (s = B->cE.alloc(etot)) || (s = B->einv.alloc(etot + 3)) || (s = B->cbad.alloc(P)))
     return fail(s);
   return SK_OK;
 }
@@ -1604,10 +2328,12 @@ int sk_batch_autotune(sk_batch* B, const double* x_curr, const double* x_prev, c
   hipStream_t caller = as_stream(s);
   SK_HIP_CHECK(hipEventRecord(B->ev_in, caller));
   SK_HIP_CHECK(hipStreamWaitEvent(B->st, B->ev_in, 0));
+  SK_TRY(prepare_even(B));
   // The first Newton system of a step: gradient, Hessian, gather.
   SK_TRY(start_step(B, x_curr, x_prev, x_bc));
-  if (B->coarse() && !B->coarse_built) SK_TRY(build_coarse(B));
-  SK_TRY(hessian_phase(B, false));
+  if (B->coarse() && !B->coarse_built) SK_TRY(build_coarse(B, false));
+  SK_TRY(hessian_phase(B, false, false));
+  if (B->even == 1) SK_TRY(hessian_phase(B, false, true));
   BatchArgs a = B->args();
   a.count_pcg = 0;
   hipEvent_t e0, e1;

@@ -68,6 +68,41 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Sum over the wave in lane 63 (fixed tree of DPP row shifts and broadcasts).
+template <int kCtrl, int kRows>
+__device__ __forceinline__ double dpp_add(double v) {
+  const uint64_t u = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, kCtrl, kRows, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), kCtrl, kRows, 0xf, true);
+  return v + __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+template <int kCtrl, int kRows>
+__device__ __forceinline__ float dpp_add(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kCtrl, kRows, 0xf, true));
+}
+template <typename T>
+__device__ __forceinline__ T wave_sum_last(T v) {
+  v = dpp_add<0x111, 0xf>(v);  // row_shr 1, 2, 4, 8: prefix sums of the rows of 16 lanes
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);  // row_bcast 15 into rows 1 and 3
+  v = dpp_add<0x143, 0xc>(v);  // row_bcast 31 into rows 2 and 3
+  return v;
+}
+
+// Barrier that orders LDS only: the workgroup's waves share nothing else inside
+// the loop, and __syncthreads would also wait for the words just stored.
+__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// x, of unknown value to the compiler: what is computed from it inside the
+// iteration (addresses, unpacked fields) is not hoisted out of it into
+// registers that the matrix blocks need.
+__device__ __forceinline__ int opaque(int x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* lds /* NV * kBlock/kWave */) {
   const int lane = threadIdx.x % kWave;
