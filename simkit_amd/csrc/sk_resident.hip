@@ -64,7 +64,8 @@ struct ResidentArgs {
   const int32_t* exp0;        // [G + 1] exported vertices of the workgroups before this one
   const uint16_t* exslot;     // partial slot of each exported vertex's row (see product)
   uint64_t* slots;  // [kResCopies] x [2][G][kSlotWords]: parity, workgroup, word
-  uint64_t* zx;     // [exported vertices][kVertStride<T>]: A p (or a replaced residual)
+  uint64_t* zx;     // [2][exported vertices][kVertStride<T>]: A p (or a replaced residual), by the meeting's parity
+  uint32_t zx_half; // words of one of the two
   uint64_t* xx;     // [exported vertices][8]: FP64 correction (kMixed)
   T* stream;        // [G][KS][9][NT] streamed blocks
   int* abort_flag;
@@ -273,6 +274,10 @@ struct Meet {
 // alpha and r.r are direct sums of the current residual: the expansion enters
 // beta only. Iteration counts at 48^3 equal the two-launch form's (2,731 and
 // 2,837 over a step in FP64 and mixed precision).
+// Slots and exported vertices' words exist twice and take turns by meeting: a
+// workgroup writes a buffer again only after a meeting that every workgroup
+// joined after its last read of it. (The FP64 correction's words are used once
+// between two meetings.)
 // All workgroups sum the same words in the same order and take the same
 // decisions; results are bit-reproducible for a fixed cut.
 //
@@ -588,8 +593,9 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     meet.template wave_sums<4>(va);
     lds_barrier();
     meet.template publish<4>(epoch);
-    put_exports(T(0), a.zx, epoch);
-    meet.template collect<4, T>(epoch, a.zx, reinterpret_cast<uint32_t*>(HA));
+    uint64_t* zx = a.zx + meet.parity * a.zx_half;
+    put_exports(T(0), zx, epoch);
+    meet.template collect<4, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
     T BH[kBinv];
     load_binv(row ? opaque(v) : 0, B);
     load_binv(opaque(hv), BH);
@@ -658,8 +664,9 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         meet.template wave_sums<2>(vb);
         lds_barrier();
         meet.template publish<2>(epoch);
-        put_exports(T(0), a.zx, epoch);
-        meet.template collect<2, T>(epoch, a.zx, reinterpret_cast<uint32_t*>(HA));
+        zx = a.zx + meet.parity * a.zx_half;
+        put_exports(T(0), zx, epoch);
+        meet.template collect<2, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
         lds_barrier();
         if (s_bad) break;
         meet.template totals<2>(vb);
@@ -983,7 +990,7 @@ int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32) {
   const int NT = fp32 ? kResNT32 : kResNT64;
   SK_TRY(R.slots.alloc((size_t)kResCopies * kResCopyWords));
   const size_t nx = std::max(1, plan->n_exp);
-  SK_TRY(R.zx.alloc(nx * (fp32 ? kVertStride<float> : kVertStride<double>)));
+  SK_TRY(R.zx.alloc(2 * nx * (fp32 ? kVertStride<float> : kVertStride<double>)));
   if (fp32) SK_TRY(R.xx.alloc(nx * kVertStride<double>));
   SK_TRY(R.stream.alloc(std::max<size_t>(16, (size_t)plan->G * plan->KS * 9 * NT * (fp32 ? 4 : 8))));
   SK_TRY(R.abort_flag.alloc(1));
@@ -1004,6 +1011,7 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
   const ResidentPlan& p = *R.plan;
   ResidentArgs<T> a{p.G, p.K, p.KL, p.KS, p.row0.p, m->bptr.p, p.lcol.p, p.tflag.p, p.trow.p, m->sell_pos.p, (const T*)s.vals,
                     (const T*)s.binv, s.fixed, s.g, s.dx, p.halo_ptr.p, p.hvert.p, p.halo.p, p.exp0.p, p.exslot.p, R.slots.p, R.zx.p,
+                    (uint32_t)(R.zx.n / 2),
                     R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
                     p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
   resident_pcg_kernel<T, NT, KR, kMixed><<<p.G, NT, p.lds, st>>>(a);
