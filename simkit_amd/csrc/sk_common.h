@@ -103,6 +103,13 @@ __device__ __forceinline__ int opaque(int x) {
   return x;
 }
 
+// Orders a wave's LDS accesses among its lanes (the wave's own accesses are in order).
+__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// The FP16 values in the low and high halves of a 32-bit word.
+__device__ __forceinline__ float half_lo(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xFFFFu)); }
+__device__ __forceinline__ float half_hi(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
+
 template <int NV>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* lds /* NV * kBlock/kWave */) {
   const int lane = threadIdx.x % kWave;

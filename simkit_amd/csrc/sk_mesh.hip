@@ -151,9 +151,6 @@ __device__ __forceinline__ void wave_count(bool flag, unsigned long long* count)
   if (flag && (int)__lane_id() == __ffsll((long long)m) - 1) atomicAdd(count, (unsigned long long)__popcll(m));
 }
 
-// Orders a wave's LDS accesses among its lanes (the wave's own accesses are in order).
-__device__ __forceinline__ void wave_lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
 // kMode 0: Hessian, vol weight and 9x9 Jacobi PSD projection for every
 // element. kMode 1 (densities with a closed-form eigensystem, PSD on): the
 // eigenvalue modification from that eigensystem; elements it declines are

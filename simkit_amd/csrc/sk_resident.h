@@ -1,10 +1,11 @@
-// Resident PCG: the whole block-Jacobi PCG run of one system in a single
-// launch whose workgroups (at most one per CU) keep their rows' matrix blocks
+// Resident PCG: the whole PCG run of one system (block-Jacobi or two-level) in a
+// single launch whose workgroups (at most one per CU) keep their rows' matrix blocks
 // on chip - registers first, then LDS, the rest streamed from L2 - and meet
 // once per iteration through self-tagged words in global memory instead of
 // at launch boundaries. Described at resident_pcg_kernel.
 #pragma once
 
+#include "sk_coarse.h"
 #include "sk_internal.h"
 
 #include <memory>
@@ -18,12 +19,16 @@ constexpr int kResStaticLds = 2048;   // bound on the kernel's static LDS
 constexpr int kResNT64 = 512, kResKR64 = 8, kResShort64 = 5;
 constexpr int kResNT32 = 512, kResKR32 = 12, kResShort32 = 6;
 constexpr int kResMaxTier = 4;        // blocks per thread in LDS, and streamed from L2, at most (each)
+// With the coarse correction: its values in flight leave fewer registers for blocks.
+constexpr int kResTwoKR64 = 5, kResTwoKR32 = 9, kResTwoTier = 6;
+constexpr int kResMaxPieces = 8;      // aggregates a workgroup's rows reach into, at most (one wave serves them)
 
 // Cut of a mesh's rows into contiguous ranges, one per workgroup, with the
 // index data the kernel reads (built once per mesh and cut on the host).
 struct ResidentPlan {
   std::vector<int32_t> parts;      // [G + 1] the cut (the cache key, with fp32)
   bool fp32 = false;
+  int two_ld = 0, two_need = 0, two_agg = 0;  // what LDS holds of the coarse space (part of the key)
   int G = 0, K = 0, KR = 0, KL = 0, KS = 0;  // blocks per thread: K = registers (up to KR) + LDS (KL) + streamed (KS)
   int max_rows = 0, max_local = 0, max_halo = 0, n_exp = 0;
   size_t lds = 0;                  // dynamic LDS bytes
@@ -43,10 +48,26 @@ struct ResidentResult {
   uint32_t epoch;
 };
 
+// The coarse space of the two-level preconditioner as the cut sees it. A piece
+// is the part of an aggregate that one workgroup's rows hold (pieces are
+// numbered in row order); a workgroup owns the aggregates that begin in it.
+struct ResidentTwo {
+  int n_piece = 0, max_need = 0;
+  DevBuf<int32_t> piece0;          // [G + 1] first piece of each workgroup
+  DevBuf<int32_t> pagg;            // [n_piece] aggregate of each piece
+  DevBuf<int32_t> apiece;          // [n_agg + 1] first piece of each aggregate
+  DevBuf<int32_t> own0;            // [G + 1] first aggregate owned by each workgroup
+  // the aggregates of the workgroup's rows and halo, and where each vertex's stands in that list
+  DevBuf<int32_t> need0, need;     // [G + 1], ids
+  DevBuf<uint16_t> lrow, lhalo;    // [nv], [all halos]
+  DevBuf<uint64_t> cwords, uwords; // [n_piece][8], [n_agg][8] exchanged words
+};
+
 // A simulator's side of the resident solver: its plan and exchange buffers.
 struct ResidentState {
   std::vector<int32_t> parts;            // the caller's cut; empty: the default one
   std::shared_ptr<ResidentPlan> plan;    // null: not built or not eligible
+  std::unique_ptr<ResidentTwo> two;      // with a coarse space
   bool tried = false;                    // plan has been looked for
   bool off = false;                      // a run gave up waiting: launches only from now on
   DevBuf<uint64_t> slots, zx, xx;
@@ -87,11 +108,12 @@ struct ResidentSolve {
   double rtol, inner_rtol;
   int max_iter, max_refine;
   bool fp32;          // FP32 matrix with FP64 residual replacement
+  const CoarseSpace* coarse;  // non-null: two-level preconditioner (built)
 };
 
 // Looks for (or builds) the plan of a simulator on mesh m and allocates the
 // exchange buffers; R.plan stays null when the mesh is not eligible.
-int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32);
+int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse);
 // Enqueues the run (without waiting); the result is in R.host once the stream
 // has been synchronized.
 int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st);

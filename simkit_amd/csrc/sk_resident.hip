@@ -74,7 +74,48 @@ struct ResidentArgs {
   int max_rows, max_local, max_halo;
   double rtol2, inner_rtol2;
   int max_iter, max_refine;
+  // two-level preconditioner (ResidentTwo, CoarseSpace)
+  int ld, n_agg, max_need;
+  double shift;
+  const int32_t *piece0, *pagg, *apiece, *own0, *need0, *need;
+  const uint16_t *lrow, *lhalo;
+  const int32_t *agg_ptr, *agg_col;
+  const double *tm, *dsc, *dv;
+  const _Float16* einv;
+  uint64_t *cwords, *uwords;
 };
+
+// LDS of the coarse space: offsets in doubles from its start.
+struct TwoLds {
+  int c, uw, raw, tm, dsc, s, col, agg, end;
+};
+__host__ __device__ inline TwoLds two_lds(int ld, int max_need, int n_agg) {
+  TwoLds o;
+  o.c = 0;                                // [ld] scaled restricted residual
+  o.uw = o.c + ld;                        // [max_need][6] rigid motions
+  o.raw = o.uw + 6 * max_need;            // [pieces][8 waves][6] of the restriction, then [unknowns][8 waves] of the
+                                          // coarse product: wave sums
+  o.tm = o.raw + kResMaxPieces * 8 * 6;   // [pieces][36]
+  o.dsc = o.tm + kResMaxPieces * 36;      // [pieces][6]
+  o.s = o.dsc + kResMaxPieces * 6;        // [pieces][6] staging
+  o.col = o.s + kResMaxPieces * 6;        // [pieces] first unknown, count, first and last wave (four ints)
+  o.agg = o.col + 2 * kResMaxPieces;      // [n_agg + 1] first piece and unknown of each aggregate (16 bits each)
+  o.end = o.agg + (n_agg + 2) / 2;
+  return o;
+}
+// and behind it the list's aggregates (four bytes each) and two bytes per local vertex: place of its aggregate in the workgroup's list << 3 | fixed DOFs.
+
+constexpr int kAggWords = 8;
+// Six doubles as eight words of 48 payload bits under a 16-bit tag (half a
+// line): word m of half h from its three doubles, and back.
+__device__ __forceinline__ uint64_t pack48(int m, uint64_t d0, uint64_t d1, uint64_t d2) {
+  constexpr uint64_t k48 = (1ull << 48) - 1;
+  return m == 0 ? d0 & k48 : m == 1 ? (d0 >> 48 | d1 << 16) & k48 : m == 2 ? (d1 >> 32 | d2 << 32) & k48 : d2 >> 16;
+}
+__device__ __forceinline__ void put_word48(uint64_t* p, uint32_t epoch, uint64_t v) {
+  __hip_atomic_store(p, ((uint64_t)(epoch & 0xffffu) << 48) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ bool tagged48(uint64_t w, uint32_t epoch) { return (uint32_t)(w >> 48) == (epoch & 0xffffu); }
 
 // Ends a poll that has lasted kPollTicks (about two seconds of the 100 MHz
 // clock) or that another workgroup has ended: every wait is bounded, and the
@@ -281,6 +322,22 @@ struct Meet {
 // All workgroups sum the same words in the same order and take the same
 // decisions; results are bit-reproducible for a fixed cut.
 //
+// kTwo adds the coarse correction W E^-1 W^T r of the two-level preconditioner
+// (sk_coarse.h), and with it a second meeting per iteration. In the first,
+// workgroups also publish the restriction of their rows' A p to each aggregate
+// they reach into (a piece: six doubles in one 64-byte chunk); everybody then
+// holds the whole restricted residual c, and multiplies the rows of the coarse
+// inverse of the aggregates that begin in it, read from L2. In the second they
+// publish r.r, r.z with their share of c.y, and their aggregates' rigid motions,
+// which the workgroups whose rows or halo lie in these add to z. Measured over a
+// step, launches then this kernel: 48^3 FP64 33.1 -> 23.2 ms, mixed 26.6 -> 19.1;
+// 32^3 13.0 -> 8.2 and 12.3 -> 8.1; 10^3 5.7 -> 3.7 and 6.3 -> 3.9. An iteration
+// at 48^3 (35.7 and 29 us) is bound by its chain of phases: product 8 (FP64, five
+// of a thread's blocks from L2) or 2 to 5, pieces of all 512 aggregates 4,
+// rows of the inverse 3.5 to 4.5, second meeting 3 to 5, update 3, the rest around
+// 1 each. With more blocks in registers the values in flight spill (152 registers
+// at eight FP64 blocks: product 16 us).
+//
 // Why: the two-launch form reads 107 MB (FP64) of values per iteration and
 // pays two launch boundaries; 256 CUs hold 128 MB in registers and 40 MB in
 // LDS, so nothing but the halo has to move. Measured per iteration over a
@@ -291,13 +348,14 @@ struct Meet {
 // a thread's twelve blocks streamed from L2). Exchanging B^-1 A p instead of
 // A p, so that the halo needs neither r nor B^-1, was slower: the owner's x and
 // r then leave LDS (FP64 10.7 -> 12.7 us, mixed equal).
-template <typename T, int NT, int KR, bool kMixed>
+template <typename T, int NT, int KR, bool kMixed, bool kTwo>
 __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs<T> a) {
   extern __shared__ double dyn[];
   __shared__ double s_red[4 * (NT / kWave)];
   __shared__ double s_tot[4 * (NT / kWave)];
   __shared__ int s_bad;
   using PV = std::conditional_t<kMixed, double, T>;  // partials
+  constexpr int kTier = kTwo ? kResTwoTier : kResMaxTier;
   const int t = threadIdx.x;
   // workgroup b runs on XCD b % 8: neighbouring parts there, so that most halo words stay in its L2
   const int me = a.G % 8 == 0 ? (blockIdx.x % 8) * (a.G / 8) + blockIdx.x / 8 : blockIdx.x;
@@ -315,14 +373,21 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   T* L = reinterpret_cast<T*>(P64 + (kMixed ? 3 * a.max_local : 0));  // [KL][9][NT]
   int32_t* HX = reinterpret_cast<int32_t*>(L + (size_t)9 * NT * a.KL);  // [max_halo] places of the halo vertices
   uint16_t* EX = reinterpret_cast<uint16_t*>(HX + a.max_halo);        // [NT] partial slots of the exported rows
+  const TwoLds tl = two_lds(a.ld, a.max_need, a.n_agg);
+  double* W2 = reinterpret_cast<double*>(EX + NT + (a.max_halo & 1) * 2);  // coarse space (kTwo)
+  double *C2 = W2 + tl.c, *UW = W2 + tl.uw, *RAW = W2 + tl.raw, *YS = RAW, *TM = W2 + tl.tm, *DS = W2 + tl.dsc, *SD = W2 + tl.s;
+  int4* PC = reinterpret_cast<int4*>(W2 + tl.col);
+  ushort2* AG = reinterpret_cast<ushort2*>(W2 + tl.agg);
+  int32_t* NE = reinterpret_cast<int32_t*>(W2 + tl.end);               // [max_need] the list's aggregates
+  uint16_t* LN = reinterpret_cast<uint16_t*>(NE + a.max_need);         // [max_local]
   T* S = a.stream + (size_t)me * a.KS * 9 * NT;
   if (t == 0) s_bad = 0;
 
   // the thread's blocks, their columns' byte offsets and which of them end a row
   T A[KR][9];
-  uint32_t meta[(KR + 2 * kResMaxTier + 1) / 2];
+  uint32_t meta[(KR + 2 * kTier + 1) / 2];
 #pragma unroll
-  for (int k = 0; k < (KR + 2 * kResMaxTier + 1) / 2; ++k) meta[k] = 0;
+  for (int k = 0; k < (KR + 2 * kTier + 1) / 2; ++k) meta[k] = 0;
   const int tb0 = t * K;
   auto load_block = [&](int k, T (&B)[9]) -> uint32_t {
 #pragma unroll
@@ -338,7 +403,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
 #pragma unroll
   for (int k = 0; k < KR; ++k) meta[k / 2] |= load_block(k, A[k]) << (16 * (k & 1));
 #pragma unroll
-  for (int k = 0; k < kResMaxTier; ++k)
+  for (int k = 0; k < kTier; ++k)
     if (k < a.KL) {
       T B[9];
       meta[(KR + k) / 2] |= load_block(KR + k, B) << (16 * ((KR + k) & 1));
@@ -346,10 +411,10 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       for (int m = 0; m < 9; ++m) L[(k * 9 + m) * NT + t] = B[m];
     }
 #pragma unroll
-  for (int k = 0; k < kResMaxTier; ++k)
+  for (int k = 0; k < kTier; ++k)
     if (k < a.KS) {
       T B[9];
-      constexpr int k0 = KR + kResMaxTier;
+      constexpr int k0 = KR + kTier;
       meta[(k0 + k) / 2] |= load_block(KR + a.KL + k, B) << (16 * ((k0 + k) & 1));
 #pragma unroll
       for (int m = 0; m < 9; ++m) S[(k * 9 + m) * NT + t] = B[m];
@@ -364,7 +429,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     using V = std::remove_cv_t<std::remove_reference_t<decltype(src[0])>>;
     constexpr int U = sizeof(V) == 8 ? 2 : 4;
 #pragma unroll
-    for (int k = 0; k < (KR + 2 * kResMaxTier + 1) / 2; ++k) meta[k] = (uint32_t)opaque((int)meta[k]);
+    for (int k = 0; k < (KR + 2 * kTier + 1) / 2; ++k) meta[k] = (uint32_t)opaque((int)meta[k]);
     const int tt = opaque(t);
     V y0 = 0, y1 = 0, y2 = 0;
     PV* o = part + 3 * slot0;
@@ -408,7 +473,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
     }
 #pragma unroll
-    for (int k = 0; k < kResMaxTier; ++k)
+    for (int k = 0; k < kTier; ++k)
       if (k < a.KL) {
         T B[9];
         V q[3];
@@ -419,18 +484,18 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
     if (a.KS > 0) {
       V q[3];
-      read(word(KR + kResMaxTier), q);
-      add(B0, q, fl & (1u << (KR + kResMaxTier)));
+      read(word(KR + kTier), q);
+      add(B0, q, fl & (1u << (KR + kTier)));
     }
 #pragma unroll
-    for (int k = 1; k < kResMaxTier; ++k)
+    for (int k = 1; k < kTier; ++k)
       if (k < a.KS) {
         T B[9];
         V q[3];
-        read(word(KR + kResMaxTier + k), q);
+        read(word(KR + kTier + k), q);
 #pragma unroll
         for (int m = 0; m < 9; ++m) B[m] = S[(k * 9 + m) * NT + tt];
-        add(B, q, fl & (1u << (KR + kResMaxTier + k)));
+        add(B, q, fl & (1u << (KR + kTier + k)));
       }
     o[0] = (PV)y0;  // the open row's partial (or a slot that no row reads)
     o[1] = (PV)y1;
@@ -515,6 +580,256 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   for (int j = t; j < E; j += NT) EX[j] = a.exslot[x0 + j];
   const int hv = t < H ? a.hvert[h0 + t] : 0;
 
+  // ---- coarse space
+  const int p0 = kTwo ? a.piece0[me] : 0, np = kTwo ? a.piece0[me + 1] - p0 : 0;
+  const int a0 = kTwo ? a.own0[me] : 0, nown = kTwo ? a.own0[me + 1] - a0 : 0;
+  const int n0 = kTwo ? a.need0[me] : 0, nneed = kTwo ? a.need0[me + 1] - n0 : 0;
+  const int wid = t / kWave;
+  int my_piece = -1, pf = 0, pl = -1;  // of the thread's row; of the wave's rows
+  if constexpr (kTwo) {
+    for (int j = t; j < R; j += NT) {
+      const int64_t k = 3 * (int64_t)(v0 + j);
+      const int f = a.fixed ? (a.fixed[k] ? 1 : 0) | (a.fixed[k + 1] ? 2 : 0) | (a.fixed[k + 2] ? 4 : 0) : 0;
+      LN[j] = (uint16_t)(a.lrow[v0 + j] << 3 | f);
+    }
+    for (int j = t; j < H; j += NT) {
+      const int64_t k = 3 * (int64_t)a.hvert[h0 + j];
+      const int f = a.fixed ? (a.fixed[k] ? 1 : 0) | (a.fixed[k + 1] ? 2 : 0) | (a.fixed[k + 2] ? 4 : 0) : 0;
+      LN[R + j] = (uint16_t)(a.lhalo[h0 + j] << 3 | f);
+    }
+    for (int j = t; j < nneed; j += NT) NE[j] = a.need[n0 + j];
+    for (int j = t; j < np * 36; j += NT) TM[j] = a.tm[36 * (int64_t)a.pagg[p0 + j / 36] + j % 36];
+    for (int j = t; j < np * 6; j += NT) {
+      const int c = a.agg_col[a.pagg[p0 + j / 6]] + j % 6;
+      DS[j] = c < a.agg_col[a.pagg[p0 + j / 6] + 1] ? a.dsc[c] : 0.0;
+    }
+    for (int j = t; j <= a.n_agg; j += NT) AG[j] = make_ushort2((uint16_t)a.apiece[j], (uint16_t)a.agg_col[j]);
+    for (int j = t; j < np; j += NT) {
+      const int c = a.agg_col[a.pagg[p0 + j]];
+      const int r0 = max(0, a.agg_ptr[a.pagg[p0 + j]] - v0), r1 = min(R, a.agg_ptr[a.pagg[p0 + j] + 1] - v0);
+      PC[j] = make_int4(c, a.agg_col[a.pagg[p0 + j] + 1] - c, r0 / kWave, (r1 - 1) / kWave);
+    }
+    for (int j = t; j < a.ld; j += NT) C2[j] = 0.0;
+    auto piece_of = [&](int r) {
+      // pieces of one workgroup are aggregates pagg[p0], pagg[p0] + 1, ...
+      int j = 0;
+      while (j + 1 < np && v0 + r >= a.agg_ptr[a.pagg[p0 + j + 1]]) ++j;
+      return j;
+    };
+    if (row) my_piece = piece_of(t);
+    if (wid * kWave < R) {
+      pf = piece_of(wid * kWave);
+      pl = piece_of(min(wid * kWave + kWave - 1, R - 1));
+    }
+  }
+  // The wave's shares of W^T q over the thread's rows, by piece (every thread).
+  auto restrict_rows = [&](double q0, double q1, double q2) {
+    const int t = opaque((int)threadIdx.x);
+    double d[3] = {0.0, 0.0, 0.0};
+    if (row) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) d[q] = a.dv[3 * (int64_t)(v0 + t) + q];
+    }
+    const double m[6] = {q0, q1, q2, d[1] * q2 - d[2] * q1, d[2] * q0 - d[0] * q2, d[0] * q1 - d[1] * q0};
+    for (int j = pf; j <= pl; ++j) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const double w = wave_sum_last(j == my_piece ? m[q] : 0.0);
+        if (t % kWave == kWave - 1) RAW[(j * (NT / kWave) + t / kWave) * 6 + q] = w;
+      }
+    }
+  };
+  // The pieces' scaled restrictions (wave 0, after a barrier).
+  auto put_pieces = [&](uint32_t epoch) {
+    const int t = opaque((int)threadIdx.x);
+    if (t >= kWave) return;
+    const int j = t / 6, q = t % 6;
+    if (t < np * 6) {
+      const int w0 = PC[j].z, w1 = PC[j].w;
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < NT / kWave; ++w)
+        if (w >= w0 && w <= w1) s += RAW[(j * (NT / kWave) + w) * 6 + q];
+      SD[t] = s;
+    }
+    wave_lds_fence();
+    double d = 0.0;
+    if (t < np * 6) {
+#pragma unroll
+      for (int m = 0; m < 6; ++m) d += TM[36 * j + 6 * m + q] * SD[6 * j + m];
+      d *= DS[t];
+    }
+    wave_lds_fence();
+    if (t < np * 6) SD[t] = d;
+    wave_lds_fence();
+    if (t < np * kAggWords) {
+      const uint64_t* d3 = reinterpret_cast<const uint64_t*>(SD + 3 * (t / 4));
+      put_word48(a.cwords + (size_t)p0 * kAggWords + t, epoch, pack48(t % 4, d3[0], d3[1], d3[2]));
+    }
+  };
+  // c = keep c + f (sum over an aggregate's pieces). Slot n is word n % 8 of aggregate n / 8: neighbouring lanes
+  // read neighbouring words, and lanes 0 to 2 of a quad make a double each of their own word and the next one.
+  // The thread's first kSlots sums stay in registers until f is known, further ones are read again.
+  constexpr int kSlots = 8;
+  auto three_of_four = [&](uint64_t w) {
+    constexpr uint64_t k48 = (1ull << 48) - 1;
+    const int m = threadIdx.x % 4;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)w, 0xF9, 0xf, 0xf, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(w >> 32), 0xF9, 0xf, 0xf, true);
+    const uint64_t next = ((uint64_t)hi << 32) | lo;  // quad_perm [1, 2, 3, 3]
+    return __longlong_as_double((long long)((w & k48) >> (16 * m) | next << (48 - 16 * m)));
+  };
+  // sums of the slots t + (i0 + i) NT
+  auto get_slots = [&](int i0, uint32_t epoch, auto& d) {
+    constexpr int N = sizeof(d) / sizeof(double);
+    const int t = opaque((int)threadIdx.x) + i0 * NT;
+    Poll poll;
+    int most = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int I = (t + i * NT) / kAggWords;
+      d[i] = 0.0;
+      if (I < a.n_agg) most = max(most, AG[I + 1].x - AG[I].x);
+    }
+    for (int k = 0; k < most; ++k) {  // the k-th pieces of all slots together
+      uint64_t u[N];
+      uint32_t need = 0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const int I = (t + i * NT) / kAggWords;
+        u[i] = 0;
+        if (I < a.n_agg && k < AG[I + 1].x - AG[I].x) need |= 1u << i;
+      }
+      const uint32_t mine = need;
+      while (need) {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          if (need >> i & 1) u[i] = get_word(a.cwords + (uint32_t)((AG[(t + i * NT) / kAggWords].x + k) * kAggWords + t % kAggWords));
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+          if ((need >> i & 1) && tagged48(u[i], epoch)) need &= ~(1u << i);
+        if (need && poll.give_up(a.abort_flag)) {
+          s_bad = 1;
+          break;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const double x = three_of_four(u[i]);
+        if (mine >> i & 1) d[i] += x;
+      }
+    }
+  };
+  auto add_slots = [&](int i0, const auto& d, double keep, double f) {
+    constexpr int N = sizeof(d) / sizeof(double);
+    const int t = opaque((int)threadIdx.x) + i0 * NT, m = t % kAggWords, q = m % 4 + m / 4 * 3;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int I = (t + i * NT) / kAggWords;
+      if (I < a.n_agg && m % 4 < 3 && AG[I].y + q < AG[I + 1].y) {
+        double* c = C2 + AG[I].y + q;
+        *c = fma(f, d[i], keep * *c);
+      }
+    }
+  };
+  auto add_all = [&](uint32_t epoch, const double (&dh)[kSlots], double keep, double f) {
+    add_slots(0, dh, keep, f);
+    for (int i0 = kSlots; i0 * NT < a.n_agg * kAggWords; ++i0) {
+      double d[1];
+      get_slots(i0, epoch, d);
+      add_slots(i0, d, keep, f);
+    }
+  };
+  // y = (S16 + shift) c for the unknowns of the aggregates that begin here, as wave shares (after a barrier).
+  auto coarse_product = [&]() {
+    const uint4* E8 = reinterpret_cast<const uint4*>(a.einv);
+    const int t = opaque((int)threadIdx.x), ld8 = a.ld >> 3;
+    double c[8];
+#pragma unroll
+    for (int h = 0; h < 8; ++h) c[h] = t < ld8 ? C2[8 * t + h] : 0.0;
+    for (int i = 0; i < nown; ++i) {
+      const int4 pc = PC[i + np - nown];
+      uint4 e[6];
+#pragma unroll
+      for (int q = 0; q < 6; ++q)
+        e[q] = q < pc.y && t < ld8 ? E8[(uint32_t)((pc.x + q) * ld8 + t)] : make_uint4(0u, 0u, 0u, 0u);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) {
+        const uint32_t wd[4] = {e[q].x, e[q].y, e[q].z, e[q].w};
+        double y = 0.0;
+#pragma unroll
+        for (int h = 0; h < 4; ++h)
+          y += (double)half_lo(wd[h]) * c[2 * h] + (double)half_hi(wd[h]) * c[2 * h + 1];
+        y = wave_sum_last(y);
+        if (t % kWave == kWave - 1) YS[(6 * i + q) * (NT / kWave) + t / kWave] = y;
+      }
+    }
+  };
+  // From the wave shares (after a barrier; wave 0): the aggregates' rigid motions; c.y is added to s_red[0].
+  auto put_motions = [&](uint32_t epoch) {
+    const int t = opaque((int)threadIdx.x);
+    if (t >= kWave) return;
+    const int i = t / 6, q = t % 6, j = i + np - nown;  // piece of owned aggregate i
+    double cy = 0.0;
+    if (t < nown * 6) {
+      const int4 pc = PC[j];
+      double y = 0.0;
+      if (q < pc.y) {
+#pragma unroll
+        for (int w = 0; w < NT / kWave; ++w) y += YS[t * (NT / kWave) + w];
+        const double c = C2[pc.x + q];
+        y += a.shift * c;
+        cy = c * y;
+        y *= DS[6 * j + q];
+      }
+      SD[t] = y;
+    }
+    cy = wave_sum_last(cy);
+    if (t == kWave - 1) s_red[0] += cy;
+    wave_lds_fence();
+    double u = 0.0;
+    if (t < nown * 6) {
+#pragma unroll
+      for (int m = 0; m < 6; ++m) u += TM[36 * j + 6 * q + m] * SD[6 * i + m];
+    }
+    wave_lds_fence();
+    if (t < nown * 6) SD[t] = u;
+    wave_lds_fence();
+    if (t < nown * kAggWords) {
+      const uint64_t* d3 = reinterpret_cast<const uint64_t*>(SD + 3 * (t / 4));
+      put_word48(a.uwords + (size_t)a0 * kAggWords + t, epoch, pack48(t % 4, d3[0], d3[1], d3[2]));
+    }
+  };
+  // The rigid motions of the workgroup's list, into UW.
+  auto get_motions = [&](uint32_t epoch) {
+    Poll poll;
+    for (int j = opaque((int)threadIdx.x); j < nneed * kAggWords; j += NT) {
+      const uint64_t* p = a.uwords + (uint32_t)(NE[j / kAggWords] * kAggWords + j % kAggWords);
+      uint64_t w = get_word(p);
+      while (!tagged48(w, epoch)) {
+        if (poll.give_up(a.abort_flag)) {
+          s_bad = 1;
+          break;
+        }
+        w = get_word(p);
+      }
+      uint16_t* o = reinterpret_cast<uint16_t*>(UW) + 3 * j;
+      o[0] = (uint16_t)w;
+      o[1] = (uint16_t)(w >> 16);
+      o[2] = (uint16_t)(w >> 32);
+    }
+  };
+  // z += the rigid motion of local vertex l (mesh vertex w) on its free DOFs
+  auto prolong = [&](int l, const double (&d)[3], T (&z)[3]) {
+    const int n = LN[l];
+    const double* u = UW + 6 * (n >> 3);
+    const double c[3] = {u[0] + u[4] * d[2] - u[5] * d[1], u[1] + u[5] * d[0] - u[3] * d[2],
+                         u[2] + u[3] * d[1] - u[4] * d[0]};
+#pragma unroll
+    for (int q = 0; q < 3; ++q)
+      if (!((n >> q) & 1)) z[q] = (T)((double)z[q] + c[q]);
+  };
+
   // start: r = b, x = 0, p = z
   double acc0[1] = {0.0};
   if (row) {
@@ -551,6 +866,255 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   double tol2 = 0.0, target = 0.0;
   bool fresh = true;  // the tolerance starts from this residual
   __syncthreads();
+  if constexpr (kTwo) {
+    double acc1[1] = {acc0[0]};
+    double dh[kSlots];
+    // what `directions` reads from memory: offsets of the row and of the first halo vertex, B^-1 of the latter
+    T BH[kBinv];
+    double dr[3], dq[3];
+    auto prefetch_directions = [&]() {
+      const int64_t w = row ? opaque(v) : 0, u = opaque(hv);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        dr[q] = a.dv[3 * w + q];
+        dq[q] = a.dv[3 * u + q];
+      }
+      load_binv(u, BH);
+    };
+    // Second meeting of an iteration (c complete, after a barrier): totals of r.z and r.r
+    auto second = [&](double rzb, double rrl, double& rz_out, double& rr_out) -> bool {
+      coarse_product();
+      double vb[2] = {rzb, rrl};
+      meet.template wave_sums<2>(vb);
+      lds_barrier();
+      ++epoch;
+      put_motions(epoch);
+      meet.template publish<2>(epoch);
+      meet.template collect<2, T>(epoch, nullptr, nullptr);
+      prefetch_directions();
+      get_motions(epoch);
+      lds_barrier();
+      if (s_bad) return false;
+      meet.template totals<2>(vb);
+      rz_out = vb[0];
+      rr_out = vb[1];
+      return true;
+    };
+    // p = z + beta p, z = B^-1 r + coarse part (zb: the row's B^-1 r)
+    auto directions = [&](T beta, const T (&zb)[3]) {
+      const int l = opaque(t);
+      if (row) {
+        T z[3] = {zb[0], zb[1], zb[2]};
+        prolong(l, dr, z);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) P[3 * l + q] = fma(beta, P[3 * l + q], z[q]);
+      }
+      for (int j = l; j < H; j += NT) {
+        if (j != l) {
+          const int64_t w = a.hvert[h0 + j];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) dq[q] = a.dv[3 * w + q];
+          load_binv(w, BH);
+        }
+        T z[3];
+        const T rh[3] = {RL[3 * (R + j)], RL[3 * (R + j) + 1], RL[3 * (R + j) + 2]};
+        precondition(BH, rh, z);
+        prolong(R + j, dq, z);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) P[3 * (R + j) + q] = fma(beta, P[3 * (R + j) + q], z[q]);
+      }
+      lds_barrier();
+    };
+    T z[3] = {T(0), T(0), T(0)};  // the row's B^-1 r
+    double rz = 0.0, rr = 0.0;
+    bool go = true;
+    {  // the first residual
+      T B[kBinv], r[3] = {T(0), T(0), T(0)};
+      double v2[2] = {0.0, 0.0};
+      if (row) {
+        load_binv(v, B);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[q] = RL[3 * t + q];
+        precondition(B, r, z);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          v2[0] += (double)r[q] * (double)z[q];
+          v2[1] += (double)r[q] * (double)r[q];
+        }
+      }
+      restrict_rows((double)r[0], (double)r[1], (double)r[2]);
+      meet.template wave_sums<1>(acc1);
+      lds_barrier();
+      meet.template publish<1>(++epoch);
+      put_pieces(epoch);
+      meet.template collect<1, T>(epoch, nullptr, nullptr);
+      get_slots(0, epoch, dh);
+      add_all(epoch, dh, 0.0, 1.0);
+      lds_barrier();
+      go = !s_bad;
+      if (go) {
+        meet.template totals<1>(acc1);
+        target = a.rtol2 * acc1[0];
+        go = second(v2[0], v2[1], rz, rr);
+      }
+      if (go) {
+        tol2 = (kMixed ? a.inner_rtol2 : a.rtol2) * rr;
+        if (!(isfinite(acc1[0]) && isfinite(rr) && isfinite(rz))) done = 3;
+        else if (!(rr > tol2)) done = 1;
+        go = done == 0;
+        if (go) directions(T(0), z);
+      }
+    }
+    while (go) {
+      if (!kMixed && iter >= a.max_iter) break;
+      product(P);
+      T B[kBinv], r[3] = {T(0), T(0), T(0)}, ap[3] = {T(0), T(0), T(0)};
+      lds_barrier();
+      double va[1] = {0.0};
+      if (row) {
+        const int l = opaque(t);
+        PV y[3];
+        row_sum(y);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          ap[q] = (T)y[q];
+          part[3 * s0 + q] = (PV)ap[q];
+          va[0] += (double)P[3 * l + q] * (double)ap[q];
+        }
+      }
+      restrict_rows((double)ap[0], (double)ap[1], (double)ap[2]);
+      meet.template wave_sums<1>(va);
+      lds_barrier();
+      meet.template publish<1>(++epoch);
+      uint64_t* zx = a.zx + meet.parity * a.zx_half;
+      put_exports(T(0), zx, epoch);
+      put_pieces(epoch);
+      get_slots(0, epoch, dh);
+      meet.template collect<1, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
+      load_binv(row ? opaque(v) : 0, B);
+      double xg[3];
+      if (!kMixed && row) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) xg[q] = a.x[3 * (int64_t)opaque(v) + q];
+      }
+      lds_barrier();
+      if (s_bad) break;
+      meet.template totals<1>(va);
+      const double pAp = va[0];
+      if (!(pAp > 0.0)) {
+        done = isfinite(pAp) ? 2 : 3;
+        break;
+      }
+      const T alpha = (T)(rz / pAp);
+      ++iter;
+      add_all(epoch, dh, 1.0, -(double)alpha);
+      const int l = opaque(t);
+      double v2[2] = {0.0, 0.0};
+      if (row) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          if (kMixed) XL[3 * l + q] = fma(alpha, P[3 * l + q], XL[3 * l + q]);
+          else a.x[3 * (int64_t)(v0 + l) + q] = fma((double)alpha, (double)P[3 * l + q], xg[q]);
+          r[q] = fma(-alpha, ap[q], RL[3 * l + q]);
+          RL[3 * l + q] = r[q];
+        }
+        precondition(B, r, z);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          v2[0] += (double)r[q] * (double)z[q];
+          v2[1] += (double)r[q] * (double)r[q];
+        }
+      }
+      for (int j = l; j < H; j += NT) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) RL[3 * (R + j) + q] = fma(-alpha, HA[3 * j + q], RL[3 * (R + j) + q]);
+      }
+      lds_barrier();
+      double rz_next;
+      if (!second(v2[0], v2[1], rz_next, rr)) break;
+      if (!isfinite(rr)) {
+        done = 3;
+        break;
+      }
+      const bool conv = !(rr > tol2), limit = iter >= a.max_iter;
+      if constexpr (!kMixed) {
+        if (conv) {
+          done = 1;
+          break;
+        }
+      } else if (conv || limit) {
+        // residual replacement: dx += x and r = b - A dx in FP64; the search direction is kept
+        ++epoch;
+        ++refines;
+        if (row) {
+          double x64[3];
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            double& dx = a.x[3 * (int64_t)v + q];
+            x64[q] = refines == 1 ? (double)XL[3 * t + q] : dx + (double)XL[3 * t + q];
+            dx = x64[q];
+            XL[3 * t + q] = T(0);
+            P64[3 * t + q] = x64[q];
+            part[3 * s0 + q] = x64[q];
+          }
+        }
+        lds_barrier();
+        put_exports(double(0), a.xx, epoch);
+        meet.template collect<0, double>(epoch, a.xx, reinterpret_cast<uint32_t*>(P64 + 3 * R));
+        lds_barrier();
+        if (s_bad) break;
+        product(P64);
+        lds_barrier();
+        double vb[1] = {0.0};
+        v2[0] = v2[1] = 0.0;
+        if (row) {
+          PV y[3];
+          row_sum(y);
+          load_binv(v, B);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            const double rq = ((fx >> q) & 1) ? 0.0 : rhs(q) - (double)y[q];
+            vb[0] += rq * rq;
+            r[q] = (T)rq;
+            part[3 * s0 + q] = (PV)r[q];
+            RL[3 * t + q] = r[q];
+          }
+          precondition(B, r, z);
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            v2[0] += (double)r[q] * (double)z[q];
+            v2[1] += (double)r[q] * (double)r[q];
+          }
+        }
+        restrict_rows((double)r[0], (double)r[1], (double)r[2]);
+        meet.template wave_sums<1>(vb);
+        lds_barrier();
+        meet.template publish<1>(++epoch);
+        zx = a.zx + meet.parity * a.zx_half;
+        put_exports(T(0), zx, epoch);
+        put_pieces(epoch);
+        meet.template collect<1, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
+        get_slots(0, epoch, dh);
+        add_all(epoch, dh, 0.0, 1.0);
+        lds_barrier();
+        if (s_bad) break;
+        meet.template totals<1>(vb);
+        if (!(vb[0] > target) || refines >= a.max_refine || limit) {
+          done = vb[0] <= target ? 1 : isfinite(vb[0]) ? 0 : 3;
+          break;
+        }
+        for (int j = t; j < H; j += NT) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) RL[3 * (R + j) + q] = HA[3 * j + q];
+        }
+        if (!second(v2[0], v2[1], rz_next, rr)) break;
+        tol2 = a.inner_rtol2 * rr;
+      }
+      const T beta = (T)(rz_next / rz);
+      rz = rz_next;
+      directions(beta, z);
+    }
+  } else {
   if (kMixed) {  // ||b||^2 in FP64
     meet.template wave_sums<1>(acc0);
     lds_barrier();
@@ -731,6 +1295,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     }
     lds_barrier();
   }
+  }
   __syncthreads();
   if (s_bad) {
     if (t == 0) {
@@ -768,6 +1333,9 @@ size_t base_lds(bool fp32, int max_rows, int max_local, int max_halo) {
   const size_t v = fp32 ? 12 : 24;
   return 24 * (size_t)(max_rows + NT + 1) + (fp32 ? 24 * (size_t)max_local + 12 * (size_t)max_rows : 0) +
          2 * v * max_local + v * max_halo + 4 * (size_t)max_halo + 2 * (size_t)NT + 64;
+}
+size_t two_lds_bytes(int ld, int max_need, int n_agg, int max_local) {
+  return 8 * (size_t)two_lds(ld, max_need, n_agg).end + 4 * (size_t)max_need + 2 * (size_t)max_local + 16;
 }
 size_t tier_lds(bool fp32) { return (fp32 ? kResNT32 : kResNT64) * (9 * (fp32 ? 4 : 8)) * (size_t)1; }
 
@@ -846,12 +1414,13 @@ int resident_parts(int64_t nv, int64_t nblk, bool fp32) {
 // Blocks per thread in registers: the short variant where all of a thread's
 // blocks fit it (no register spilled: 10^3 FP64 5.8 us an iteration against
 // 6.5 us with the long one), else the long one.
-static int resident_kr(bool fp32, int K) {
-  if (fp32) return K <= kResShort32 ? kResShort32 : kResKR32;
-  return K <= kResShort64 ? kResShort64 : kResKR64;
+static int resident_kr(bool fp32, bool two, int K) {
+  if (fp32) return K <= kResShort32 ? kResShort32 : two ? kResTwoKR32 : kResKR32;
+  return K <= kResShort64 ? kResShort64 : two ? kResTwoKR64 : kResKR64;
 }
 
-static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<int32_t>& parts, bool fp32, int* status) {
+static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<int32_t>& parts, bool fp32, int two_ld,
+                                                int two_need, int two_agg, int* status) {
   *status = SK_OK;
   const int NT = fp32 ? kResNT32 : kResNT64;
   const int G = (int)parts.size() - 1;
@@ -859,6 +1428,9 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   auto p = std::make_shared<ResidentPlan>();
   p->parts = parts;
   p->fp32 = fp32;
+  p->two_ld = two_ld;
+  p->two_need = two_need;
+  p->two_agg = two_agg;
   p->G = G;
   int max_nb = 0;
   for (int g = 0; g < G; ++g) {
@@ -867,7 +1439,8 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   }
   if (p->max_rows > NT) return nullptr;
   p->K = std::max(1, (max_nb + NT - 1) / NT);
-  p->KR = resident_kr(fp32, p->K);
+  p->KR = resident_kr(fp32, two_ld > 0, p->K);
+  const int tier = two_ld ? kResTwoTier : kResMaxTier;
   const int KR = p->KR;
   std::vector<int32_t> loc(m->nv, -1), halo_ptr(1, 0), halo;
   std::vector<int16_t> place(m->nv, -1);
@@ -928,19 +1501,20 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
       const int32_t r0 = parts[owner[v]];
       exslot[exp0[owner[v]] + place[v]] = (uint16_t)(v - r0 + (bptr[v] - bptr[r0]) / p->K);
     }
-  const size_t base = base_lds(fp32, p->max_rows, p->max_local, p->max_halo) + kResStaticLds;
+  const size_t base = base_lds(fp32, p->max_rows, p->max_local, p->max_halo) +
+                      (two_ld ? two_lds_bytes(two_ld, two_need, two_agg, p->max_local) : 0) + kResStaticLds;
   if (base > (size_t)kResLds) return nullptr;
   const int rest = std::max(0, p->K - KR);
-  p->KL = (int)std::min<size_t>(std::min(rest, kResMaxTier), (kResLds - base) / tier_lds(fp32));
+  p->KL = (int)std::min<size_t>(std::min(rest, tier), (kResLds - base) / tier_lds(fp32));
   p->KS = rest - p->KL;
-  if (p->KS > kResMaxTier) return nullptr;
-  // the threads' row-end bits: registers, the LDS tier (kResMaxTier bits), the streamed tier
-  static_assert(kResKR32 + 2 * kResMaxTier <= 32 && kResKR64 + 2 * kResMaxTier <= 32, "one bit per block");
+  if (p->KS > tier) return nullptr;
+  // the threads' row-end bits: registers, the LDS tier (`tier` bits), the streamed tier
+  static_assert(kResKR32 + 2 * kResMaxTier <= 32 && kResTwoKR32 + 2 * kResTwoTier <= 32, "one bit per block");
   std::vector<uint32_t> tflag((size_t)G * NT, 0);
   for (int g = 0; g < G; ++g)
     for (int32_t r = parts[g]; r < parts[g + 1]; ++r) {
       const int th = tlast[r] / p->K, k = tlast[r] % p->K;
-      tflag[(size_t)g * NT + th] |= 1u << (k < KR + p->KL ? k : KR + kResMaxTier + (k - KR - p->KL));
+      tflag[(size_t)g * NT + th] |= 1u << (k < KR + p->KL ? k : KR + tier + (k - KR - p->KL));
     }
   p->lds = base - kResStaticLds + p->KL * tier_lds(fp32);
   // more than half of a CU's LDS: one workgroup per CU, so the runs spread over the chip
@@ -962,23 +1536,134 @@ static std::shared_ptr<ResidentPlan> build_plan(sk_mesh* m, const std::vector<in
   return *status == SK_OK ? p : nullptr;
 }
 
-int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32) {
+// The coarse space seen by a cut; null when a workgroup would reach into more
+// than kResMaxPieces aggregates.
+static std::unique_ptr<ResidentTwo> build_two(const sk_mesh* m, const std::vector<int32_t>& parts, const CoarseSpace& C,
+                                              int* status) {
+  *status = SK_OK;
+  const int G = (int)parts.size() - 1, n_agg = C.n_agg;
+  std::vector<int32_t> ap(n_agg + 1), vagg(m->nv);
+  if (hipMemcpy(ap.data(), C.agg_ptr.p, ap.size() * sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess) {
+    set_error("resident PCG: the aggregates could not be read");
+    *status = SK_ERR_HIP;
+    return nullptr;
+  }
+  for (int I = 0; I < n_agg; ++I)
+    for (int32_t v = ap[I]; v < ap[I + 1]; ++v) vagg[v] = I;
+  auto two = std::make_unique<ResidentTwo>();
+  std::vector<int32_t> piece0(1, 0), pagg, apiece(n_agg + 1, -1), own0(G + 1), need0(1, 0), need, mine, ids;
+  std::vector<uint16_t> lrow(m->nv), lhalo;
+  std::vector<int32_t> seen(m->nv, -1), place(n_agg, -1);
+  for (int g = 0; g < G; ++g) {
+    const int32_t r0 = parts[g], r1 = parts[g + 1];
+    own0[g] = (int32_t)(std::lower_bound(ap.begin(), ap.end() - 1, r0) - ap.begin());
+    for (int I = vagg[r0]; I <= vagg[r1 - 1]; ++I) {
+      if (apiece[I] < 0) apiece[I] = (int32_t)pagg.size();
+      pagg.push_back(I);
+    }
+    if (vagg[r1 - 1] - vagg[r0] >= kResMaxPieces) return nullptr;
+    piece0.push_back((int32_t)pagg.size());
+    // the halo in the plan's order (ascending) and the aggregates of rows and halo
+    mine.clear();
+    for (int32_t b = m->h_bptr[r0]; b < m->h_bptr[r1]; ++b) {
+      const int32_t w = m->h_bcol[b];
+      if ((w < r0 || w >= r1) && seen[w] != g) {
+        seen[w] = g;
+        mine.push_back(w);
+      }
+    }
+    std::sort(mine.begin(), mine.end());
+    ids.clear();
+    auto list = [&](int32_t w) {
+      const int I = vagg[w];
+      if (place[I] < 0) {
+        place[I] = (int32_t)ids.size();
+        ids.push_back(I);
+      }
+      return (uint16_t)place[I];
+    };
+    for (int32_t r = r0; r < r1; ++r) lrow[r] = list(r);
+    for (int32_t w : mine) lhalo.push_back(list(w));
+    for (int32_t I : ids) place[I] = -1;
+    if (ids.size() >= (1u << 13)) return nullptr;
+    need.insert(need.end(), ids.begin(), ids.end());
+    need0.push_back((int32_t)need.size());
+    two->max_need = std::max(two->max_need, (int)ids.size());
+  }
+  own0[G] = n_agg;
+  apiece[n_agg] = (int32_t)pagg.size();
+  two->n_piece = (int)pagg.size();
+  if (two->n_piece > 65535) return nullptr;  // 16-bit numbers in LDS
+  if (lhalo.empty()) lhalo.push_back(0);
+  auto up = [&]() -> int {
+    SK_TRY(two->piece0.upload(piece0));
+    SK_TRY(two->pagg.upload(pagg));
+    SK_TRY(two->apiece.upload(apiece));
+    SK_TRY(two->own0.upload(own0));
+    SK_TRY(two->need0.upload(need0));
+    SK_TRY(two->need.upload(need));
+    SK_TRY(two->lrow.upload(lrow));
+    SK_TRY(two->lhalo.upload(lhalo));
+    SK_TRY(two->cwords.alloc((size_t)two->n_piece * 8));
+    SK_TRY(two->uwords.alloc((size_t)n_agg * 8));
+    SK_HIP_CHECK(hipMemset(two->cwords.p, 0, two->cwords.n * 8));
+    SK_HIP_CHECK(hipMemset(two->uwords.p, 0, two->uwords.n * 8));
+    return SK_OK;
+  };
+  *status = up();
+  return *status == SK_OK ? std::move(two) : nullptr;
+}
+
+int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse) {
   if (R.tried) return SK_OK;
   R.tried = true;
+  R.two.reset();
   std::vector<int32_t> parts = R.parts;
   if (parts.empty()) {
     const int G = resident_parts(m->nv, m->nblk, fp32);
     if (G == 0) return SK_OK;
-    for (int g = 0; g <= G; ++g) parts.push_back((int32_t)(m->nv * g / G));
+    std::vector<int32_t> ap;
+    int most = 0;
+    if (coarse) {
+      ap.resize(coarse->n_agg + 1);
+      SK_HIP_CHECK(hipMemcpy(ap.data(), coarse->agg_ptr.p, ap.size() * sizeof(int32_t), hipMemcpyDeviceToHost));
+      for (int I = 0; I < coarse->n_agg; ++I) most = std::max(most, ap[I + 1] - ap[I]);
+    }
+    // With a coarse space and workgroups enough for one per aggregate, a whole number of workgroups for each, as few
+    // as let the average one's blocks fit the short variant: pieces of an aggregate are read one after the other.
+    // (A step, at 1 / 2 / 4 workgroups per aggregate and with equal cuts: 10^3 FP64 3.7 / 3.9 / 4.3 / 5.0 ms, 24^3 8.2
+    // / 8.0 / 9.0 / 10.0, an 8 x 60 x 8 box 10.9 / 9.5 / 10.3 / 14.7.)
+    const int64_t NT = fp32 ? kResNT32 : kResNT64, fill = NT * (fp32 ? kResShort32 : kResShort64);
+    const int split = !coarse ? 0 : (int)std::max((most + NT - 1) / NT, (m->nblk + coarse->n_agg * fill - 1) / (coarse->n_agg * fill));
+    if (coarse && G >= coarse->n_agg && split * coarse->n_agg <= kResMaxParts) {
+      parts.push_back(0);
+      for (int I = 0; I < coarse->n_agg; ++I)
+        for (int k = 1; k <= split; ++k) {
+          const int32_t end = ap[I] + (int32_t)((int64_t)(ap[I + 1] - ap[I]) * k / split);
+          if (end > parts.back()) parts.push_back(end);
+        }
+    } else {
+      for (int g = 0; g <= G; ++g) parts.push_back((int32_t)(m->nv * g / G));
+    }
   }
+  std::unique_ptr<ResidentTwo> two;
+  if (coarse) {
+    int s = SK_OK;
+    two = build_two(m, parts, *coarse, &s);
+    if (s != SK_OK) return s;
+    if (!two) return SK_OK;
+  }
+  const int two_ld = coarse ? coarse->ld : 0, two_need = coarse ? two->max_need : 0,
+            two_agg = coarse ? coarse->n_agg : 0;
   std::shared_ptr<ResidentPlan> plan;
   {
     std::lock_guard<std::mutex> lock(m->plan_mu);
     for (auto& p : m->plans)
-      if (p->fp32 == fp32 && p->parts == parts) plan = p;
+      if (p->fp32 == fp32 && p->two_ld == two_ld && p->two_need == two_need &&
+          p->two_agg == two_agg && p->parts == parts) plan = p;
     if (!plan) {
       int s = SK_OK;
-      plan = build_plan(m, parts, fp32, &s);
+      plan = build_plan(m, parts, fp32, two_ld, two_need, two_agg, &s);
       if (s != SK_OK) return s;
       if (plan) {
         if (m->plans.size() >= 4) m->plans.erase(m->plans.begin());
@@ -999,14 +1684,15 @@ int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32) {
   if (fp32) SK_HIP_CHECK(hipMemset(R.xx.p, 0, R.xx.n * 8));
   SK_HIP_CHECK(hipMemset(R.abort_flag.p, 0, sizeof(int)));
   SK_HIP_CHECK(hipDeviceSynchronize());
-  SK_HIP_CHECK(hipHostMalloc((void**)&R.host, sizeof(ResidentResult), hipHostMallocCoherent));
+  if (!R.host) SK_HIP_CHECK(hipHostMalloc((void**)&R.host, sizeof(ResidentResult), hipHostMallocCoherent));
   *R.host = ResidentResult{};
   R.epoch = 0;
   R.plan = plan;
+  R.two = std::move(two);
   return SK_OK;
 }
 
-template <typename T, int NT, int KR, bool kMixed>
+template <typename T, int NT, int KR, bool kMixed, bool kTwo>
 static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st) {
   const ResidentPlan& p = *R.plan;
   ResidentArgs<T> a{p.G, p.K, p.KL, p.KS, p.row0.p, m->bptr.p, p.lcol.p, p.tflag.p, p.trow.p, m->sell_pos.p, (const T*)s.vals,
@@ -1014,7 +1700,31 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
                     (uint32_t)(R.zx.n / 2),
                     R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
                     p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
-  resident_pcg_kernel<T, NT, KR, kMixed><<<p.G, NT, p.lds, st>>>(a);
+  if (kTwo) {
+    const CoarseSpace& C = *s.coarse;
+    const ResidentTwo& w = *R.two;
+    a.ld = C.ld;
+    a.n_agg = C.n_agg;
+    a.max_need = w.max_need;
+    a.shift = C.shift;
+    a.piece0 = w.piece0.p;
+    a.pagg = w.pagg.p;
+    a.apiece = w.apiece.p;
+    a.own0 = w.own0.p;
+    a.need0 = w.need0.p;
+    a.need = w.need.p;
+    a.lrow = w.lrow.p;
+    a.lhalo = w.lhalo.p;
+    a.agg_ptr = C.agg_ptr.p;
+    a.agg_col = C.agg_col.p;
+    a.tm = C.tm.p;
+    a.dsc = C.dsc.p;
+    a.dv = C.dv64.p;
+    a.einv = C.einv.p;
+    a.cwords = w.cwords.p;
+    a.uwords = w.uwords.p;
+  }
+  resident_pcg_kernel<T, NT, KR, kMixed, kTwo><<<p.G, NT, p.lds, st>>>(a);
   SK_HIP_CHECK(hipGetLastError());
   return SK_OK;
 }
@@ -1025,14 +1735,23 @@ int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStr
     SK_TRY(clear_words(R.slots, st));
     SK_TRY(clear_words(R.zx, st));
     SK_TRY(clear_words(R.xx, st));
+    if (R.two) {
+      SK_TRY(clear_words(R.two->cwords, st));
+      SK_TRY(clear_words(R.two->uwords, st));
+    }
     R.epoch = 0;
   }
   *R.host = ResidentResult{0, 0, 0, 0, R.epoch};
-  if (s.fp32)
-    return R.plan->KR == kResShort32 ? launch<float, kResNT32, kResShort32, true>(R, m, s, st)
-                                     : launch<float, kResNT32, kResKR32, true>(R, m, s, st);
-  return R.plan->KR == kResShort64 ? launch<double, kResNT64, kResShort64, false>(R, m, s, st)
-                                   : launch<double, kResNT64, kResKR64, false>(R, m, s, st);
+  auto run = [&](auto two) {
+    constexpr bool kTwo = decltype(two)::value;
+    constexpr int kLong32 = kTwo ? kResTwoKR32 : kResKR32, kLong64 = kTwo ? kResTwoKR64 : kResKR64;
+    if (s.fp32)
+      return R.plan->KR == kResShort32 ? launch<float, kResNT32, kResShort32, true, kTwo>(R, m, s, st)
+                                       : launch<float, kResNT32, kLong32, true, kTwo>(R, m, s, st);
+    return R.plan->KR == kResShort64 ? launch<double, kResNT64, kResShort64, false, kTwo>(R, m, s, st)
+                                     : launch<double, kResNT64, kLong64, false, kTwo>(R, m, s, st);
+  };
+  return s.coarse ? run(std::true_type{}) : run(std::false_type{});
 }
 
 

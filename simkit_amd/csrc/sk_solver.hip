@@ -1,5 +1,9 @@
 // Preconditioned conjugate gradients and the device backward-Euler driver.
 //
+// Meshes that fit the chip are solved by one launch (sk_resident.h). The forms
+// here serve larger ones, launch widths that the caller sets, a device that
+// does not let all workgroups run at once, and the pipelined variant.
+//
 // PCG iteration k = 2 launches, no fences, no atomics:
 //   spmv(k):   every block first sums the previous launch's per-block
 //              partials (r.z, r.r) in a fixed order, derives beta and the
@@ -756,10 +760,6 @@ __global__ __launch_bounds__(kBlock) void bpcg_update_kernel(BlockPcgArgs<T> a) 
   }
   finish_vertex_pass<kAgg>(a, rz, rr, raw, pre);
 }
-
-// The FP16 values in the low and high halves of a 32-bit word.
-__device__ __forceinline__ float half_lo(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w & 0xFFFFu)); }
-__device__ __forceinline__ float half_hi(uint32_t w) { return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16)); }
 
 // A vertex of the coarse kernel's prolongation: aggregate-order position t
 // (none when t >= t1), its vertex, centroid offset, z and free mask.
@@ -1614,11 +1614,12 @@ struct sk_sim {
   // recurrences' identity p.Ap = delta - beta gamma / alpha_prev in FP32 (the replaced residual is
   // no longer r_prev - alpha s_prev to the recurrences' accuracy; a numpy emulation of the FP32 run
   // breaks down at the second replacement).
-  // The resident PCG serves the classic block-Jacobi form with the library's own launch shape; a caller
+  // The resident PCG serves the classic form (block-Jacobi, or two-level with the vertices numbered
+  // aggregate by aggregate) with the library's own launch shape; a caller
   // that sets the launch widths or the chunk length asks for the launches.
   bool may_be_resident() const {
-    return !res.off && (prm.pcg_variant == 0 || mixed()) && !two_level() && prm.spmv_blocks == 0 && prm.update_blocks == 0 &&
-           prm.pcg_chunk == 0;
+    return !res.off && (prm.pcg_variant == 0 || mixed() || two_level()) && (!two_level() || coarse.ident) &&
+           prm.spmv_blocks == 0 && prm.update_blocks == 0 && prm.pcg_chunk == 0 && prm.pcg_max_iter > 0;
   }
   bool pipelined() const { return prm.pcg_variant == 1 && !two_level() && !mixed(); }
 };
@@ -2014,6 +2015,9 @@ int sk_sim_destroy(sk_sim* S) {
 int sk_sim_set_coarse(sk_sim* S, const double* X, int per_agg) {
   SK_REQUIRE(S, "sk_sim_set_coarse: null simulator");
   S->coarse = CoarseSpace();
+  S->res.plan.reset();  // the cut and its LDS depend on the coarse space
+  S->res.two.reset();
+  S->res.tried = false;
   if (per_agg <= 0) return SK_OK;
   SK_REQUIRE(X, "sk_sim_set_coarse: null positions");
   const int64_t n3 = 3 * S->mesh->nv;
@@ -2023,8 +2027,12 @@ int sk_sim_set_coarse(sk_sim* S, const double* X, int per_agg) {
     SK_HIP_CHECK(hipMemcpy(fixed.data(), S->fixed.p, n3, hipMemcpyDeviceToHost));
   }
   const int s = coarse_setup(S->coarse, S->mesh, X, S->fixed.p ? fixed.data() : nullptr, per_agg);
-  if (s != SK_OK) S->coarse = CoarseSpace();
-  return s;
+  if (s != SK_OK) {
+    S->coarse = CoarseSpace();
+    return s;
+  }
+  // the resident solver's plan goes with it
+  return S->may_be_resident() ? resident_prepare(S->res, S->mesh, S->mixed(), &S->coarse) : SK_OK;
 }
 
 int sk_sim_set_order(sk_sim* S, const int32_t* order_host) {
@@ -2158,10 +2166,13 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
     bool resident = false;
     ResidentPermit permit;
     if (S->may_be_resident()) {
-      SK_TRY(resident_prepare(S->res, m, mixed));
+      SK_TRY(resident_prepare(S->res, m, mixed, S->two_level() ? &S->coarse : nullptr));
       if (S->res.plan && permit.acquire(S->res.plan->G, st)) {
         ResidentSolve rs{S->vals.p, S->binv.p, fixed, S->g.p, S->dx.p, P.pcg_rtol, P.inner_rtol, P.pcg_max_iter,
-                         P.max_refine, mixed};
+                         P.max_refine, mixed, S->two_level() ? &S->coarse : nullptr};
+        // the coarse operator is formed from the first system solved and kept
+        if (S->two_level() && !S->coarse.built)
+          SK_TRY(coarse_build(S->coarse, m, mixed ? (const void*)S->vals32.p : S->vals.p, mixed, fixed, st));
         if (mixed) {
           rs.vals = S->vals32.p;
           rs.binv = S->binv32.p;

@@ -46,15 +46,16 @@ class BackwardEulerSim:
         raised as needed to keep the coarse space within the library's 4,096 unknowns; the coarse
         operator is formed from the first system solved). Both solve to pcg_rtol.
         renumber: the simulator numbers the vertices internally in the order its kernels read
-        them (two-level: aggregate by aggregate, so that each aggregate is a contiguous range, and
-        in the sliced-ELL order within an aggregate; block-Jacobi: the sliced-ELL row order, so
-        that the SpMV's row stores are contiguous);
+        them (two-level: aggregate by aggregate, so that each aggregate is a contiguous range;
+        block-Jacobi: boxes of the mesh, one per workgroup of the PCG kernel, sk_part_order);
         states passed in and returned keep the caller's vertex order (the library permutes them in the
         step's first and last kernels, sk_sim_set_order).
         max_inverted: < 0 no limit; otherwise a step that ends with more elements of det F <= 0 reports
         status SK_ERR_INVERTED (info["inverted_elems"] always holds the count).
-        pcg: "classic" (two launches per block-Jacobi PCG iteration) or "pipelined" (one launch per
-        iteration: Ghysels-Vanroose recurrences on A B^-1); the two-level preconditioner is classic.
+        pcg: "classic" (each solve in one launch that keeps the matrix on chip, for meshes that fit;
+        else, or when spmv_blocks, update_blocks or pcg_chunk is given, two launches per block-Jacobi
+        iteration) or "pipelined" (one launch per iteration: Ghysels-Vanroose recurrences on A B^-1;
+        FP64 block-Jacobi).
         psd_solver: "closed_form" (stable neo-Hookean's Hessian eigensystem from the SVD of F, the 9x9
         Jacobi for other densities and near-singular F) or "jacobi" (the 9x9 Jacobi for every element)."""
         if preconditioner not in ("bjacobi", "two_level"):
@@ -90,14 +91,7 @@ class BackwardEulerSim:
             order = np.empty(self.nv, np.int32)
             Tc = np.ascontiguousarray(T, dtype=np.int32)
             if preconditioner == "two_level":
-                _lib.call("sk_sell_order", Tc.ctypes.data_as(ctypes.c_void_p), int(self.nv), int(self.nt),
-                          order.ctypes.data_as(ctypes.c_void_p))
-                # aggregate by aggregate, each aggregate's vertices in the sliced-ELL order (descending
-                # block count, ties by index), so that a SELL chunk's rows are mostly consecutive
-                rank = np.empty(self.nv, np.int64)
-                rank[order] = np.arange(self.nv)
-                key = np.repeat(np.arange(len(agg_ptr) - 1, dtype=np.int64), np.diff(agg_ptr)) * self.nv
-                order[:] = agg_order[np.argsort(key + rank[agg_order], kind="stable")]
+                order[:] = agg_order  # aggregate by aggregate, each in index order
             else:
                 Xc = np.ascontiguousarray(X, dtype=np.float64)
                 n_parts, ptr_ = ctypes.c_int(), np.empty(257, np.int32)
