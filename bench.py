@@ -10,7 +10,8 @@ Armijo backtracking. A "step" is one full backward-Euler step; the timed
 region runs the first --steps steps from rest with the mesh resident in HBM.
 
 Prints one JSON line (rank 0). Also measures, on the same stream with HIP
-events, the average duration of the dominant kernel (the block-CSR PCG SpMV)
+events, the average duration of the block-CSR SpMV of the launch-per-phase PCG
+(the step itself solves in one resident launch that keeps the matrix on chip)
 for the roofline object, and times the CPU oracle on a bounded sample of the
 same workload for cpu_baseline.
 """
@@ -37,7 +38,7 @@ FP64_PEAK_TFLOPS = 78.6
 # element pass of the stable neo-Hookean density: the closed-form eigensystem launch (the Jacobi
 # fallback launch that follows it runs only on the elements the first declines)
 HESS_KERNEL = {"fp64": "elem_hess_kernel<SNH, 1, double, 1>", "mixed": "elem_hess_kernel<SNH, 1, float, 1>"}
-# dominant kernel of each path (the FP32 SpMV walks chunk ranges with 1024 workgroups)
+# SpMV of the launch-per-phase PCG, the kernel that streams the whole matrix
 SPMV_KERNEL = {"fp64": "bpcg_spmv_kernel<double, false>", "mixed": "bpcg_spmv_kernel<float, false>"}
 METRIC = "BE steps/s, 48^3-cell neo-Hookean (353k DOF), learned+FP32 vs plain FP64"
 
@@ -65,9 +66,9 @@ def spmv_bytes(nv, nblk, value_bytes):
 
 def elem_bytes(nv, nt, value_bytes):
     """Algorithmic HBM bytes of one element pass: per tet its 4 vertex ids, 12 shape-function
-    derivatives, mu, lambda and volume (FP64), a flag byte, and the 10 staged 3x3 blocks (90 values)
+    derivatives, mu, lambda and volume (FP64), a flag byte, and the staged symmetric stiffness (78 values)
     written; the positions read once per vertex."""
-    return nt * (16 + 96 + 24 + 1 + 90 * value_bytes) + 24 * nv
+    return nt * (16 + 96 + 24 + 1 + 78 * value_bytes) + 24 * nv
 
 
 def pmc_traffic(path_key):
@@ -241,7 +242,7 @@ def run_path(args, X, T, bottom, top, mu, lam, name):
     x_final, infos = run(args.steps)
     torch.cuda.synchronize()
     elapsed = time.perf_counter() - t0
-    # dominant kernel: the PCG SpMV, average over back-to-back launches on this stream
+    # the SpMV of the launch-per-phase PCG, average over back-to-back launches on this stream
     stream = torch.cuda.current_stream()
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     e0.record(stream)
