@@ -2327,7 +2327,13 @@ int sk_sim_spmv_reps(sk_sim* S, int reps, sk_stream_t s) {
   SK_REQUIRE(S && reps >= 0, "sk_sim_spmv_reps: invalid argument");
   hipStream_t st = as_stream(s);
   // Per-step scratch vectors only; rtol 0 so every launch runs iteration 0 in
-  // full. Right-hand side: the last gradient (FP64) or the last FP32 residual.
+  // full. Right-hand side: the last gradient (rounded to FP32 on the mixed path).
+  if (S->mixed()) {
+    sk_mesh* m = S->mesh;
+    ResidualArgs ra{m->nv, sell_view(m), S->vals32.p, S->fixed.p, S->g.p, nullptr, S->r.p, S->r32.p,
+                    m->red.partials.p + 4 * (size_t)Reducer::kMaxBlocks};
+    ir_residual_kernel<<<sell_grid(m), kBlock, 0, st>>>(ra);
+  }
   // The pipelined form runs its iteration kernel: one start launch, then reps
   // consecutive iterations (rtol 0: none stops early on an SPD system).
   if (S->pipelined()) {
