@@ -112,8 +112,9 @@ struct ResidentSolve {
 };
 
 // Looks for (or builds) the plan of a simulator on mesh m and allocates the
-// exchange buffers; R.plan stays null when the mesh is not eligible.
-int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse);
+// exchange buffers, once; R.plan stays null when the mesh is not eligible or
+// memory runs out.
+void resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse);
 // Enqueues the run (without waiting); the result is in R.host once the stream
 // has been synchronized.
 int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st);

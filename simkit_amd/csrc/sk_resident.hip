@@ -1614,10 +1614,7 @@ static std::unique_ptr<ResidentTwo> build_two(const sk_mesh* m, const std::vecto
   return *status == SK_OK ? std::move(two) : nullptr;
 }
 
-int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse) {
-  if (R.tried) return SK_OK;
-  R.tried = true;
-  R.two.reset();
+static int prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse) {
   std::vector<int32_t> parts = R.parts;
   if (parts.empty()) {
     const int G = resident_parts(m->nv, m->nblk, fp32);
@@ -1690,6 +1687,21 @@ int resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace*
   R.plan = plan;
   R.two = std::move(two);
   return SK_OK;
+}
+
+void resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace* coarse) {
+  if (R.tried) return;
+  R.tried = true;
+  R.plan.reset();
+  R.two.reset();
+  if (prepare(R, m, fp32, coarse) == SK_OK) return;
+  // no memory for it: the launches need none of this
+  (void)hipGetLastError();
+  R.plan.reset();
+  R.two.reset();
+  for (DevBuf<uint64_t>* b : {&R.slots, &R.zx, &R.xx}) b->release();
+  R.stream.release();
+  R.abort_flag.release();
 }
 
 template <typename T, int NT, int KR, bool kMixed, bool kTwo>

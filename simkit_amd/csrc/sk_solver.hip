@@ -2032,7 +2032,8 @@ int sk_sim_set_coarse(sk_sim* S, const double* X, int per_agg) {
     return s;
   }
   // the resident solver's plan goes with it
-  return S->may_be_resident() ? resident_prepare(S->res, S->mesh, S->mixed(), &S->coarse) : SK_OK;
+  if (S->may_be_resident()) resident_prepare(S->res, S->mesh, S->mixed(), &S->coarse);
+  return SK_OK;
 }
 
 int sk_sim_set_order(sk_sim* S, const int32_t* order_host) {
@@ -2166,7 +2167,7 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
     bool resident = false;
     ResidentPermit permit;
     if (S->may_be_resident()) {
-      SK_TRY(resident_prepare(S->res, m, mixed, S->two_level() ? &S->coarse : nullptr));
+      resident_prepare(S->res, m, mixed, S->two_level() ? &S->coarse : nullptr);
       if (S->res.plan && permit.acquire(S->res.plan->G, st)) {
         ResidentSolve rs{S->vals.p, S->binv.p, fixed, S->g.p, S->dx.p, P.pcg_rtol, P.inner_rtol, P.pcg_max_iter,
                          P.max_refine, mixed, S->two_level() ? &S->coarse : nullptr};
