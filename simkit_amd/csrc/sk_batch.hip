@@ -1569,11 +1569,27 @@ int coarse_scratch(const sk_batch* B) {
 // faster one at every size tried (a step, lane per row against dealt evenly): 512 beams of 8 to 64 cells block-Jacobi
 // 77.1 / 44.0 ms, of 36 to 46 two-level 20.5 / 14.1, of 16 to 24 13.0 / 8.7, of 4 to 10 7.0 / 5.3, 64 beams of 4 to
 // 10 3.6 / 2.4, 2,048 of 4 to 10 20.7 / 16.2.
+bool even_launch(int block, int lanes, int lds) { return block == kEvenNT && lanes == 1 && lds; }
 bool pcg_even(const sk_batch* B, int block, int lanes, int lds) {
-  return B->even == 1 && block == kEvenNT && lanes == 1 && lds;
+  return B->even == 1 && even_launch(block, lanes, lds);
 }
-// Before the first launch (and never within a captured one): decides whether
-// the evenly dealt PCG can serve the batch and allocates what it streams.
+// Gives back what prepare_even allocated, and the captured graph, which may hold its addresses.
+void drop_even(sk_batch* B) {
+  (void)hipStreamSynchronize(B->st);
+  if (B->exec) (void)hipGraphExecDestroy(B->exec);
+  if (B->graph) (void)hipGraphDestroy(B->graph);
+  B->exec = nullptr;
+  B->graph = nullptr;
+  B->even = -1;
+  B->even_vals.release();
+  B->even_word.release();
+  B->even_pos.release();
+  B->even_order.release();
+  B->even_slot0.release();
+}
+// Before the first launch of its shape (and never within a captured one):
+// decides whether the evenly dealt PCG can serve the batch and allocates what it
+// streams, a second copy of the matrix values.
 int prepare_even(sk_batch* B) {
   if (B->even >= 0) return SK_OK;
   B->even = 0;
@@ -1597,10 +1613,8 @@ int prepare_even(sk_batch* B) {
   if (B->even_vals.alloc(9 * slots) || B->even_word.alloc(slots) || B->even_pos.alloc(m->nblk) ||
       B->even_order.upload(order) || B->even_slot0.upload(slot0)) {
     (void)hipGetLastError();  // no memory for it: the lane-per-row kernel needs none
-    for (DevBuf<int32_t>* b : {&B->even_order, &B->even_pos}) b->release();
-    B->even_vals.release();
-    B->even_word.release();
-    B->even_slot0.release();
+    drop_even(B);
+    B->even = 0;
     return SK_OK;
   }
   SK_HIP_CHECK(hipMemsetAsync(B->even_vals.p, 0, B->even_vals.n * sizeof(float), B->st));  // slots without a block
@@ -2159,7 +2173,7 @@ int sk_batch_step(sk_batch* B, const double* x_curr, const double* x_prev, const
   SK_HIP_CHECK(hipEventRecord(B->ev_in, caller));
   SK_HIP_CHECK(hipStreamWaitEvent(B->st, B->ev_in, 0));
   const int block = batch_block(B), lanes = batch_lanes(B), lds = batch_lds(B);
-  SK_TRY(prepare_even(B));
+  if (even_launch(block, lanes, lds)) SK_TRY(prepare_even(B));
   SK_TRY(start_step(B, x_curr, x_prev, x_bc));
   if (B->coarse() && (!B->coarse_built || (B->coarse_period > 0 && B->steps_since_coarse >= B->coarse_period))) {
     SK_TRY(build_coarse(B, pcg_even(B, block, lanes, lds)));
@@ -2213,13 +2227,9 @@ int sk_batch_step(sk_batch* B, const double* x_curr, const double* x_prev, const
 int sk_batch_set_coarse(sk_batch* B, const double* X, int agg_rows, int period) {
   SK_REQUIRE(B, "sk_batch_set_coarse: null batch");
   SK_REQUIRE(period >= 0, "sk_batch_set_coarse: period must be >= 0");
-  if (B->exec) (void)hipGraphExecDestroy(B->exec);
-  if (B->graph) (void)hipGraphDestroy(B->graph);
-  B->exec = nullptr;
-  B->graph = nullptr;
+  drop_even(B);  // the coarse scratch changes what fits
   B->agg_rows = B->n_agg = B->max_agg = B->max_nc = 0;
   B->coarse_built = false;
-  B->even = -1;  // the coarse scratch changes what fits
   for (DevBuf<float>* b : {&B->cdv, &B->ctm, &B->einv}) b->release();
   for (DevBuf<int32_t>* b : {&B->cagg0, &B->ccol, &B->cagg_prob, &B->cadj_ptr, &B->cadj, &B->cnq}) b->release();
   B->einv_off.release();
@@ -2370,6 +2380,7 @@ int sk_batch_autotune(sk_batch* B, const double* x_curr, const double* x_prev, c
   B->prm.block = bb;
   B->prm.lanes = bl;
   B->prm.lds = bd;
+  if (!even_launch(bb, bl, bd)) drop_even(B);
   *block_out = bb;
   *lanes_out = bl;
   if (lds_out) *lds_out = bd;
