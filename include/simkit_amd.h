@@ -32,7 +32,7 @@ typedef void* sk_stream_t; /* hipStream_t */
 enum sk_status {
   SK_OK = 0,
   SK_ERR_INVALID = -1,
-  SK_ERR_HIP = -2,
+  SK_ERR_HIP = -2,           /* a HIP call failed, or memory (device or host) ran out */
   SK_ERR_LS_FAIL = -3,       /* Armijo search found no step (backtracking_line_search.py:66-67 returns t=0) */
   SK_ERR_PCG_BREAKDOWN = -4, /* p^T A p <= 0: system not positive definite */
   SK_ERR_PCG_MAXIT = -5,     /* PCG hit its iteration limit before rtol */

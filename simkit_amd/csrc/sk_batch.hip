@@ -1587,11 +1587,9 @@ void drop_even(sk_batch* B) {
   B->even_order.release();
   B->even_slot0.release();
 }
-// Before the first launch of its shape (and never within a captured one):
-// decides whether the evenly dealt PCG can serve the batch and allocates what it
-// streams, a second copy of the matrix values.
-int prepare_even(sk_batch* B) {
-  if (B->even >= 0) return SK_OK;
+// Decides whether the evenly dealt PCG can serve the batch and allocates what
+// it streams, a second copy of the matrix values.
+int build_even(sk_batch* B) {
   B->even = 0;
   if (!pcg_lds_fits(B)) return SK_OK;
   std::vector<int32_t> vs(B->P + 1), order(B->P);
@@ -1611,12 +1609,8 @@ int prepare_even(sk_batch* B) {
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return blocks(x) > blocks(y); });
   const sk_mesh* m = B->mesh;
   if (B->even_vals.alloc(9 * slots) || B->even_word.alloc(slots) || B->even_pos.alloc(m->nblk) ||
-      B->even_order.upload(order) || B->even_slot0.upload(slot0)) {
-    (void)hipGetLastError();  // no memory for it: the lane-per-row kernel needs none
-    drop_even(B);
-    B->even = 0;
-    return SK_OK;
-  }
+      B->even_order.upload(order) || B->even_slot0.upload(slot0))
+    return SK_ERR_HIP;
   SK_HIP_CHECK(hipMemsetAsync(B->even_vals.p, 0, B->even_vals.n * sizeof(float), B->st));  // slots without a block
   SK_HIP_CHECK(hipMemsetAsync(B->even_word.p, 0, B->even_word.n * sizeof(uint16_t), B->st));
   even_map_kernel<<<grid_for(m->nblk), kBlock, 0, B->st>>>(m->nblk, m->brow.p, m->bcol.p, m->bptr.p, B->pid.p,
@@ -1624,6 +1618,14 @@ int prepare_even(sk_batch* B) {
   SK_HIP_CHECK(hipGetLastError());
   B->even = 1;
   return SK_OK;
+}
+// The same before the first launch of its shape (and never within a captured one); without memory for it the
+// lane-per-row kernel, which needs none, keeps the batch.
+void prepare_even(sk_batch* B) {
+  if (B->even >= 0 || no_throw([&] { return build_even(B); }) == SK_OK) return;
+  (void)hipGetLastError();
+  drop_even(B);
+  B->even = 0;
 }
 
 int launch_pcg(const sk_batch* B, const BatchArgs& a, int block, int lanes, int lds) {
@@ -2173,7 +2175,7 @@ int sk_batch_step(sk_batch* B, const double* x_curr, const double* x_prev, const
   SK_HIP_CHECK(hipEventRecord(B->ev_in, caller));
   SK_HIP_CHECK(hipStreamWaitEvent(B->st, B->ev_in, 0));
   const int block = batch_block(B), lanes = batch_lanes(B), lds = batch_lds(B);
-  if (even_launch(block, lanes, lds)) SK_TRY(prepare_even(B));
+  if (even_launch(block, lanes, lds)) prepare_even(B);
   SK_TRY(start_step(B, x_curr, x_prev, x_bc));
   if (B->coarse() && (!B->coarse_built || (B->coarse_period > 0 && B->steps_since_coarse >= B->coarse_period))) {
     SK_TRY(build_coarse(B, pcg_even(B, block, lanes, lds)));
@@ -2338,7 +2340,7 @@ int sk_batch_autotune(sk_batch* B, const double* x_curr, const double* x_prev, c
   hipStream_t caller = as_stream(s);
   SK_HIP_CHECK(hipEventRecord(B->ev_in, caller));
   SK_HIP_CHECK(hipStreamWaitEvent(B->st, B->ev_in, 0));
-  SK_TRY(prepare_even(B));
+  prepare_even(B);
   // The first Newton system of a step: gradient, Hessian, gather.
   SK_TRY(start_step(B, x_curr, x_prev, x_bc));
   if (B->coarse() && !B->coarse_built) SK_TRY(build_coarse(B, false));

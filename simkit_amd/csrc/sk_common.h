@@ -48,6 +48,21 @@ void set_error(const std::string& msg);
     if (_s != SK_OK) return _s;                                                       \
   } while (0)
 
+// f(), which returns a status; an exception of the host code (no memory)
+// becomes one, since none may leave a C entry point or a host thread.
+template <typename F>
+int no_throw(F&& f) {
+  try {
+    return f();
+  } catch (...) {
+    try {
+      set_error("out of host memory");
+    } catch (...) {
+    }
+    return SK_ERR_HIP;
+  }
+}
+
 constexpr int kWave = 64;
 constexpr int kBlock = 256;
 

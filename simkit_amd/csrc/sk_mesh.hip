@@ -16,8 +16,8 @@
 #include "sk_resident.h"
 
 #include <algorithm>
+#include <exception>
 #include <numeric>
-#include <system_error>
 #include <thread>
 
 namespace sk {
@@ -800,16 +800,27 @@ static int build_mesh(const int32_t* T, int64_t nv, int64_t nt, sk_mesh* m) {
   const int nth = host_threads(nt);
   std::vector<std::vector<int32_t>> cols(nth);
   auto ranges = [&](auto&& fn) {
+    std::vector<std::exception_ptr> failed(nth);  // a thread must not end by an exception
+    auto run = [&](int k) {
+      try {
+        fn(k, nv * k / nth, nv * (k + 1) / nth);
+      } catch (...) {
+        failed[k] = std::current_exception();
+      }
+    };
     std::vector<std::thread> pool;
+    pool.reserve(nth);
     for (int k = 1; k < nth; ++k) {
       try {
-        pool.emplace_back([&fn, k, nv, nth] { fn(k, nv * k / nth, nv * (k + 1) / nth); });
-      } catch (const std::system_error&) {  // no thread to be had: here, then
-        fn(k, nv * k / nth, nv * (k + 1) / nth);
+        pool.emplace_back(run, k);
+      } catch (...) {  // no thread to be had: here, then
+        run(k);
       }
     }
-    fn(0, (int64_t)0, nv / nth);
+    run(0);
     for (auto& t : pool) t.join();
+    for (auto& e : failed)
+      if (e) std::rethrow_exception(e);
   };
   ranges([&](int k, int64_t v0, int64_t v1) {
     std::vector<int32_t> seen(nv, -1), nb;
@@ -1055,8 +1066,11 @@ int sk_mesh_create(const int32_t* T_host, const double* D, int64_t nv, int64_t n
   *out = nullptr;
   SK_REQUIRE(nv > 0 && nt > 0, "sk_mesh_create: empty mesh");
   SK_REQUIRE(T_host && D, "sk_mesh_create: null T or D");
-  sk_mesh* m = new sk_mesh();
-  int s = build_mesh(T_host, nv, nt, m);
+  sk_mesh* m = nullptr;
+  int s = no_throw([&] {
+    m = new sk_mesh();
+    return build_mesh(T_host, nv, nt, m);
+  });
   if (s == SK_OK) {
     aos_to_soa_kernel<<<grid_for(nt), kBlock>>>(D, nt, m->D.p);
     hipError_t e = hipGetLastError();
@@ -1078,10 +1092,12 @@ int sk_sell_order(const int32_t* T, int64_t nv, int64_t nt, int32_t* order) {
   SK_REQUIRE(T && order, "sk_sell_order: null argument");
   SK_REQUIRE(nv > 0 && nt > 0, "sk_sell_order: empty mesh");
   for (int64_t k = 0; k < 4 * nt; ++k) SK_REQUIRE(T[k] >= 0 && T[k] < nv, "sk_sell_order: tet index out of range");
-  std::vector<int32_t> deg;
-  vertex_degrees(T, nv, nt, deg);
-  degree_order(deg, order);
-  return SK_OK;
+  return no_throw([&] {
+    std::vector<int32_t> deg;
+    vertex_degrees(T, nv, nt, deg);
+    degree_order(deg, order);
+    return (int)SK_OK;
+  });
 }
 
 int sk_mesh_destroy(sk_mesh* m) {

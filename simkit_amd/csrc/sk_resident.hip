@@ -1694,7 +1694,7 @@ void resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace
   R.tried = true;
   R.plan.reset();
   R.two.reset();
-  if (prepare(R, m, fp32, coarse) == SK_OK) return;
+  if (no_throw([&] { return prepare(R, m, fp32, coarse); }) == SK_OK) return;
   // no memory for it: the launches need none of this
   (void)hipGetLastError();
   R.plan.reset();
@@ -1822,8 +1822,8 @@ static void bisect(const double* X, const std::vector<float>& w, std::vector<int
   bisect(X, w, idx, cut, hi, gm, g1, ptr);
 }
 
-int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
-                  int* n_parts, int32_t* part_ptr) {
+static int part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
+                      int* n_parts, int32_t* part_ptr) {
   SK_REQUIRE(X && T && order && n_parts && part_ptr, "sk_part_order: null argument");
   SK_REQUIRE(precision == SK_PREC_FP64 || precision == SK_PREC_MIXED, "sk_part_order: bad precision");
   SK_REQUIRE(nv > 0 && nt > 0, "sk_part_order: empty mesh");
@@ -1852,6 +1852,11 @@ int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int
   std::copy(idx.begin(), idx.end(), order);
   *n_parts = G;
   return SK_OK;
+}
+
+int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
+                  int* n_parts, int32_t* part_ptr) {
+  return no_throw([&] { return part_order(X, T, nv, nt, precision, order, n_parts, part_ptr); });
 }
 
 }  // extern "C"

@@ -2058,7 +2058,10 @@ int sk_sim_set_parts(sk_sim* S, int n, const int32_t* ptr) {
   SK_REQUIRE(n >= 0 && n <= kResMaxParts, "sk_sim_set_parts: 0..256 parts");
   for (int g = 0; g < n; ++g) SK_REQUIRE(ptr[g] < ptr[g + 1], "sk_sim_set_parts: parts must be non-empty ranges");
   SK_REQUIRE(n == 0 || (ptr[0] == 0 && ptr[n] == S->mesh->nv), "sk_sim_set_parts: parts must cover the vertices");
-  S->res.parts.assign(ptr, ptr + (n ? n + 1 : 0));
+  SK_TRY(no_throw([&] {
+    S->res.parts.assign(ptr, ptr + (n ? n + 1 : 0));
+    return (int)SK_OK;
+  }));
   S->res.plan.reset();
   S->res.tried = false;
   return SK_OK;
