@@ -22,6 +22,8 @@ constexpr int kResMaxTier = 4;        // blocks per thread in LDS, and streamed 
 // With the coarse correction: its values in flight leave fewer registers for blocks.
 constexpr int kResTwoKR64 = 5, kResTwoKR32 = 9, kResTwoTier = 6;
 constexpr int kResMaxPieces = 8;      // aggregates a workgroup's rows reach into, at most (one wave serves them)
+constexpr double kResWait = 2.0;      // seconds a workgroup waits for another before the run is given up
+constexpr uint32_t kResMaxEpoch = 0x70000000u;  // exchanges are numbered anew from a run that starts past this one
 
 // Cut of a mesh's rows into contiguous ranges, one per workgroup, with the
 // index data the kernel reads (built once per mesh and cut on the host).
@@ -70,6 +72,8 @@ struct ResidentState {
   std::unique_ptr<ResidentTwo> two;      // with a coarse space
   bool tried = false;                    // plan has been looked for
   bool off = false;                      // a run gave up waiting: launches only from now on
+  int64_t runs = 0, launch_solves = 0, gave_up = 0;  // solves by this kernel and by launches; runs given up
+  double wait = kResWait;                // 0: a run of several workgroups gives up at once
   DevBuf<uint64_t> slots, zx, xx;
   DevBuf<char> stream;
   DevBuf<int> abort_flag;
@@ -118,6 +122,8 @@ void resident_prepare(ResidentState& R, sk_mesh* m, bool fp32, const CoarseSpace
 // Enqueues the run (without waiting); the result is in R.host once the stream
 // has been synchronized.
 int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st);
+// Has the next run number its exchanges from `epoch` on, with all words cleared.
+int resident_set_epoch(ResidentState& R, uint32_t epoch);
 // Number of neighbour vertices (itself included) of every vertex.
 void vertex_degrees(const int32_t* T, int64_t nv, int64_t nt, std::vector<int32_t>& deg);
 // The vertices by descending degree, ties in index order (sk_sell_order).

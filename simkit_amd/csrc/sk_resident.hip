@@ -74,6 +74,7 @@ struct ResidentArgs {
   int max_rows, max_local, max_halo;
   double rtol2, inner_rtol2;
   int max_iter, max_refine;
+  long long wait_ticks;  // bound of a wait (Poll)
   // two-level preconditioner (ResidentTwo, CoarseSpace)
   int ld, n_agg, max_need;
   double shift;
@@ -117,18 +118,18 @@ __device__ __forceinline__ void put_word48(uint64_t* p, uint32_t epoch, uint64_t
 }
 __device__ __forceinline__ bool tagged48(uint64_t w, uint32_t epoch) { return (uint32_t)(w >> 48) == (epoch & 0xffffu); }
 
-// Ends a poll that has lasted kPollTicks (about two seconds of the 100 MHz
-// clock) or that another workgroup has ended: every wait is bounded, and the
-// host then solves by launches.
-constexpr long long kPollTicks = 200000000ll;
+// Ends a poll that has lasted `ticks` (of the 100 MHz clock) or that another
+// workgroup has ended: every wait is bounded, and the host then solves by
+// launches.
+constexpr double kTicksPerSecond = 1e8;
 struct Poll {
   int n = 0;
   long long t0 = 0;
-  __device__ __forceinline__ bool give_up(const int* abort_flag) {
+  __device__ __forceinline__ bool give_up(const int* abort_flag, long long ticks) {
     if ((++n & 255) != 0) return false;
     const long long now = wall_clock64();
     if (t0 == 0) t0 = now;
-    return now - t0 > kPollTicks || __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return now - t0 > ticks || __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
   }
 };
 
@@ -159,6 +160,7 @@ struct Meet {
   int G;
   int parity;
   const int* abort_flag;
+  long long ticks;
   const int32_t* halo;  // [H] in LDS
   int H;
 
@@ -231,7 +233,7 @@ struct Meet {
           dest[(t + k * NT) / VS * VW + hw] = (uint32_t)b[k];
           need &= ~(1u << (NS + k));
         }
-      if (need && poll.give_up(abort_flag)) {
+      if (need && poll.give_up(abort_flag, ticks)) {
         *bad = 1;
         break;
       }
@@ -242,7 +244,7 @@ struct Meet {
         const uint64_t* p = words + (size_t)halo[j / VS] * VS + hw;
         uint64_t w = get_word(p);
         while (!tagged(w, epoch)) {
-          if (poll.give_up(abort_flag)) {
+          if (poll.give_up(abort_flag, ticks)) {
             *bad = 1;
             break;
           }
@@ -381,7 +383,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   int32_t* NE = reinterpret_cast<int32_t*>(W2 + tl.end);               // [max_need] the list's aggregates
   uint16_t* LN = reinterpret_cast<uint16_t*>(NE + a.max_need);         // [max_local]
   T* S = a.stream + (size_t)me * a.KS * 9 * NT;
-  if (t == 0) s_bad = 0;
+  if (t == 0) s_bad = a.G > 1 && a.wait_ticks <= 0;  // a run that must not wait ends at its first meeting
 
   // the thread's blocks, their columns' byte offsets and which of them end a row
   T A[KR][9];
@@ -708,7 +710,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
 #pragma unroll
         for (int i = 0; i < N; ++i)
           if ((need >> i & 1) && tagged48(u[i], epoch)) need &= ~(1u << i);
-        if (need && poll.give_up(a.abort_flag)) {
+        if (need && poll.give_up(a.abort_flag, a.wait_ticks)) {
           s_bad = 1;
           break;
         }
@@ -807,7 +809,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       const uint64_t* p = a.uwords + (uint32_t)(NE[j / kAggWords] * kAggWords + j % kAggWords);
       uint64_t w = get_word(p);
       while (!tagged48(w, epoch)) {
-        if (poll.give_up(a.abort_flag)) {
+        if (poll.give_up(a.abort_flag, a.wait_ticks)) {
           s_bad = 1;
           break;
         }
@@ -860,7 +862,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     direction(R + j, B, r, T(0));
   }
 
-  Meet<NT> meet{s_red, s_tot, &s_bad, a.slots, a.G, 0, a.abort_flag, HX, H};
+  Meet<NT> meet{s_red, s_tot, &s_bad, a.slots, a.G, 0, a.abort_flag, a.wait_ticks, HX, H};
   uint32_t epoch = a.epoch;
   int iter = 0, done = 0, refines = 0;
   double tol2 = 0.0, target = 0.0;
@@ -1316,13 +1318,13 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   }
 }
 
-__global__ void resident_clear_kernel(int64_t n, uint64_t* p) {
+__global__ void resident_fill_kernel(int64_t n, uint64_t* p, uint64_t word) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
+  if (i < n) p[i] = word;
 }
 
-int clear_words(DevBuf<uint64_t>& b, hipStream_t st) {
-  if (b.n) resident_clear_kernel<<<grid_for((int64_t)b.n), kBlock, 0, st>>>((int64_t)b.n, b.p);
+int fill_words(DevBuf<uint64_t>& b, uint64_t word, hipStream_t st) {
+  if (b.n) resident_fill_kernel<<<grid_for((int64_t)b.n), kBlock, 0, st>>>((int64_t)b.n, b.p, word);
   SK_HIP_CHECK(hipGetLastError());
   return SK_OK;
 }
@@ -1711,7 +1713,8 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
                     (const T*)s.binv, s.fixed, s.g, s.dx, p.halo_ptr.p, p.hvert.p, p.halo.p, p.exp0.p, p.exslot.p, R.slots.p, R.zx.p,
                     (uint32_t)(R.zx.n / 2),
                     R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
-                    p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
+                    p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine,
+                    (long long)(R.wait * kTicksPerSecond)};
   if (kTwo) {
     const CoarseSpace& C = *s.coarse;
     const ResidentTwo& w = *R.two;
@@ -1741,16 +1744,26 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
   return SK_OK;
 }
 
+// Every word tagged with `epoch`, so that none belongs to a later exchange.
+static int clear_all_words(ResidentState& R, uint32_t epoch, hipStream_t st) {
+  for (DevBuf<uint64_t>* b : {&R.slots, &R.zx, &R.xx}) SK_TRY(fill_words(*b, (uint64_t)epoch << 32, st));
+  if (R.two)
+    for (DevBuf<uint64_t>* b : {&R.two->cwords, &R.two->uwords}) SK_TRY(fill_words(*b, (uint64_t)epoch << 48, st));
+  return SK_OK;
+}
+
+int resident_set_epoch(ResidentState& R, uint32_t epoch) {
+  SK_TRY(clear_all_words(R, epoch, nullptr));
+  SK_HIP_CHECK(hipDeviceSynchronize());
+  R.epoch = epoch;
+  *R.host = ResidentResult{0, 0, 0, 0, epoch};
+  return SK_OK;
+}
+
 int resident_launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStream_t st) {
   if (R.host->epoch > R.epoch) R.epoch = R.host->epoch;
-  if (R.epoch > 0x70000000u) {  // tags start over long before they wrap
-    SK_TRY(clear_words(R.slots, st));
-    SK_TRY(clear_words(R.zx, st));
-    SK_TRY(clear_words(R.xx, st));
-    if (R.two) {
-      SK_TRY(clear_words(R.two->cwords, st));
-      SK_TRY(clear_words(R.two->uwords, st));
-    }
+  if (R.epoch > kResMaxEpoch) {  // tags start over long before they wrap
+    SK_TRY(clear_all_words(R, 0, st));
     R.epoch = 0;
   }
   *R.host = ResidentResult{0, 0, 0, 0, R.epoch};

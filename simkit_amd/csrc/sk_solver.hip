@@ -21,6 +21,7 @@
 #include "sk_coarse.h"
 #include "sk_resident.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace sk {
@@ -2067,6 +2068,27 @@ int sk_sim_set_parts(sk_sim* S, int n, const int32_t* ptr) {
   return SK_OK;
 }
 
+int sk_sim_solver_info(const sk_sim* S, int* workgroups, int64_t* resident_solves, int64_t* launch_solves,
+                       int64_t* gave_up, int64_t* exchanges) {
+  SK_REQUIRE(S, "sk_sim_solver_info: null simulator");
+  const ResidentState& R = S->res;
+  if (workgroups) *workgroups = R.plan && S->may_be_resident() ? R.plan->G : 0;
+  if (resident_solves) *resident_solves = R.runs;
+  if (launch_solves) *launch_solves = R.launch_solves;
+  if (gave_up) *gave_up = R.gave_up;
+  if (exchanges) *exchanges = R.host ? std::max(R.epoch, R.host->epoch) : 0;
+  return SK_OK;
+}
+
+int sk_sim_resident_hook(sk_sim* S, double wait_seconds, int64_t exchanges) {
+  SK_REQUIRE(S, "sk_sim_resident_hook: null simulator");
+  SK_REQUIRE(wait_seconds >= 0.0 && wait_seconds <= kResWait, "sk_sim_resident_hook: the wait must be in [0, 2] s");
+  SK_REQUIRE(exchanges >= 0 && exchanges <= (int64_t)kResMaxEpoch, "sk_sim_resident_hook: exchange number out of range");
+  S->res.wait = wait_seconds;
+  if (S->may_be_resident()) resident_prepare(S->res, S->mesh, S->mixed(), S->two_level() ? &S->coarse : nullptr);
+  return S->res.plan ? resident_set_epoch(S->res, (uint32_t)exchanges) : SK_OK;
+}
+
 int sk_sim_coarse_info(const sk_sim* S, int* n_agg, int* nc, int* built, double* build_ms) {
   SK_REQUIRE(S, "sk_sim_coarse_info: null simulator");
   if (n_agg) *n_agg = S->coarse.n_agg;
@@ -2187,6 +2209,7 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
     }
   launches:
     if (!resident) {
+    ++S->res.launch_solves;
     // The RHS is negated in place.
     axpy_kernel<<<grid_for(n3), kBlock, 0, st>>>(n3, -2.0, S->g.p, S->g.p);
     // The FP64 solve is not waited for: the slope's launches follow it in the
@@ -2207,9 +2230,11 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
       const volatile ResidentResult* h = S->res.host;
       if (h->aborted) {  // the run gave up waiting for a workgroup: solve by launches, now and later
         S->res.off = true;
+        ++S->res.gave_up;
         resident = false;
         goto launches;
       }
+      ++S->res.runs;
       it = h->iter;
       done = h->done;
       refines = h->refines;

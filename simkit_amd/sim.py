@@ -189,6 +189,14 @@ class BackwardEulerSim:
         return {"aggregates": n.value, "coarse_unknowns": nc.value, "built": bool(built.value),
                 "build_ms": ms.value, "vertices_per_aggregate": self.coarse_vertices}
 
+    def solver_info(self):
+        """How the Newton systems have been solved: workgroups of the resident PCG (0: the next solve goes by
+        launches), solves by it and by launches, and its runs that were given up (sk_sim_solver_info)."""
+        wg, n = ctypes.c_int(), [ctypes.c_int64() for _ in range(4)]
+        _lib.call("sk_sim_solver_info", self._h, ctypes.byref(wg), *[ctypes.byref(v) for v in n])
+        return {"workgroups": wg.value, "resident_solves": n[0].value, "launch_solves": n[1].value,
+                "gave_up": n[2].value, "exchanges": n[3].value}
+
     def step(self, x_curr, x_prev, x_bc=None, out=None):
         """One BE step on device tensors (3nv,). Returns (x_next, info dict)."""
         info = _lib.SkStepInfo()

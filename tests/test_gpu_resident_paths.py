@@ -1,0 +1,114 @@
+"""Which path a solve takes, and the resident PCG's rare ones: every mesh of the two comparison tests runs where it is
+meant to (a comparison of the launches with themselves would pass), a run that gives up is solved by launches, exchange
+numbers start over, and runs of several simulators share the device."""
+import ctypes
+import threading
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+import test_gpu_resident as bj  # noqa: E402
+import test_gpu_resident_two as two  # noqa: E402
+
+
+def _hook(sim, wait=2.0, exchanges=0):
+    from simkit_amd import _lib
+    _lib.call("sk_sim_resident_hook", sim._h, wait, exchanges)
+
+
+def _sim(n, precision="fp64", material="snh", per_agg=0, chunk=0, **kw):
+    if per_agg:
+        return two._sim(n, precision, material, per_agg, chunk, **kw)
+    from simkit_amd.sim import BackwardEulerSim
+    from simkit_amd.ympr_to_lame import ympr_to_lame
+    X, T, fixed = bj._box(n, 3)
+    mu, lam = ympr_to_lame(1e6, 0.45)
+    return BackwardEulerSim(X, T, mu, lam, rho=1000.0, material=material, fixed_vertices=fixed, gravity=-9.8,
+                            precision=precision, pcg_chunk=chunk, **kw)
+
+
+@pytest.mark.parametrize("n,precision,material,renumber", bj.CASES)
+def test_block_jacobi_cases_run_resident(n, precision, material, renumber):
+    sim = _sim(n, precision, material, renumber=renumber)
+    _, info = sim.step(sim.X_dev, sim.X_dev)
+    print(n, sim.solver_info())
+    got = sim.solver_info()
+    assert got["workgroups"] > 0 and got["gave_up"] == 0
+    assert (got["resident_solves"], got["launch_solves"]) == (info["newton_iters"], 0)
+    sim = _sim(n, precision, material, chunk=8, renumber=renumber)
+    _, info = sim.step(sim.X_dev, sim.X_dev)
+    got = sim.solver_info()
+    assert got["workgroups"] == 0 and (got["resident_solves"], got["launch_solves"]) == (0, info["newton_iters"])
+
+
+# FP64 at 49 x 48 x 47 cells: vectors, halo and the coarse space together exceed the LDS
+TWO_LAUNCHES = {((49, 48, 47), "fp64", "snh", 216)}
+
+
+@pytest.mark.parametrize("n,precision,material,per_agg", two.CASES)
+def test_two_level_cases_run_where_they_are_meant_to(n, precision, material, per_agg):
+    sim = _sim(n, precision, material, per_agg)
+    _, info = sim.step(sim.X_dev, sim.X_dev)
+    got, k = sim.solver_info(), info["newton_iters"]
+    assert got["gave_up"] == 0
+    resident = (n, precision, material, per_agg) not in TWO_LAUNCHES
+    assert (got["resident_solves"], got["launch_solves"]) == ((k, 0) if resident else (0, k)), got
+
+
+def test_two_level_fp64_with_streamed_blocks_matches_the_launches():
+    """To the bounds of test_gpu_resident_two, at a size with more blocks a thread than its registers hold (8.2 on average
+    against 5)."""
+    out = []
+    for chunk in (0, 4):
+        sim = _sim((42, 43, 44), "fp64", "snh", 216, chunk)
+        out.append(sim.rollout(2))
+        info = sim.solver_info()
+        assert (info["resident_solves"] > 0, info["launch_solves"] > 0) == (chunk == 0, chunk != 0), info
+    (k0, i0), (k1, i1) = out
+    for s in (1, 2):
+        assert np.abs(k0[s] - k1[s]).max() / np.abs(k1[s]).max() < 1e-10
+        a, b = i0[s - 1], i1[s - 1]
+        assert a["newton_iters"] == b["newton_iters"]
+        assert abs(a["pcg_iters"] - b["pcg_iters"]) <= 0.03 * b["pcg_iters"] + 4, (a, b)
+
+
+FORMS = [("fp64", 0), ("mixed", 0), ("fp64", 100), ("mixed", 100)]
+
+
+@pytest.mark.parametrize("precision,per_agg", FORMS)
+def test_a_run_that_gives_up_is_solved_by_launches(precision, per_agg):
+    n = (14, 15, 13)
+    sim, ref = _sim(n, precision, per_agg=per_agg), _sim(n, precision, per_agg=per_agg, chunk=8)
+    _hook(sim, wait=0.0)
+    kept, infos = sim.rollout(2)
+    want, winfos = ref.rollout(2)
+    assert all(i["status"] == 0 for i in infos), infos
+    for s in (1, 2):  # the same launches; the chunk length only says how often the host looks
+        assert np.abs(kept[s] - want[s]).max() <= 1e-12 * np.abs(want[s]).max()
+        assert infos[s - 1]["pcg_iters"] == winfos[s - 1]["pcg_iters"]
+    got = sim.solver_info()
+    assert (got["resident_solves"], got["gave_up"], got["workgroups"]) == (0, 1, 0), got
+    assert got["launch_solves"] == sum(i["newton_iters"] for i in infos)
+    one = _sim((1, 1, 1), precision, per_agg=per_agg)  # one workgroup: nobody to wait for
+    _hook(one, wait=0.0)
+    _, info = one.step(one.X_dev, one.X_dev)
+    assert one.solver_info()["resident_solves"] == info["newton_iters"]
+
+
+@pytest.mark.parametrize("precision,per_agg", FORMS)
+@pytest.mark.parametrize("start", [0x70000000 - 40, 0x70000000, 65536 - 40, 65535])
+def test_exchange_numbers_start_over_and_wrap_their_tags(precision, per_agg, start):
+    """Past 0x70000000 the next run starts at 0 again; the two-level words carry the low 16 bits only."""
+    n = (11, 12, 10)
+    sim, ref = _sim(n, precision, per_agg=per_agg), _sim(n, precision, per_agg=per_agg)
+    _hook(sim, exchanges=start)
+    kept, infos = sim.rollout(3)
+    want, winfos = ref.rollout(3)
+    assert all(np.array_equal(kept[s], want[s]) for s in (1, 2, 3))
+    assert [i["pcg_iters"] for i in infos] == [i["pcg_iters"] for i in winfos]
+    got, total = sim.solver_info(), ref.solver_info()["exchanges"]
+    assert got["launch_solves"] == got["gave_up"] == 0
+    assert got["exchanges"] < total if start > 65536 else got["exchanges"] == start + total
