@@ -85,17 +85,20 @@ struct ResidentState {
 // Workgroups for a mesh of nv vertices and nblk blocks; 0: not eligible.
 int resident_parts(int64_t nv, int64_t nblk, bool fp32);
 
-// A block of `need` CUs of the current device for one resident run, held
-// until the run has ended: runs of one process that overlap on one GPU never
-// ask for more workgroups together than can be resident at once.
+// The CUs of the current device that one resident run of `parts` workgroups
+// needs, held until the run has ended: runs of one process that overlap on one
+// GPU never ask for more workgroups together than can be resident at once, on
+// any XCD. (Other processes are not seen. Where one holds CUs for long, a run
+// waits out kResWait, is solved by launches, and so are its simulator's later
+// ones.)
 class ResidentPermit {
  public:
   ResidentPermit() = default;
   ~ResidentPermit() { release(); }
   ResidentPermit(const ResidentPermit&) = delete;
   ResidentPermit& operator=(const ResidentPermit&) = delete;
-  // False when the device (or the stream's CU mask) has fewer than `need` CUs.
-  bool acquire(int need, hipStream_t st);
+  // False when the device has fewer CUs than that, or the stream's CU mask leaves out some.
+  bool acquire(int parts, hipStream_t st);
   void release();
 
  private:

@@ -1354,15 +1354,17 @@ ResidentState::~ResidentState() {
   if (host) (void)hipHostFree(host);
 }
 
-bool ResidentPermit::acquire(int need, hipStream_t st) {
+bool ResidentPermit::acquire(int parts, hipStream_t st) {
   int dev = -1;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
-  // a stream restricted to some CUs
+  // Workgroups are dealt to the XCDs in turn, so one XCD takes up to an eighth, rounded up: charged for that on every
+  // XCD, the runs that hold a permit fit each of them, not only the chip as a whole.
+  const int need = (parts + 7) / 8 * 8;
   uint32_t mask[16] = {};
+  int allowed = -1;
   if (hipExtStreamGetCUMask(st, 16, mask) == hipSuccess) {
-    int n = 0;
-    for (uint32_t w : mask) n += __builtin_popcount(w);
-    if (n < need) return false;
+    allowed = 0;
+    for (uint32_t w : mask) allowed += __builtin_popcount(w);
   } else {
     (void)hipGetLastError();
   }
@@ -1372,7 +1374,8 @@ bool ResidentPermit::acquire(int need, hipStream_t st) {
     int n = 0;
     P.cus = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess ? n : 0;
   }
-  if (need > P.cus) return false;
+  // A stream restricted to some CUs: what it leaves on each XCD, and which other streams share it, is not known here.
+  if (need > P.cus || (allowed >= 0 && allowed < P.cus)) return false;
   P.cv.wait(lock, [&] { return P.used + need <= P.cus; });
   P.used += need;
   dev_ = dev;

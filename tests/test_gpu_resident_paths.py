@@ -112,3 +112,62 @@ def test_exchange_numbers_start_over_and_wrap_their_tags(precision, per_agg, sta
     got, total = sim.solver_info(), ref.solver_info()["exchanges"]
     assert got["launch_solves"] == got["gave_up"] == 0
     assert got["exchanges"] < total if start > 65536 else got["exchanges"] == start + total
+
+
+def _hip():
+    """The HIP runtime that torch and the library have loaded."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64.so" in line)
+    return ctypes.CDLL(path)
+
+
+def test_a_stream_with_a_cu_mask_takes_the_launches():
+    """Half of the CUs: where its workgroups could run on each XCD is not known, so they must not wait for each other."""
+    hip, stream = _hip(), ctypes.c_void_p()
+    sim, ref = _sim((9, 8, 10)), _sim((9, 8, 10), chunk=8)
+    torch.cuda.synchronize()
+    mask = (ctypes.c_uint32 * 8)(*[0xFFFFFFFF] * 4 + [0] * 4)
+    assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(stream), 8, mask) == 0
+    try:
+        with torch.cuda.stream(torch.cuda.ExternalStream(stream.value)):
+            x1, info = sim.step(sim.X_dev, sim.X_dev)
+            torch.cuda.current_stream().synchronize()
+        want, _ = ref.step(ref.X_dev, ref.X_dev)
+        got = sim.solver_info()
+        assert (got["resident_solves"], got["launch_solves"], got["gave_up"]) == (0, info["newton_iters"], 0), got
+        assert (x1 - want).abs().max() <= 1e-12 * want.abs().max()
+        _, info = sim.step(sim.X_dev, sim.X_dev)  # and on an ordinary stream again resident
+        assert sim.solver_info()["resident_solves"] == info["newton_iters"]
+    finally:
+        assert hip.hipStreamDestroy(stream) == 0
+
+
+def test_runs_of_several_threads_share_the_device():
+    """Simulators stepped by threads of their own on streams of their own: cuts that fit the chip together and cuts that
+    need all of it, with workgroup counts that are no multiple of the eight XCDs among them. Nobody gives up, and every
+    trajectory is the one its simulator has alone."""
+    specs = [((23, 29, 31), "mixed", 216), ((13, 11, 12), "fp64", 100), ((24, 25, 23), "fp64", 0),
+             ((4, 40, 4), "fp64", 100), ((9, 5, 11), "mixed", 60)]
+    sims = [_sim(n, p, per_agg=a) for n, p, a in specs]
+    want = [_sim(n, p, per_agg=a).rollout(4)[0] for n, p, a in specs]
+    torch.cuda.synchronize()
+    kept, errors = [None] * len(sims), []
+
+    def run(k):
+        try:
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                kept[k] = sims[k].rollout(4)[0]
+                stream.synchronize()
+        except Exception as e:  # noqa: BLE001 (reported by the main thread)
+            errors.append((k, e))
+
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(len(sims))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for sim, got, ref in zip(sims, kept, want):
+        info = sim.solver_info()
+        assert info["gave_up"] == info["launch_solves"] == 0, info
+        assert all(np.array_equal(got[s], ref[s]) for s in range(1, 5))
