@@ -495,7 +495,8 @@ int sk_sell_order(const int32_t* T, int64_t nv, int64_t nt, int32_t* order);
  * bisection of X (host, nv x 3); part g is order[part_ptr[g] ..
  * part_ptr[g + 1]), by descending number of neighbours within it. part_ptr
  * holds up to 257 entries. n_parts = 0 (a mesh too large for one row per
- * thread): order is sk_sell_order's. precision: sk_precision. */
+ * thread, or with more blocks than a thread can hold): order is
+ * sk_sell_order's. precision: sk_precision. */
 int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int precision, int32_t* order,
                   int* n_parts, int32_t* part_ptr);
 /* The rows of the simulator's mesh as n contiguous ranges (ptr_host[n + 1],

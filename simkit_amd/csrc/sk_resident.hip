@@ -1861,6 +1861,17 @@ static int part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt,
   std::iota(idx.begin(), idx.end(), 0);
   bisect(X, w, idx, 0, nv, 0, G, part_ptr);
   part_ptr[G] = (int32_t)nv;
+  const bool fp32 = precision == SK_PREC_MIXED;
+  const int NT = fp32 ? kResNT32 : kResNT64;
+  for (int g = 0; g < G; ++g) {  // a part that build_plan will refuse: the launches' order then
+    int64_t nb = 0;
+    for (int32_t i = part_ptr[g]; i < part_ptr[g + 1]; ++i) nb += deg[idx[i]];
+    const int K = (int)((nb + NT - 1) / NT);
+    if (part_ptr[g + 1] - part_ptr[g] > NT || K > resident_kr(fp32, false, K) + 2 * kResMaxTier) {
+      degree_order(deg, order);
+      return SK_OK;
+    }
+  }
   for (int g = 0; g < G; ++g)
     std::sort(idx.begin() + part_ptr[g], idx.begin() + part_ptr[g + 1], [&](int32_t p, int32_t q) {
       return deg[p] != deg[q] ? deg[p] > deg[q] : p < q;

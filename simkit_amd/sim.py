@@ -27,6 +27,7 @@ from .gravity_force import gravity_force
 
 
 _COARSE_MAX = 4096  # coarse unknowns the library accepts (sk_sim_set_coarse)
+_RESIDENT_MAX = 256 * 512  # vertices the resident PCG serves at most: a thread each (sk_part_order)
 
 
 class BackwardEulerSim:
@@ -46,9 +47,10 @@ class BackwardEulerSim:
         raised as needed to keep the coarse space within the library's 4,096 unknowns; the coarse
         operator is formed from the first system solved). Both solve to pcg_rtol.
         renumber: the simulator numbers the vertices internally in the order its kernels read
-        them (two-level: aggregate by aggregate, so that each aggregate is a contiguous range;
-        block-Jacobi: boxes of the mesh, one per workgroup of the PCG kernel, sk_part_order);
-        states passed in and returned keep the caller's vertex order (the library permutes them in the
+        them. For the single-launch PCG: boxes of the mesh, one per workgroup (block-Jacobi, sk_part_order),
+        or aggregate by aggregate, each in index order (two-level). For the launches: by descending number of
+        neighbours (the sliced-ELL order, sk_sell_order; two-level: within each aggregate), so that the
+        SpMV's row stores are contiguous. States passed in and returned keep the caller's vertex order (the library permutes them in the
         step's first and last kernels, sk_sim_set_order).
         max_inverted: < 0 no limit; otherwise a step that ends with more elements of det F <= 0 reports
         status SK_ERR_INVERTED (info["inverted_elems"] always holds the count).
@@ -87,11 +89,25 @@ class BackwardEulerSim:
         # internal vertex order: order[t] = caller's vertex at internal position t
         self._order = self._pos = None
         parts = None
+        # whether the solves may run resident (the library's own rule, but for what only a plan can tell)
+        resident = (self.nv <= _RESIDENT_MAX and spmv_blocks == 0 and update_blocks == 0 and pcg_chunk == 0
+                    and not (pcg == "pipelined" and precision == "fp64" and preconditioner == "bjacobi"))
         if renumber:
             order = np.empty(self.nv, np.int32)
             Tc = np.ascontiguousarray(T, dtype=np.int32)
-            if preconditioner == "two_level":
-                order[:] = agg_order  # aggregate by aggregate, each in index order
+            if preconditioner == "two_level" and resident:
+                order[:] = agg_order
+            elif not resident:
+                # a step by launches takes longer in the boxes' order (pipelined 24^3 17.8 against 16.6 ms, a 40 x 30 x
+                # 35 box 37.7 / 37.0, two launches an iteration there 33.4 / 32.9, mixed 28.6 / 28.2) and in the
+                # aggregates' index order (two-level at 56^3, FP64 42.0 / 40.7, mixed 31.0 / 30.1)
+                _lib.call("sk_sell_order", Tc.ctypes.data_as(ctypes.c_void_p), int(self.nv), int(self.nt),
+                          order.ctypes.data_as(ctypes.c_void_p))
+                if preconditioner == "two_level":
+                    rank = np.empty(self.nv, np.int64)
+                    rank[order] = np.arange(self.nv)
+                    key = np.repeat(np.arange(len(agg_ptr) - 1, dtype=np.int64), np.diff(agg_ptr)) * self.nv
+                    order[:] = agg_order[np.argsort(key + rank[agg_order], kind="stable")]
             else:
                 Xc = np.ascontiguousarray(X, dtype=np.float64)
                 n_parts, ptr_ = ctypes.c_int(), np.empty(257, np.int32)

@@ -81,14 +81,19 @@ FORMS = [("fp64", 0), ("mixed", 0), ("fp64", 100), ("mixed", 100)]
 @pytest.mark.parametrize("precision,per_agg", FORMS)
 def test_a_run_that_gives_up_is_solved_by_launches(precision, per_agg):
     n = (14, 15, 13)
-    sim, ref = _sim(n, precision, per_agg=per_agg), _sim(n, precision, per_agg=per_agg, chunk=8)
+    # in one numbering the very same launches (two-level: the aggregates' vertices in another order, to the bounds of
+    # the comparison tests); the chunk length only says how often the host looks
+    kw = {"per_agg": per_agg} if per_agg else {"renumber": False}
+    tol, slack = (1e-10, 0.03) if per_agg else (1e-12, 0.0)
+    sim, ref = _sim(n, precision, **kw), _sim(n, precision, chunk=8, **kw)
     _hook(sim, wait=0.0)
     kept, infos = sim.rollout(2)
     want, winfos = ref.rollout(2)
     assert all(i["status"] == 0 for i in infos), infos
-    for s in (1, 2):  # the same launches; the chunk length only says how often the host looks
-        assert np.abs(kept[s] - want[s]).max() <= 1e-12 * np.abs(want[s]).max()
-        assert infos[s - 1]["pcg_iters"] == winfos[s - 1]["pcg_iters"]
+    for s in (1, 2):
+        a, b = infos[s - 1]["pcg_iters"], winfos[s - 1]["pcg_iters"]
+        assert np.abs(kept[s] - want[s]).max() <= tol * np.abs(want[s]).max()
+        assert abs(a - b) <= slack * b + (4 if slack else 0)
     got = sim.solver_info()
     assert (got["resident_solves"], got["gave_up"], got["workgroups"]) == (0, 1, 0), got
     assert got["launch_solves"] == sum(i["newton_iters"] for i in infos)
@@ -123,7 +128,7 @@ def _hip():
 def test_a_stream_with_a_cu_mask_takes_the_launches():
     """Half of the CUs: where its workgroups could run on each XCD is not known, so they must not wait for each other."""
     hip, stream = _hip(), ctypes.c_void_p()
-    sim, ref = _sim((9, 8, 10)), _sim((9, 8, 10), chunk=8)
+    sim, ref = _sim((9, 8, 10), renumber=False), _sim((9, 8, 10), chunk=8, renumber=False)
     torch.cuda.synchronize()
     mask = (ctypes.c_uint32 * 8)(*[0xFFFFFFFF] * 4 + [0] * 4)
     assert hip.hipExtStreamCreateWithCUMask(ctypes.byref(stream), 8, mask) == 0
