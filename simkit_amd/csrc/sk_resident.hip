@@ -86,12 +86,23 @@ struct ResidentArgs {
   uint64_t *cwords, *uwords;
 };
 
+// Dynamic LDS (bytes): everything but the matrix tiers and the coarse space, one tier block per thread, and where
+// the coarse space starts behind both. It holds 16-byte words.
+__host__ __device__ constexpr size_t base_lds(bool fp32, int max_rows, int max_local, int max_halo) {
+  const size_t NT = fp32 ? kResNT32 : kResNT64, v = fp32 ? 12 : 24;
+  return 24 * (max_rows + NT + 1) + (fp32 ? 24 * (size_t)max_local + 12 * (size_t)max_rows : 0) + 2 * v * max_local +
+         v * max_halo + 4 * (size_t)max_halo + 2 * NT + 64;
+}
+__host__ __device__ constexpr size_t tier_lds(bool fp32) { return (fp32 ? kResNT32 * 36 : kResNT64 * 72); }
+__host__ __device__ constexpr size_t two_start(bool fp32, int max_rows, int max_local, int max_halo, int KL) {
+  return (base_lds(fp32, max_rows, max_local, max_halo) + KL * tier_lds(fp32) + 15) / 16 * 16;
+}
 // LDS of the coarse space: offsets in doubles from its start.
 struct TwoLds {
   int c, uw, raw, tm, dsc, s, col, agg, end;
 };
-__host__ __device__ inline TwoLds two_lds(int ld, int max_need, int n_agg) {
-  TwoLds o;
+__host__ __device__ constexpr TwoLds two_lds(int ld, int max_need, int n_agg) {
+  TwoLds o{};
   o.c = 0;                                // [ld] scaled restricted residual
   o.uw = o.c + ld;                        // [max_need][6] rigid motions
   o.raw = o.uw + 6 * max_need;            // [pieces][8 waves][6] of the restriction, then [unknowns][8 waves] of the
@@ -105,6 +116,15 @@ __host__ __device__ inline TwoLds two_lds(int ld, int max_need, int n_agg) {
   return o;
 }
 // and behind it the list's aggregates (four bytes each) and two bytes per local vertex: place of its aggregate in the workgroup's list << 3 | fixed DOFs.
+
+constexpr bool two_lds_aligned() {
+  for (int n = 0; n < 32; ++n) {
+    const int rows = 100 + n % 2, local = 200 + n / 2 % 2, halo = 300 + n / 4 % 2, KL = n / 8 % 2;
+    if (two_start(n & 16, rows, local, halo, KL) % 16 || two_lds(8, 1 + n % 2, 1 + n / 2 % 2).col % 2) return false;
+  }
+  return true;
+}
+static_assert(two_lds_aligned(), "the pieces' int4 lie on 16 bytes whatever the sizes");
 
 constexpr int kAggWords = 8;
 // Six doubles as eight words of 48 payload bits under a 16-bit tag (half a
@@ -352,7 +372,7 @@ struct Meet {
 // r then leave LDS (FP64 10.7 -> 12.7 us, mixed equal).
 template <typename T, int NT, int KR, bool kMixed, bool kTwo>
 __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs<T> a) {
-  extern __shared__ double dyn[];
+  extern __shared__ __align__(16) double dyn[];
   __shared__ double s_red[4 * (NT / kWave)];
   __shared__ double s_tot[4 * (NT / kWave)];
   __shared__ int s_bad;
@@ -376,7 +396,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   int32_t* HX = reinterpret_cast<int32_t*>(L + (size_t)9 * NT * a.KL);  // [max_halo] places of the halo vertices
   uint16_t* EX = reinterpret_cast<uint16_t*>(HX + a.max_halo);        // [NT] partial slots of the exported rows
   const TwoLds tl = two_lds(a.ld, a.max_need, a.n_agg);
-  double* W2 = reinterpret_cast<double*>(EX + NT + (a.max_halo & 1) * 2);  // coarse space (kTwo)
+  double* W2 = dyn + two_start(sizeof(T) == 4, a.max_rows, a.max_local, a.max_halo, a.KL) / 8;  // coarse space (kTwo)
   double *C2 = W2 + tl.c, *UW = W2 + tl.uw, *RAW = W2 + tl.raw, *YS = RAW, *TM = W2 + tl.tm, *DS = W2 + tl.dsc, *SD = W2 + tl.s;
   int4* PC = reinterpret_cast<int4*>(W2 + tl.col);
   ushort2* AG = reinterpret_cast<ushort2*>(W2 + tl.agg);
@@ -1329,18 +1349,9 @@ int fill_words(DevBuf<uint64_t>& b, uint64_t word, hipStream_t st) {
   return SK_OK;
 }
 
-// Dynamic LDS without the matrix tiers, and of one tier block per thread.
-size_t base_lds(bool fp32, int max_rows, int max_local, int max_halo) {
-  const int NT = fp32 ? kResNT32 : kResNT64;
-  const size_t v = fp32 ? 12 : 24;
-  return 24 * (size_t)(max_rows + NT + 1) + (fp32 ? 24 * (size_t)max_local + 12 * (size_t)max_rows : 0) +
-         2 * v * max_local + v * max_halo + 4 * (size_t)max_halo + 2 * (size_t)NT + 64;
-}
 size_t two_lds_bytes(int ld, int max_need, int n_agg, int max_local) {
-  return 8 * (size_t)two_lds(ld, max_need, n_agg).end + 4 * (size_t)max_need + 2 * (size_t)max_local + 16;
+  return 8 * (size_t)two_lds(ld, max_need, n_agg).end + 4 * (size_t)max_need + 2 * (size_t)max_local + 16;  // 16: its start is rounded up
 }
-size_t tier_lds(bool fp32) { return (fp32 ? kResNT32 : kResNT64) * (9 * (fp32 ? 4 : 8)) * (size_t)1; }
-
 struct Permits {
   std::mutex mu;
   std::condition_variable cv;
