@@ -513,11 +513,10 @@ int sk_sim_set_parts(sk_sim* sim, int n, const int32_t* ptr_host);
  * are all later ones of this simulator), and the number of exchanges so far. */
 int sk_sim_solver_info(const sk_sim* sim, int* workgroups, int64_t* resident_solves, int64_t* launch_solves,
                        int64_t* gave_up, int64_t* exchanges);
-/* Test hook for the resident PCG's rare paths: bounds its waits at
- * wait_seconds (at most the default 2; 0: a run of several workgroups gives up
- * at once) and numbers its exchanges from `exchanges` on (at most 0x70000000,
- * past which a run starts over at 0). Waits for the device. */
-int sk_sim_resident_hook(sk_sim* sim, double wait_seconds, int64_t exchanges);
+/* Test hook for the resident PCG's rare paths: with give_up, its next run
+ * counts as given up; exchanges are numbered from `exchanges` on (at most
+ * 0x70000000, past which a run starts over at 0). Waits for the device. */
+int sk_sim_resident_hook(sk_sim* sim, int give_up, int64_t exchanges);
 /* Host-only, no counterpart in the reference: the vertices of X (host,
  * nv x 3) grouped by the aggregates sk_sim_set_coarse would form with
  * per_agg, ascending within each aggregate (order[nv]), the number of

@@ -221,7 +221,7 @@ SIGNATURES = {
     "sk_part_order": [_P, _P, _I64, _I64, _INT, _P, _P, _P],
     "sk_sim_set_parts": [_P, _INT, _P],
     "sk_sim_solver_info": [_P, _P, _P, _P, _P, _P],
-    "sk_sim_resident_hook": [_P, _D, _I64],
+    "sk_sim_resident_hook": [_P, _INT, _I64],
     "sk_sim_coarse_info": [_P, _P, _P, _P, _P],
     "sk_sim_set_order": [_P, _P],
 }

@@ -73,7 +73,7 @@ struct ResidentState {
   bool tried = false;                    // plan has been looked for
   bool off = false;                      // a run gave up waiting: launches only from now on
   int64_t runs = 0, launch_solves = 0, gave_up = 0;  // solves by this kernel and by launches; runs given up
-  double wait = kResWait;                // 0: a run of several workgroups gives up at once
+  bool give_up = false;                  // runs count as given up (test hook)
   DevBuf<uint64_t> slots, zx, xx;
   DevBuf<char> stream;
   DevBuf<int> abort_flag;

@@ -74,7 +74,6 @@ struct ResidentArgs {
   int max_rows, max_local, max_halo;
   double rtol2, inner_rtol2;
   int max_iter, max_refine;
-  long long wait_ticks;  // bound of a wait (Poll)
   // two-level preconditioner (ResidentTwo, CoarseSpace)
   int ld, n_agg, max_need;
   double shift;
@@ -138,18 +137,18 @@ __device__ __forceinline__ void put_word48(uint64_t* p, uint32_t epoch, uint64_t
 }
 __device__ __forceinline__ bool tagged48(uint64_t w, uint32_t epoch) { return (uint32_t)(w >> 48) == (epoch & 0xffffu); }
 
-// Ends a poll that has lasted `ticks` (of the 100 MHz clock) or that another
-// workgroup has ended: every wait is bounded, and the host then solves by
-// launches.
-constexpr double kTicksPerSecond = 1e8;
+// Ends a poll that has lasted kPollTicks (kResWait seconds of the 100 MHz
+// clock) or that another workgroup has ended: every wait is bounded, and the
+// host then solves by launches.
+constexpr long long kPollTicks = (long long)(kResWait * 1e8);
 struct Poll {
   int n = 0;
   long long t0 = 0;
-  __device__ __forceinline__ bool give_up(const int* abort_flag, long long ticks) {
+  __device__ __forceinline__ bool give_up(const int* abort_flag) {
     if ((++n & 255) != 0) return false;
     const long long now = wall_clock64();
     if (t0 == 0) t0 = now;
-    return now - t0 > ticks || __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    return now - t0 > kPollTicks || __hip_atomic_load(abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
   }
 };
 
@@ -180,7 +179,6 @@ struct Meet {
   int G;
   int parity;
   const int* abort_flag;
-  long long ticks;
   const int32_t* halo;  // [H] in LDS
   int H;
 
@@ -253,7 +251,7 @@ struct Meet {
           dest[(t + k * NT) / VS * VW + hw] = (uint32_t)b[k];
           need &= ~(1u << (NS + k));
         }
-      if (need && poll.give_up(abort_flag, ticks)) {
+      if (need && poll.give_up(abort_flag)) {
         *bad = 1;
         break;
       }
@@ -264,7 +262,7 @@ struct Meet {
         const uint64_t* p = words + (size_t)halo[j / VS] * VS + hw;
         uint64_t w = get_word(p);
         while (!tagged(w, epoch)) {
-          if (poll.give_up(abort_flag, ticks)) {
+          if (poll.give_up(abort_flag)) {
             *bad = 1;
             break;
           }
@@ -403,7 +401,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
   int32_t* NE = reinterpret_cast<int32_t*>(W2 + tl.end);               // [max_need] the list's aggregates
   uint16_t* LN = reinterpret_cast<uint16_t*>(NE + a.max_need);         // [max_local]
   T* S = a.stream + (size_t)me * a.KS * 9 * NT;
-  if (t == 0) s_bad = a.G > 1 && a.wait_ticks <= 0;  // a run that must not wait ends at its first meeting
+  if (t == 0) s_bad = 0;
 
   // the thread's blocks, their columns' byte offsets and which of them end a row
   T A[KR][9];
@@ -730,7 +728,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
 #pragma unroll
         for (int i = 0; i < N; ++i)
           if ((need >> i & 1) && tagged48(u[i], epoch)) need &= ~(1u << i);
-        if (need && poll.give_up(a.abort_flag, a.wait_ticks)) {
+        if (need && poll.give_up(a.abort_flag)) {
           s_bad = 1;
           break;
         }
@@ -829,7 +827,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       const uint64_t* p = a.uwords + (uint32_t)(NE[j / kAggWords] * kAggWords + j % kAggWords);
       uint64_t w = get_word(p);
       while (!tagged48(w, epoch)) {
-        if (poll.give_up(a.abort_flag, a.wait_ticks)) {
+        if (poll.give_up(a.abort_flag)) {
           s_bad = 1;
           break;
         }
@@ -882,7 +880,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     direction(R + j, B, r, T(0));
   }
 
-  Meet<NT> meet{s_red, s_tot, &s_bad, a.slots, a.G, 0, a.abort_flag, a.wait_ticks, HX, H};
+  Meet<NT> meet{s_red, s_tot, &s_bad, a.slots, a.G, 0, a.abort_flag, HX, H};
   uint32_t epoch = a.epoch;
   int iter = 0, done = 0, refines = 0;
   double tol2 = 0.0, target = 0.0;
@@ -1727,8 +1725,7 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
                     (const T*)s.binv, s.fixed, s.g, s.dx, p.halo_ptr.p, p.hvert.p, p.halo.p, p.exp0.p, p.exslot.p, R.slots.p, R.zx.p,
                     (uint32_t)(R.zx.n / 2),
                     R.xx.p, reinterpret_cast<T*>(R.stream.p), R.abort_flag.p, R.host, R.epoch, p.max_rows,
-                    p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine,
-                    (long long)(R.wait * kTicksPerSecond)};
+                    p.max_local, p.max_halo, s.rtol * s.rtol, s.inner_rtol * s.inner_rtol, s.max_iter, s.max_refine};
   if (kTwo) {
     const CoarseSpace& C = *s.coarse;
     const ResidentTwo& w = *R.two;

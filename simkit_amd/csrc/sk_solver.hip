@@ -2080,11 +2080,10 @@ int sk_sim_solver_info(const sk_sim* S, int* workgroups, int64_t* resident_solve
   return SK_OK;
 }
 
-int sk_sim_resident_hook(sk_sim* S, double wait_seconds, int64_t exchanges) {
+int sk_sim_resident_hook(sk_sim* S, int give_up, int64_t exchanges) {
   SK_REQUIRE(S, "sk_sim_resident_hook: null simulator");
-  SK_REQUIRE(wait_seconds >= 0.0 && wait_seconds <= kResWait, "sk_sim_resident_hook: the wait must be in [0, 2] s");
   SK_REQUIRE(exchanges >= 0 && exchanges <= (int64_t)kResMaxEpoch, "sk_sim_resident_hook: exchange number out of range");
-  S->res.wait = wait_seconds;
+  S->res.give_up = give_up != 0;
   if (S->may_be_resident()) resident_prepare(S->res, S->mesh, S->mixed(), S->two_level() ? &S->coarse : nullptr);
   return S->res.plan ? resident_set_epoch(S->res, (uint32_t)exchanges) : SK_OK;
 }
@@ -2228,7 +2227,7 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
     if (resident) {
       permit.release();
       const volatile ResidentResult* h = S->res.host;
-      if (h->aborted) {  // the run gave up waiting for a workgroup: solve by launches, now and later
+      if (h->aborted || S->res.give_up) {  // the run gave up waiting for a workgroup: solve by launches, now and later
         S->res.off = true;
         ++S->res.gave_up;
         resident = false;
