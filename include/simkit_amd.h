@@ -501,8 +501,9 @@ int sk_part_order(const double* X, const int32_t* T, int64_t nv, int64_t nt, int
                   int* n_parts, int32_t* part_ptr);
 /* The rows of the simulator's mesh as n contiguous ranges (ptr_host[n + 1],
  * as sk_part_order returns them), one per workgroup of the resident PCG; n =
- * 0 restores the default cut into equal ranges. No counterpart in the
- * reference. */
+ * 0 restores the default cut into equal ranges. The solver's plan and buffers
+ * are made here; without this call (and without a coarse space) the first step
+ * makes them, waiting for the device. No counterpart in the reference. */
 int sk_sim_set_parts(sk_sim* sim, int n, const int32_t* ptr_host);
 /* How the simulator's Newton systems have been solved (no counterpart in the
  * reference; any output may be null): workgroups of the resident PCG (0: the

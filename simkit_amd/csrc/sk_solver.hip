@@ -2065,6 +2065,8 @@ int sk_sim_set_parts(sk_sim* S, int n, const int32_t* ptr) {
   }));
   S->res.plan.reset();
   S->res.tried = false;
+  // here and not in the first step: it allocates and waits for the device
+  if (S->may_be_resident()) resident_prepare(S->res, S->mesh, S->mixed(), S->two_level() ? &S->coarse : nullptr);
   return SK_OK;
 }
 

@@ -172,3 +172,19 @@ def test_runs_of_several_threads_share_the_device():
         info = sim.solver_info()
         assert info["gave_up"] == info["launch_solves"] == 0, info
         assert all(np.array_equal(got[s], ref[s]) for s in range(1, 5))
+
+
+@pytest.mark.parametrize("precision,per_agg", [("fp64", 0), ("mixed", 0)])
+def test_the_first_step_allocates_nothing(precision, per_agg):
+    """A numbered simulator has its plan and buffers when it is built: a first step that allocates would wait for
+    whatever else runs on the device. (Two-level, the first step still forms the coarse operator.)"""
+    warm = _sim((40, 38, 39), precision, per_agg=per_agg)
+    warm.step(warm.X_dev, warm.X_dev)  # kernels loaded
+    sim = _sim((40, 39, 38), precision, per_agg=per_agg)
+    x, out = sim.X_dev, torch.empty_like(sim.X_dev)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    sim.step(x, x, out=out)
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
+    assert sim.solver_info()["launch_solves"] == 0 < sim.solver_info()["resident_solves"]
