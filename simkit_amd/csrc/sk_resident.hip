@@ -335,6 +335,12 @@ struct Meet {
 // alpha and r.r are direct sums of the current residual: the expansion enters
 // beta only. Iteration counts at 48^3 equal the two-launch form's (2,731 and
 // 2,837 over a step in FP64 and mixed precision).
+// On hard systems FP64 counts stay too (nu = 0.499, stiffness of 1e3 and 1e9 in
+// layers or anything between at random: within 0.5%), while FP32 ones move either
+// way: from the direct sum to this, at random 658 -> 778 (12^3) and 1,189 -> 1,483
+// (20^3), in layers 27,874 -> 3,581. With z.Ap in the exchange as a fifth sum (rz
+// - 2 alpha z.Ap + alpha^2 Ap.B^-1 Ap) they are the direct sum's again, 708, 1,188
+// and 32,915.
 // Slots and exported vertices' words exist twice and take turns by meeting: a
 // workgroup writes a buffer again only after a meeting that every workgroup
 // joined after its last read of it. (The FP64 correction's words are used once
