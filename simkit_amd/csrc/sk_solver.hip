@@ -2235,6 +2235,12 @@ int step_core(sk_sim* S, double c_mass, const double* const* guesses, int n_gues
         resident = false;
         goto launches;
       }
+      // A run that lost its numbers (r.z or p.Ap below the smallest normal, as with rtol 0, where the reciprocals it
+      // takes of them overflow): the launches divide, and say whether that is a breakdown.
+      if (h->done == 3) {
+        resident = false;
+        goto launches;
+      }
       ++S->res.runs;
       it = h->iter;
       done = h->done;

@@ -100,6 +100,22 @@ def test_a_run_that_gives_up_is_solved_by_launches(precision, per_agg):
 
 
 @pytest.mark.parametrize("precision,per_agg", FORMS)
+@pytest.mark.parametrize("n", [(1, 1, 3), (5, 3, 8), (13, 12, 14)])
+def test_a_solve_run_to_underflow_has_the_launches_status(n, precision, per_agg):
+    """With rtol 0 the residual shrinks until its products underflow. Whatever a solve by launches of the same system
+    reports for that, in the same numbering, a simulator that runs resident reports too."""
+    kw = {"per_agg": per_agg, "pcg_rtol": 0.0, "pcg_max_iter": 4000, "newton_max_iter": 1}
+    sim, ref = _sim(n, precision, **kw), _sim(n, precision, **kw)
+    _hook(ref, give_up=1)
+    x, info = sim.step(sim.X_dev, sim.X_dev)
+    y, want = ref.step(ref.X_dev, ref.X_dev)
+    assert ref.solver_info()["gave_up"] == 1
+    assert info["status"] == want["status"], (info, want)
+    if sim.solver_info()["launch_solves"]:
+        assert (x - y).abs().max() == 0.0
+
+
+@pytest.mark.parametrize("precision,per_agg", FORMS)
 @pytest.mark.parametrize("start", [0x70000000 - 40, 0x70000000, 65536 - 40, 65535])
 def test_exchange_numbers_start_over_and_wrap_their_tags(precision, per_agg, start):
     """Past 0x70000000 the next run starts at 0 again; the two-level words carry the low 16 bits only."""
