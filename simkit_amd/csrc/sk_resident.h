@@ -62,7 +62,7 @@ struct ResidentTwo {
   // the aggregates of the workgroup's rows and halo, and where each vertex's stands in that list
   DevBuf<int32_t> need0, need;     // [G + 1], ids
   DevBuf<uint16_t> lrow, lhalo;    // [nv], [all halos]
-  DevBuf<uint64_t> cwords, uwords; // [n_piece][8], [n_agg][8] exchanged words
+  DevBuf<uint64_t> cwords, uwords; // [2][n_piece][8] (of A p, of a residual), [n_agg][8] exchanged words
 };
 
 // A simulator's side of the resident solver: its plan and exchange buffers.

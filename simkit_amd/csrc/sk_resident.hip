@@ -82,7 +82,7 @@ struct ResidentArgs {
   const int32_t *agg_ptr, *agg_col;
   const double *tm, *dsc, *dv;
   const _Float16* einv;
-  uint64_t *cwords, *uwords;
+  uint64_t *cwords, *rwords, *uwords;
 };
 
 // Dynamic LDS (bytes): everything but the matrix tiers and the coarse space, one tier block per thread, and where
@@ -124,6 +124,16 @@ constexpr bool two_lds_aligned() {
   return true;
 }
 static_assert(two_lds_aligned(), "the pieces' int4 lie on 16 bytes whatever the sizes");
+
+// The restricted residual c follows r by c -= alpha W^T A p. What rounding leaves between them stays at the size that
+// c had, while r goes on to shrink, and a preconditioner that is applied to two different residuals ends in
+// directions that p.Ap does not bound: FP64 solves to 1e-16 and below ran to the iteration limit and returned them.
+// So c is formed from r again once r has shrunk by a million since the last time (FP64, once in a solve to 1e-8; by a
+// thousand where r is rounded to FP32), and every 4,096 iterations at the latest, long before the 16-bit tags of its
+// words come round. A step at 48^3 takes 14.15 ms with this and took 14.28 without (mixed 11.91 and 11.87).
+template <bool kMixed>
+constexpr double kRenew = kMixed ? 1e-6 : 1e-12;  // of r.r
+constexpr int kRenewAfter = 4096;
 
 constexpr int kAggWords = 8;
 // Six doubles as eight words of 48 payload bits under a 16-bit tag (half a
@@ -665,8 +675,8 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
     }
   };
-  // The pieces' scaled restrictions (wave 0, after a barrier).
-  auto put_pieces = [&](uint32_t epoch) {
+  // The pieces' scaled restrictions (wave 0, after a barrier) as `words`: of A p in cwords, of a residual in rwords.
+  auto put_pieces = [&](uint32_t epoch, uint64_t* words) {
     const int t = opaque((int)threadIdx.x);
     if (t >= kWave) return;
     const int j = t / 6, q = t % 6;
@@ -690,7 +700,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     wave_lds_fence();
     if (t < np * kAggWords) {
       const uint64_t* d3 = reinterpret_cast<const uint64_t*>(SD + 3 * (t / 4));
-      put_word48(a.cwords + (size_t)p0 * kAggWords + t, epoch, pack48(t % 4, d3[0], d3[1], d3[2]));
+      put_word48(words + (size_t)p0 * kAggWords + t, epoch, pack48(t % 4, d3[0], d3[1], d3[2]));
     }
   };
   // c = keep c + f (sum over an aggregate's pieces). Slot n is word n % 8 of aggregate n / 8: neighbouring lanes
@@ -706,7 +716,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
     return __longlong_as_double((long long)((w & k48) >> (16 * m) | next << (48 - 16 * m)));
   };
   // sums of the slots t + (i0 + i) NT
-  auto get_slots = [&](int i0, uint32_t epoch, auto& d) {
+  auto get_slots = [&](int i0, uint32_t epoch, const uint64_t* words, auto& d) {
     constexpr int N = sizeof(d) / sizeof(double);
     const int t = opaque((int)threadIdx.x) + i0 * NT;
     Poll poll;
@@ -730,7 +740,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       while (need) {
 #pragma unroll
         for (int i = 0; i < N; ++i)
-          if (need >> i & 1) u[i] = get_word(a.cwords + (uint32_t)((AG[(t + i * NT) / kAggWords].x + k) * kAggWords + t % kAggWords));
+          if (need >> i & 1) u[i] = get_word(words + (uint32_t)((AG[(t + i * NT) / kAggWords].x + k) * kAggWords + t % kAggWords));
 #pragma unroll
         for (int i = 0; i < N; ++i)
           if ((need >> i & 1) && tagged48(u[i], epoch)) need &= ~(1u << i);
@@ -758,12 +768,21 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
     }
   };
-  auto add_all = [&](uint32_t epoch, const double (&dh)[kSlots], double keep, double f) {
+  auto add_all = [&](uint32_t epoch, const uint64_t* words, const double (&dh)[kSlots], double keep, double f) {
     add_slots(0, dh, keep, f);
     for (int i0 = kSlots; i0 * NT < a.n_agg * kAggWords; ++i0) {
       double d[1];
-      get_slots(i0, epoch, d);
+      get_slots(i0, epoch, words, d);
       add_slots(i0, d, keep, f);
+    }
+  };
+  // c = the residual's restriction, a slot per thread at a time: this is rare, and eight at once take registers that
+  // the product needs (ten spilled instead of none).
+  auto take_residual = [&](uint32_t epoch) {
+    for (int i0 = 0; i0 * NT < a.n_agg * kAggWords; ++i0) {
+      double d[1];
+      get_slots(i0, epoch, a.rwords, d);
+      add_slots(i0, d, 0.0, 1.0);
     }
   };
   // y = (S16 + shift) c for the unknowns of the aggregates that begin here, as wave shares (after a barrier).
@@ -972,10 +991,9 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       meet.template wave_sums<1>(acc1);
       lds_barrier();
       meet.template publish<1>(++epoch);
-      put_pieces(epoch);
+      put_pieces(epoch, a.rwords);
       meet.template collect<1, T>(epoch, nullptr, nullptr);
-      get_slots(0, epoch, dh);
-      add_all(epoch, dh, 0.0, 1.0);
+      take_residual(epoch);
       lds_barrier();
       go = !s_bad;
       if (go) {
@@ -991,6 +1009,8 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         if (go) directions(T(0), z);
       }
     }
+    double rr_hi = rr;  // largest r.r since c was last formed from r, and the iterations since
+    int since = 0;
     while (go) {
       if (!kMixed && iter >= a.max_iter) break;
       product(P);
@@ -1014,8 +1034,8 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       meet.template publish<1>(++epoch);
       uint64_t* zx = a.zx + meet.parity * a.zx_half;
       put_exports(T(0), zx, epoch);
-      put_pieces(epoch);
-      get_slots(0, epoch, dh);
+      put_pieces(epoch, a.cwords);
+      get_slots(0, epoch, a.cwords, dh);
       meet.template collect<1, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
       load_binv(row ? opaque(v) : 0, B);
       double xg[3];
@@ -1033,7 +1053,8 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
       const T alpha = (T)(rz / pAp);
       ++iter;
-      add_all(epoch, dh, 1.0, -(double)alpha);
+      const bool renew = rr < kRenew<kMixed> * rr_hi || ++since == kRenewAfter;
+      if (!renew) add_all(epoch, a.cwords, dh, 1.0, -(double)alpha);
       const int l = opaque(t);
       double v2[2] = {0.0, 0.0};
       if (row) {
@@ -1055,6 +1076,14 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
 #pragma unroll
         for (int q = 0; q < 3; ++q) RL[3 * (R + j) + q] = fma(-alpha, HA[3 * j + q], RL[3 * (R + j) + q]);
       }
+      if (renew) {
+        restrict_rows((double)r[0], (double)r[1], (double)r[2]);
+        lds_barrier();
+        put_pieces(++epoch, a.rwords);
+        take_residual(epoch);
+        rr_hi = 0.0;
+        since = 0;
+      }
       lds_barrier();
       double rz_next;
       if (!second(v2[0], v2[1], rz_next, rr)) break;
@@ -1062,6 +1091,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         done = 3;
         break;
       }
+      rr_hi = rr > rr_hi ? rr : rr_hi;
       const bool conv = !(rr > tol2), limit = iter >= a.max_iter;
       if constexpr (!kMixed) {
         if (conv) {
@@ -1118,10 +1148,10 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         meet.template publish<1>(++epoch);
         zx = a.zx + meet.parity * a.zx_half;
         put_exports(T(0), zx, epoch);
-        put_pieces(epoch);
+        put_pieces(epoch, a.rwords);
         meet.template collect<1, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
-        get_slots(0, epoch, dh);
-        add_all(epoch, dh, 0.0, 1.0);
+        get_slots(0, epoch, a.rwords, dh);
+        add_all(epoch, a.rwords, dh, 0.0, 1.0);
         lds_barrier();
         if (s_bad) break;
         meet.template totals<1>(vb);
@@ -1135,6 +1165,8 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         }
         if (!second(v2[0], v2[1], rz_next, rr)) break;
         tol2 = a.inner_rtol2 * rr;
+        rr_hi = rr;
+        since = 0;
       }
       const T beta = (T)(rz_next / rz);
       rz = rz_next;
@@ -1624,7 +1656,7 @@ static std::unique_ptr<ResidentTwo> build_two(const sk_mesh* m, const std::vecto
     SK_TRY(two->need.upload(need));
     SK_TRY(two->lrow.upload(lrow));
     SK_TRY(two->lhalo.upload(lhalo));
-    SK_TRY(two->cwords.alloc((size_t)two->n_piece * 8));
+    SK_TRY(two->cwords.alloc((size_t)two->n_piece * 16));
     SK_TRY(two->uwords.alloc((size_t)n_agg * 8));
     SK_HIP_CHECK(hipMemset(two->cwords.p, 0, two->cwords.n * 8));
     SK_HIP_CHECK(hipMemset(two->uwords.p, 0, two->uwords.n * 8));
@@ -1754,6 +1786,7 @@ static int launch(ResidentState& R, sk_mesh* m, const ResidentSolve& s, hipStrea
     a.dv = C.dv64.p;
     a.einv = C.einv.p;
     a.cwords = w.cwords.p;
+    a.rwords = w.cwords.p + w.cwords.n / 2;
     a.uwords = w.uwords.p;
   }
   resident_pcg_kernel<T, NT, KR, kMixed, kTwo><<<p.G, NT, p.lds, st>>>(a);
