@@ -130,7 +130,7 @@ static_assert(two_lds_aligned(), "the pieces' int4 lie on 16 bytes whatever the 
 // directions that p.Ap does not bound: FP64 solves to 1e-16 and below ran to the iteration limit and returned them.
 // So c is formed from r again once r has shrunk by a million since the last time (FP64, once in a solve to 1e-8; by a
 // thousand where r is rounded to FP32), and every 4,096 iterations at the latest, long before the 16-bit tags of its
-// words come round. A step at 48^3 takes 14.15 ms with this and took 14.28 without (mixed 11.91 and 11.87).
+// words come round.
 template <bool kMixed>
 constexpr double kRenew = kMixed ? 1e-6 : 1e-12;  // of r.r
 constexpr int kRenewAfter = 4096;
@@ -366,9 +366,9 @@ struct Meet {
 // inverse of the aggregates that begin in it, read from L2. In the second they
 // publish r.r, r.z with their share of c.y, and their aggregates' rigid motions,
 // which the workgroups whose rows or halo lie in these add to z. Measured over a
-// step, launches then this kernel: 48^3 FP64 33.1 -> 23.2 ms, mixed 26.6 -> 19.1;
+// step, launches then this kernel: 48^3 FP64 25.5 -> 17.5 ms, mixed 19.8 -> 13.2;
 // 32^3 13.0 -> 8.2 and 12.3 -> 8.1; 10^3 5.7 -> 3.7 and 6.3 -> 3.9. An iteration
-// at 48^3 (35.7 and 29 us) is bound by its chain of phases: product 8 (FP64, five
+// at 48^3 (31.4 and 24.7 us) is bound by its chain of phases: product 8 (FP64, five
 // of a thread's blocks from L2) or 2 to 5, pieces of all 512 aggregates 4,
 // rows of the inverse 3.5 to 4.5, second meeting 3 to 5, update 3, the rest around
 // 1 each. With more blocks in registers the values in flight spill (152 registers
@@ -768,16 +768,17 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       }
     }
   };
-  auto add_all = [&](uint32_t epoch, const uint64_t* words, const double (&dh)[kSlots], double keep, double f) {
-    add_slots(0, dh, keep, f);
+  auto add_all = [&](uint32_t epoch, const double (&dh)[kSlots], double f) {
+    add_slots(0, dh, 1.0, f);
     for (int i0 = kSlots; i0 * NT < a.n_agg * kAggWords; ++i0) {
       double d[1];
-      get_slots(i0, epoch, words, d);
-      add_slots(i0, d, keep, f);
+      get_slots(i0, epoch, a.cwords, d);
+      add_slots(i0, d, 1.0, f);
     }
   };
-  // c = the residual's restriction, a slot per thread at a time: this is rare, and eight at once take registers that
-  // the product needs (ten spilled instead of none).
+  // c = the residual's restriction, a slot per thread at a time: this is rare, and eight at once, inlined here too,
+  // take registers that the product needs (FP64 14.55 ms a step at 48^3 against 14.14; mixed, where the replaced
+  // residual is read this way as well, 16.5 against 15.5).
   auto take_residual = [&](uint32_t epoch) {
     for (int i0 = 0; i0 * NT < a.n_agg * kAggWords; ++i0) {
       double d[1];
@@ -1054,7 +1055,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
       const T alpha = (T)(rz / pAp);
       ++iter;
       const bool renew = rr < kRenew<kMixed> * rr_hi || ++since == kRenewAfter;
-      if (!renew) add_all(epoch, a.cwords, dh, 1.0, -(double)alpha);
+      if (!renew) add_all(epoch, dh, -(double)alpha);
       const int l = opaque(t);
       double v2[2] = {0.0, 0.0};
       if (row) {
@@ -1150,8 +1151,7 @@ __global__ __launch_bounds__(NT, NT / 256) void resident_pcg_kernel(ResidentArgs
         put_exports(T(0), zx, epoch);
         put_pieces(epoch, a.rwords);
         meet.template collect<1, T>(epoch, zx, reinterpret_cast<uint32_t*>(HA));
-        get_slots(0, epoch, a.rwords, dh);
-        add_all(epoch, a.rwords, dh, 0.0, 1.0);
+        take_residual(epoch);
         lds_barrier();
         if (s_bad) break;
         meet.template totals<1>(vb);
