@@ -266,6 +266,7 @@ def run_path(args, X, T, bottom, top, mu, lam, name):
         "spmv_ms": spmv_ms, "spmv_bytes": traffic, "hess_ms": hess_ms, "infos": infos,
         "x_final": x_final.cpu().numpy(),
         "coarse": sim.coarse_info() if pc == "two_level" else None,
+        "solver": sim.solver_info(),
     }
     log(f"bench[{name}]: {elapsed:.2f}s, {res['steps_per_s']:.3f} steps/s, newton {res['newton_iters']}, "
         f"pcg {res['pcg_iters']}, spmv {spmv_ms * 1e3:.1f} us, element pass {hess_ms * 1e3:.1f} us, "
@@ -522,7 +523,12 @@ def main():
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": pmc_traffic("spmv_fp64" if PATHS[head_name][0] == "fp64" else "spmv_fp32")
                      if args.cells == 48 else None,
-                     "bytes_per_launch": int(head["spmv_bytes"]), "avg_launch_ms": round(head["spmv_ms"], 5)},
+                     "bytes_per_launch": int(head["spmv_bytes"]), "avg_launch_ms": round(head["spmv_ms"], 5),
+                     "in_timed_region": head["solver"]["launch_solves"] > 0},
+        # what solved the timed region's (and the warm-up's) Newton systems, and its time per PCG iteration
+        "solver": {"kernel": "resident_pcg_kernel" if head["solver"]["resident_solves"] else "bpcg_spmv_kernel",
+                   **head["solver"],
+                   "us_per_pcg_iteration": round(1e3 * head["phase_ms_total"]["ms_pcg"] / max(1, head["pcg_iters"]), 3)},
     }
     if PATHS[head_name][0] == "fp64":
         # the element pass against HBM on its algorithmic bytes (it is neither stream- nor FP64-bound:
